@@ -277,15 +277,15 @@ int csr_alloc(fx_csr A) {
   return 0;
 }
 
-// Row patterns of a matrix given on the host: pid[i] and a dictionary of
-// plen-strided offset lists (col - row).  False when some row is longer than
+// Row patterns of a matrix given on the host: pid[i], a dictionary of
+// plen-strided offset lists (col - row) and each pattern's first row.  False when some row is longer than
 // kPatMaxLen, there are more than kPatMax distinct patterns, or the
 // dictionary exceeds kPatDict offsets.  Each
 // pattern is found by a hash of (length, offsets) and then compared entry by
 // entry, so a hash collision cannot merge two patterns.
 bool build_patterns(uint32_t nrow, const uint32_t* rp, const uint32_t* ci, uint32_t max_row,
-                    std::vector<uint8_t>& pid, std::vector<int32_t>& dict, uint32_t& plen,
-                    uint32_t& npat) {
+                    std::vector<uint8_t>& pid, std::vector<int32_t>& dict,
+                    std::vector<uint32_t>& first, uint32_t& plen, uint32_t& npat) {
   if (max_row > kPatMaxLen || nrow == 0) return false;
   plen = max_row ? max_row : 1;
   std::vector<std::vector<int32_t>> pats;
@@ -312,6 +312,7 @@ bool build_patterns(uint32_t nrow, const uint32_t* rp, const uint32_t* ci, uint3
       if (pats.size() >= kPatMax) return false;
       found = (int)pats.size();
       pats.emplace_back(off.begin(), off.begin() + len);
+      first.push_back(i);
       ids.push_back((uint32_t)found);
     }
     pid[i] = (uint8_t)found;
@@ -328,6 +329,46 @@ bool patterns_disabled() {
   const char* e = std::getenv("FASPXX_FX_NOPAT");
   return e && e[0] == '1';
 }
+
+bool row_values_enabled() {
+  const char* e = std::getenv("FASPXX_FX_NOROWVAL");
+  return !(e && e[0] == '1');
+}
+
+// vd[p * stride + j] = entry j of pattern p's row prow[p] (0 past its length),
+// and *ok = 1 before k_row_values_check clears it.
+template <class T>
+__global__ void k_row_values_fill(const uint32_t* __restrict__ rp, const T* __restrict__ va,
+                                  const uint32_t* __restrict__ prow,
+                                  const uint32_t* __restrict__ pcnt, uint32_t npat, uint32_t stride,
+                                  T* __restrict__ vd, int* __restrict__ ok) {
+  if (threadIdx.x == 0) *ok = 1;
+  for (uint32_t i = threadIdx.x; i < npat * stride; i += kThreads) {
+    const uint32_t p = i / stride, j = i % stride;
+    vd[i] = j < pcnt[p] ? va[rp[prow[p]] + j] : (T)0;
+  }
+}
+
+// Clears *ok when some row differs from its pattern's values in any bit.
+// Once it is cleared the workgroups that start later leave at once, so a
+// matrix of varying values costs next to nothing here.
+template <class T>
+__global__ __launch_bounds__(kThreads) void k_row_values_check(
+    const uint32_t* __restrict__ rp, const T* __restrict__ va, const uint8_t* __restrict__ pid,
+    const T* __restrict__ vd, uint32_t stride, uint32_t nrow, int* ok) {
+  using U = std::conditional_t<sizeof(T) == 8, unsigned long long, unsigned int>;
+  if (__hip_atomic_load(ok, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == 0) return;
+  const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
+  if (i >= nrow) return;
+  const U* v = reinterpret_cast<const U*>(va) + rp[i];
+  const U* d = reinterpret_cast<const U*>(vd) + (uint32_t)pid[i] * stride;
+  const uint32_t len = rp[i + 1] - rp[i];
+  bool same = true;
+  for (uint32_t j = 0; j < len; ++j) same = same && v[j] == d[j];
+  if (!same) __hip_atomic_store(ok, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+__global__ void k_clear_flag(int* ok) { *ok = 0; }
 
 // Matrices whose columns take neither row patterns nor 16-bit deltas get
 // rows sorted by length (default; FASPXX_FX_NOSORT=1: not), else sliced
@@ -348,6 +389,43 @@ bool sort_enabled() {
 }
 
 }  // namespace
+
+namespace {
+template <class T>
+int row_values(fx_csr A, const T* va, T* vd, int* vok, bool* host_ok) {
+  hipStream_t st = A->ctx->stream;
+  hipLaunchKernelGGL(k_row_values_fill<T>, dim3(1), dim3(kThreads), 0, st, A->rp, va, A->prow,
+                     A->pcnt, A->npat, A->vstride, vd, vok);
+  hipLaunchKernelGGL(k_row_values_check<T>, dim3((A->nrow + kThreads - 1) / kThreads),
+                     dim3(kThreads), 0, st, A->rp, va, A->pid, (const T*)vd, A->vstride, A->nrow, vok);
+  FX_HIP(hipGetLastError());
+  int ok = 0;
+  FX_HIP(hipMemcpyAsync(&ok, vok, sizeof(int), hipMemcpyDeviceToHost, st));
+  FX_HIP(hipStreamSynchronize(st));
+  *host_ok = ok == 1;
+  return 0;
+}
+}  // namespace
+
+int csr_row_values(fx_csr A, const double* va, double* vd, int* vok, bool* host_ok) {
+  return row_values(A, va, vd, vok, host_ok);
+}
+int csr_row_values(fx_csr A, const float* va, float* vd, int* vok, bool* host_ok) {
+  return row_values(A, va, vd, vok, host_ok);
+}
+
+// Later launches are not given the row values (vconst), and solvers set up
+// on A make new replay graphs (gen) on the grid of single row blocks;
+// launches that a caller captured earlier find the flag cleared when they
+// run.
+int csr_drop_row_values(fx_csr A) {
+  if (!A->vconst) return 0;
+  A->vconst = false;
+  A->gen = next_handle_gen();
+  hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1), 0, A->ctx->stream, A->vok);
+  FX_HIP(hipGetLastError());
+  return 0;
+}
 
 // The values of the slices from the CSR values: dst[p] = src[smap[p]]
 // (0 in padding slots).
@@ -574,12 +652,13 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
   const bool col32 = col32_env || sell == 2;
   std::vector<uint8_t> pid;
   std::vector<int32_t> dict;
+  std::vector<uint32_t> first;
   uint32_t plen = 0, npat = 0;
   bool pat = false;
   if (host_ci && A->nnz && !col32 && !patterns_disabled()) {
     uint32_t longest = 0;
     for (uint32_t r = 0; r < A->nrow; ++r) longest = std::max(longest, host_rp[r + 1] - host_rp[r]);
-    pat = build_patterns(A->nrow, host_rp, host_ci, longest, pid, dict, plen, npat);
+    pat = build_patterns(A->nrow, host_rp, host_ci, longest, pid, dict, first, plen, npat);
   }
   uint32_t mx = 0;
   const std::vector<uint32_t> rows =
@@ -611,6 +690,28 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
                           hipMemcpyHostToDevice, st));
     A->plen = plen;
     A->npat = npat;
+    if (A->has_values && A->nrow > kRowValMin && row_values_enabled()) {
+      std::vector<uint32_t> cnt(npat);
+      for (uint32_t p = 0; p < npat; ++p) cnt[p] = host_rp[first[p] + 1] - host_rp[first[p]];
+      A->vstride = plen <= 8 && npat * 8 <= kPatDict ? 8 : plen;
+      std::vector<int32_t> vdict((size_t)npat * A->vstride);
+      for (uint32_t p = 0; p < npat; ++p)
+        for (uint32_t j = 0; j < A->vstride; ++j)
+          vdict[(size_t)p * A->vstride + j] =
+              cnt[p] ? dict[(size_t)p * plen + std::min(j, cnt[p] - 1)] : 0;
+      FX_HIP(hipMalloc(&A->vdict, sizeof(int32_t) * vdict.size()));
+      FX_HIP(hipMemcpyAsync(A->vdict, vdict.data(), sizeof(int32_t) * vdict.size(),
+                            hipMemcpyHostToDevice, st));
+      FX_HIP(hipMalloc(&A->prow, sizeof(uint32_t) * npat));
+      FX_HIP(hipMalloc(&A->pcnt, sizeof(uint32_t) * npat));
+      FX_HIP(hipMalloc(&A->vok, sizeof(int)));
+      FX_HIP(hipMalloc(&A->vd64, sizeof(double) * vdict.size()));
+      FX_HIP(hipMemcpyAsync(A->prow, first.data(), sizeof(uint32_t) * npat, hipMemcpyHostToDevice,
+                            st));
+      FX_HIP(hipMemcpyAsync(A->pcnt, cnt.data(), sizeof(uint32_t) * npat, hipMemcpyHostToDevice,
+                            st));
+      FX_TRY(csr_row_values(A, A->va, A->vd64, A->vok, &A->vconst));
+    }
     FX_HIP(hipStreamSynchronize(st));  // the host vectors go out of scope
     return 0;
   }
@@ -658,6 +759,8 @@ void csr_free(fx_csr A) {
   (void)hipFree(A->pid);
   (void)hipFree(A->pdict);
   (void)hipFree(A->src);
+  void* row_value_arrays[] = {A->vok, A->prow, A->pcnt, A->vdict, A->vd64, A->vd32};
+  for (void* q : row_value_arrays) (void)hipFree(q);
   void* sell_arrays[] = {A->sblk, A->swin, A->soff, A->slane, A->scol,
                          A->smap, A->sval, A->lwin, A->lrow};
   for (void* q : sell_arrays) (void)hipFree(q);
@@ -887,6 +990,13 @@ int fx_csr_make_f32(fx_csr A) {
   hipLaunchKernelGGL(k_f64_to_f32, dim3(stream_blocks(A->nnz)), dim3(kThreads), 0, A->ctx->stream,
                      A->va, A->va32, A->nnz);
   FX_HIP(hipGetLastError());
+  if (A->vconst) {  // the row values too: the same conversion of the same values
+    const uint32_t nd = A->npat * A->vstride;
+    if (!A->vd32) FX_HIP(hipMalloc(&A->vd32, sizeof(float) * nd));
+    hipLaunchKernelGGL(k_f64_to_f32, dim3(stream_blocks(nd)), dim3(kThreads), 0, A->ctx->stream,
+                       A->vd64, A->vd32, nd);
+    FX_HIP(hipGetLastError());
+  }
   if (A->sorted) {  // the sorted copy's f32 values, converted from its f64 ones
     if (!A->oval32) FX_HIP(hipMalloc(&A->oval32, sizeof(float) * A->nnz));
     hipLaunchKernelGGL(k_f64_to_f32, dim3(stream_blocks(A->nnz)), dim3(kThreads), 0,
@@ -900,6 +1010,7 @@ int fx_csr_set_values_dev(fx_csr A, const double* dev_values) {
   clear_error();
   FX_CHECK(A && dev_values, FX_ERROR_INPUT_PAR, "null argument");
   if (A->nnz == 0) return 0;
+  FX_TRY(csr_drop_row_values(A));
   if (dev_values != A->va)
     FX_HIP(hipMemcpyAsync(A->va, dev_values, sizeof(double) * A->nnz, hipMemcpyDeviceToDevice,
                           A->ctx->stream));
@@ -913,7 +1024,11 @@ int fx_csr_set_values_dev(fx_csr A, const double* dev_values) {
   return 0;
 }
 
-double* fx_csr_values_dev(fx_csr A) { return A ? A->va : nullptr; }
+double* fx_csr_values_dev(fx_csr A) {
+  if (!A) return nullptr;
+  // the caller may write the values through the pointer at any later time
+  return csr_drop_row_values(A) == 0 ? A->va : nullptr;
+}
 
 int fx_spmv(fx_ctx ctx, fx_csr A, fx_vec v, fx_vec w) {
   clear_error();

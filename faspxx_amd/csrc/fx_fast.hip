@@ -1583,7 +1583,7 @@ int fast_solve(fx_solver S, fx_vec b, fx_vec x, fx_result* res) {
                           ? gmres_state_bytes()
                                                       : sizeof(CgState);
     int rc = ws_alloc(*S->fast, S->ctx, FX_F64, n, S->prm.maxIter, sb,
-                      S->op ? op_grid(n) : spmv_grid_of<double>(S->A, S->ctx->sms));
+                      S->op ? op_grid(n) : spmv_grid_max<double>(S->A));
     if (!rc && S->op) {  // the operator's work vectors, before any graph is captured
       const size_t vb = pack_round(n) * sizeof(double);
       if (hipMalloc(&S->fast->opy, vb) != hipSuccess || hipMalloc(&S->fast->opx, vb) != hipSuccess) {
@@ -1653,6 +1653,8 @@ struct fx_ir_s {
   int* bad = nullptr;
   uint32_t* blk512 = nullptr;  // row-pattern matrices: As's own 512-row blocks
   uint16_t* rpb512 = nullptr;
+  int* vok32 = nullptr;  // row values of S A S (see fx_csr_s), where it has them
+  float* vd32 = nullptr;
   fx_csr_s As{};
   ~fx_ir_s() {
     if (ctx) (void)hipStreamSynchronize(ctx->stream);
@@ -1672,6 +1674,8 @@ struct fx_ir_s {
     (void)hipFree(bad);
     (void)hipFree(blk512);
     (void)hipFree(rpb512);
+    (void)hipFree(vok32);
+    (void)hipFree(vd32);
   }
 };
 
@@ -1733,6 +1737,15 @@ int ir_scale(fx_ir ir) {
     ir->As.rpb = ir->rpb512;
     ir->As.nblk = nb;
     ir->As.pat_rows = kPat2Rows;
+    // S A S keeps the row values of A when rows of one pattern scale alike
+    if (A->vconst) {
+      FX_HIP(hipMalloc(&ir->vok32, sizeof(int)));
+      FX_HIP(hipMalloc(&ir->vd32, sizeof(float) * A->npat * A->vstride));
+      ir->As.vconst = false;
+      FX_TRY(csr_row_values(A, (const float*)ir->vs32, ir->vd32, ir->vok32, &ir->As.vconst));
+    }
+    ir->As.vok = ir->vok32;
+    ir->As.vd32 = ir->vd32;
   }
   ir->scaled = true;
   return 0;
@@ -1779,7 +1792,7 @@ int fx_ir_create(fx_ctx ctx, int inner_type, fx_csr A, double weight, const fx_p
     if (rc) return fail(rc);
   }
   const size_t nb = n ? n : 1;
-  const size_t np = 8 * ((size_t)std::max(spmv_grid_of<double>(A), spmv_grid_of<float>(A)) +
+  const size_t np = 8 * ((size_t)std::max(spmv_grid_max<double>(A), spmv_grid_max<float>(A)) +
                          kMaxRedBlocks);
   if (hipMalloc(&ir->r32, sizeof(float) * nb) || hipMalloc(&ir->d32, sizeof(float) * nb) ||
       hipMalloc(&ir->dsc, sizeof(double) * 4) ||
@@ -1791,7 +1804,7 @@ int fx_ir_create(fx_ctx ctx, int inner_type, fx_csr A, double weight, const fx_p
   if (inner_type == FX_SOLVER_CG) {
     ir->W = new FastWs();
     const size_t sb = sizeof(CgState) > sizeof(IrState) ? sizeof(CgState) : sizeof(IrState);
-    rc = ws_alloc(*ir->W, ctx, FX_F32, n, inner->maxIter, sb, spmv_grid_of<float>(A, ctx->sms));
+    rc = ws_alloc(*ir->W, ctx, FX_F32, n, inner->maxIter, sb, spmv_grid_max<float>(A));
     if (rc) return fail(rc);
     // the scaled inner solve's second r buffer (odd iterations' r)
     if (ir->scaled && hipMalloc(&ir->W->s, sizeof(float) * pack_round(n))) {

@@ -133,6 +133,23 @@ struct fx_csr_s {
   int32_t* pdict = nullptr;
   uint32_t plen = 0, npat = 0;
   uint32_t pat_rows = 256;  // rows per row block of a row-pattern matrix (256 or 512)
+  // Row values, for a row-pattern matrix whose rows of one pattern also hold
+  // the same values bit for bit (constant-coefficient stencils): entry j of
+  // such a row is vd64[pid * vstride + j] in column i + vdict[pid * vstride +
+  // j] (f32 kernels: vd32), and the SpMV kernels then read no per-entry data
+  // at all.  vstride is 8 where rows hold at most 8 entries and the padded
+  // dictionary still fits (the padding repeats the last offset), else plen.
+  // The kernels take this form while *vok is 1, so that launches already
+  // captured in a graph follow a change of the values; vconst is its host
+  // side.  prow: a row of each pattern; pcnt: the patterns' lengths.
+  bool vconst = false;
+  int* vok = nullptr;
+  uint32_t* prow = nullptr;
+  uint32_t* pcnt = nullptr;
+  uint32_t vstride = 0;
+  int32_t* vdict = nullptr;
+  double* vd64 = nullptr;
+  float* vd32 = nullptr;
   // set on a transpose: entry p of this matrix is entry src[p] of its source
   uint32_t* src = nullptr;
   // Sliced rows, for the f64 kernels of a matrix made from host arrays
@@ -253,13 +270,38 @@ inline unsigned spmv_grid(uint32_t nblk, int /*cus*/) {
 // reduction partial each): the sliced-row windows for f64 when the matrix
 // has them, else the row blocks.
 template <class MT>
-inline uint32_t spmv_units(const fx_csr_s* A) {
+inline uint32_t spmv_blocks_of(const fx_csr_s* A) {
   if (A->sorted) return A->onblk;
   return (sizeof(MT) == 8 && A->sell) ? A->nwin : A->nblk;
+}
+// Rows a workgroup takes from a matrix with row values.  The matrix costs
+// nothing to read there, so a workgroup of 256 rows is only latency (flag,
+// dictionary, gathers, reduction, one after the other): on the 128^3 stencil
+// the f64 product takes 14.2 us with 1024 rows per workgroup and 16 us with
+// 256 (24.5 us streaming the values).  Up to kRowValMin rows the values
+// stay in L2, 1024 rows per workgroup would leave CUs without one, and the
+// dictionary is one more dependent load (256^2 points, FGMRES: 17.0 against
+// 16.9 ms), so the kernels stream the values there.
+constexpr uint32_t kRowValRows = 1024;
+constexpr uint32_t kRowValMin = 256 * kRowValRows;
+template <class MT>
+inline bool has_row_values(const fx_csr_s* A) {
+  return A->vconst && A->nrow > kRowValMin && (sizeof(MT) == 8 || A->vd32);
+}
+template <class MT>
+inline uint32_t spmv_units(const fx_csr_s* A) {
+  if (has_row_values<MT>(A)) return (A->nrow + kRowValRows - 1) / kRowValRows;
+  return spmv_blocks_of<MT>(A);
 }
 template <class MT>
 inline unsigned spmv_grid_of(const fx_csr_s* A, int cus = 0) {
   return spmv_grid(spmv_units<MT>(A), cus);
+}
+// The largest grid A's SpMV may run on, now or once its row values are
+// dropped: what a workspace for its partials is sized for.
+template <class MT>
+inline unsigned spmv_grid_max(const fx_csr_s* A) {
+  return spmv_grid(spmv_blocks_of<MT>(A), 0);
 }
 
 // ---------------------------------------------------------------------------
@@ -537,6 +579,15 @@ int csr_storage(fx_csr A);
 // 2-byte block-relative row pointers and the block count, in new device
 // allocations owned by the caller.
 int csr_pattern_blocks512(fx_csr A, uint32_t** blk, uint16_t** rpb, uint32_t* nblk);
+// Row values of a row-pattern matrix from va (CSR order): the dictionary
+// vd (npat * vstride entries) from a row of each pattern, and *vok = 1 when
+// every row holds its pattern's values bit for bit, else 0.  Device memory
+// of the caller; *host_ok: the flag, after a wait for it.
+int csr_row_values(fx_csr A, const double* va, double* vd, int* vok, bool* host_ok);
+int csr_row_values(fx_csr A, const float* va, float* vd, int* vok, bool* host_ok);
+// The values of A are about to change, or may from now on: its kernels read
+// them entry by entry again.
+int csr_drop_row_values(fx_csr A);
 void csr_release(fx_csr A);
 int scan_u32(hipStream_t st, const uint32_t* cnt, uint32_t m, uint32_t* out);
 int csr_finish_device(fx_csr A);

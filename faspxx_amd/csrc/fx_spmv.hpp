@@ -59,12 +59,21 @@ struct SpmvIn {
   // rows sorted by length (u32 columns): the matrix row of each block row,
   // or null when block rows are matrix rows
   const uint32_t* __restrict__ rmap;
+  // row patterns whose rows also share their values (see fx_csr_s): the
+  // values and lengths of the patterns, used while *vok is 1; vok is null
+  // where the matrix has none
+  const int* __restrict__ vok;
+  const MT* __restrict__ pval;
+  const uint32_t* __restrict__ pcnt;
+  const int32_t* __restrict__ vdict;
+  uint32_t npat, vstride, nrow;
 };
 
 // Column formats of the staged entries: u32 columns, 16-bit deltas to the
 // block's first row, or row patterns (no per-entry column data) in blocks
-// of 256 rows (CF_PAT) or 512 rows (CF_PAT2).
-enum { CF_U32 = 0, CF_D16 = 1, CF_PAT = 2, CF_PAT2 = 3, CF_SELL = 4 };
+// of 256 rows (CF_PAT) or 512 rows (CF_PAT2), or row patterns with row
+// values (CF_ROWVAL: no per-entry data at all).
+enum { CF_U32 = 0, CF_D16 = 1, CF_PAT = 2, CF_PAT2 = 3, CF_SELL = 4, CF_ROWVAL = 5 };
 constexpr bool is_pat(int cf) { return cf == CF_PAT || cf == CF_PAT2; }
 
 template <class MT, class VT>
@@ -79,12 +88,14 @@ inline SpmvIn<double, double> spmv_in<double, double>(fx_csr A) {
             A->oblk,  A->onblk, A->nnz, nullptr, nullptr,
             0,        0,
             nullptr, nullptr, nullptr, nullptr, nullptr,
-            nullptr, nullptr, A->omap};
+            nullptr, nullptr, A->omap, nullptr, nullptr, nullptr, nullptr, 0, 0, 0};
   return {A->rp,   A->rpb,  A->ci,  A->cd,    A->has_values ? A->va : nullptr,
           A->sell ? A->sblk : A->blk,  A->sell ? A->nwin : A->nblk, A->nnz, A->pid,   A->pdict,
           A->plen, A->npat * A->plen,
           A->swin, A->soff, A->slane, A->scol, A->has_values ? A->sval : nullptr,
-          A->lwin, A->lrow, nullptr};
+          A->lwin, A->lrow, nullptr,
+          has_row_values<double>(A) ? A->vok : nullptr, A->vd64, A->pcnt,
+          A->vdict, A->npat, A->vstride, A->nrow};
 }
 template <>
 inline SpmvIn<float, float> spmv_in<float, float>(fx_csr A) {
@@ -93,12 +104,14 @@ inline SpmvIn<float, float> spmv_in<float, float>(fx_csr A) {
             A->oblk,  A->onblk, A->nnz, nullptr, nullptr,
             0,        0,
             nullptr, nullptr, nullptr, nullptr, nullptr,
-            nullptr, nullptr, A->omap};
+            nullptr, nullptr, A->omap, nullptr, nullptr, nullptr, nullptr, 0, 0, 0};
   return {A->rp,   A->rpb,  A->ci,  A->cd,    A->has_values ? A->va32 : nullptr,
           A->blk,  A->nblk, A->nnz, A->pid,   A->pdict,
           A->plen, A->npat * A->plen,
           nullptr, nullptr, nullptr, nullptr, nullptr,
-          nullptr, nullptr, nullptr};
+          nullptr, nullptr, nullptr,
+          has_row_values<float>(A) ? A->vok : nullptr, A->vd32, A->pcnt,
+          A->vdict, A->npat, A->vstride, A->nrow};
 }
 
 // Threads per row for a block of nr rows holding nz entries: one thread per
@@ -153,19 +166,21 @@ struct SpmvLds {
   using RpT = std::conditional_t<FX_RP16 != 0, uint16_t, uint32_t>;
   using CiT = std::conditional_t<CF == CF_D16, int16_t, uint32_t>;
   static constexpr uint32_t kRows = CF == CF_SELL   ? 1
+                                    : CF == CF_ROWVAL ? kPatMax
                                     : CF == CF_PAT2 ? kPat2Rows
                                     : CF == CF_PAT  ? kPatRows
                                                     : kBlockRows;
   static constexpr uint32_t kNnz = CF == CF_SELL   ? 1
+                                   : CF == CF_ROWVAL ? kPatDict
                                    : CF == CF_PAT2 ? kPat2Nnz
                                    : CF == CF_PAT  ? kPatNnz
                                                    : kBlockNnz;
-  static constexpr uint32_t kCi = (is_pat(CF) || CF == CF_SELL) ? 1 : kBlockNnz;
-  static constexpr uint32_t kDict = is_pat(CF) ? kPatDict : 1;
+  static constexpr uint32_t kCi = (is_pat(CF) || CF == CF_SELL || CF == CF_ROWVAL) ? 1 : kBlockNnz;
+  static constexpr uint32_t kDict = (is_pat(CF) || CF == CF_ROWVAL) ? kPatDict : 1;
   RpT rp[kRows + 1];
   CiT ci[kCi];
-  int32_t dict[kDict];
-  MT va[kNnz];
+  alignas(16) int32_t dict[kDict];
+  alignas(16) MT va[kNnz];
   __device__ __forceinline__ uint32_t col(uint32_t k, uint32_t r0) const {
     if constexpr (CF == CF_D16) return (uint32_t)((int32_t)r0 + (int32_t)ci[k]);
     else return ci[k];
@@ -415,6 +430,132 @@ __device__ __forceinline__ void pat_block(const SpmvIn<MT, VT>& in, SpmvLds<MT, 
   }
 }
 
+// Rows [r0, r0 + nr) of a row-pattern matrix whose rows share their
+// patterns' values (nr <= kRowValRows): one byte per row and the dictionary
+// (offsets, values and lengths, L2-resident, copied to LDS) are all that is
+// read of the matrix, so the block is bound by the latency of its gathers
+// and by the epilogue's vectors.  Two rows per thread at a time: their
+// gathers go out before the first sum, within the registers that let eight
+// workgroups stay on a CU.  With the dictionary padded to 8 entries a row
+// reads its offsets and values as whole 16-byte packs of LDS.  Each row is
+// summed as pat_block sums the same values: the same bits.  Once *vok has
+// been cleared (a launch captured before the values changed) the rows are
+// read entry by entry from the CSR arrays, summed in the same order.
+template <int MODE, int NRED, class MT, class VT, class XF, class BF, class Epi>
+__device__ __forceinline__ void row_value_block(const SpmvIn<MT, VT>& in,
+                                                SpmvLds<MT, CF_ROWVAL>& lds, uint32_t r0,
+                                                uint32_t nr, int tid, const XF& xf, const BF& bf,
+                                                const Epi& epi,
+                                                double (&acc)[NRED > 0 ? NRED : 1]) {
+  constexpr int P = 2;                                // rows per thread at a time
+  constexpr int H = kRowValRows / (P * kThreads);     // passes
+  constexpr int kDv = kPatDict / kThreads;
+  static_assert(kPatMax <= kThreads, "one length per thread");
+  if (*in.vok == 0) {
+    for (uint32_t i = r0 + tid; i < r0 + nr; i += kThreads) {
+      double t = (MODE == ROW_AX) ? 0.0 : (double)bf(i);
+      const uint32_t s = in.rp[i], e = in.rp[i + 1];
+      for (uint32_t k = s; k < e; ++k) {
+        const double a = (double)in.va[k], x = (double)xf(in.ci[k]);
+        if (MODE == ROW_AX)
+          t = (k == s) ? a * x : fma(a, x, t);
+        else
+          t = fma(-a, x, t);
+      }
+      epi.row(i, t, acc);
+    }
+    return;
+  }
+  auto pid_at = [&](uint32_t i) { return (uint32_t)in.pid[r0 + min(i, nr - 1)]; };
+  uint32_t pidv[P];
+#pragma unroll
+  for (int q = 0; q < P; ++q) pidv[q] = pid_at(tid + q * kThreads);
+  int32_t dv[kDv];
+  MT vv[kDv];
+#pragma unroll
+  for (int j = 0; j < kDv; ++j) {
+    const uint32_t i = min((uint32_t)(tid + j * kThreads), in.npat * in.vstride - 1);
+    dv[j] = in.vdict[i];
+    vv[j] = in.pval[i];
+  }
+  const uint32_t cnt = in.pcnt[min((uint32_t)tid, in.npat - 1)];
+#pragma unroll
+  for (int j = 0; j < kDv; ++j) {  // slots past the end: copies of the last, never read
+    lds.dict[tid + j * kThreads] = dv[j];
+    lds.va[tid + j * kThreads] = vv[j];
+  }
+  if (tid < (int)kPatMax) lds.rp[tid] = cnt;
+  __syncthreads();
+  if (in.vstride == 8) {
+#pragma unroll 1
+    for (int h = 0; h < H; ++h) {
+      const uint32_t rbase = tid + h * P * kThreads;
+      if (h * P * kThreads >= nr) break;  // uniform
+      uint32_t len[P];
+      std::decay_t<decltype(xf(0u))> xv[P][8];
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const uint32_t ri = r0 + rbase + q * kThreads;
+        len[q] = rbase + q * kThreads < nr ? lds.rp[pidv[q]] : 0u;
+        const int4* pd = reinterpret_cast<const int4*>(lds.dict + pidv[q] * 8);
+        const int4 o0 = pd[0], o1 = pd[1];
+        const int off[8] = {o0.x, o0.y, o0.z, o0.w, o1.x, o1.y, o1.z, o1.w};
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+          if ((uint32_t)j < in.plen) xv[q][j] = xf(len[q] ? ri + (uint32_t)off[j] : 0u);
+      }
+      uint32_t pnext[P];
+#pragma unroll
+      for (int q = 0; q < P; ++q) pnext[q] = pid_at(rbase + (P + q) * kThreads);
+#pragma unroll
+      for (int q = 0; q < P; ++q) {
+        const uint32_t ri = r0 + rbase + q * kThreads;
+        if (rbase + q * kThreads < nr) {
+          const MT* pv = lds.va + pidv[q] * 8;
+          double t = (MODE == ROW_AX) ? 0.0 : (double)bf(ri);
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            if ((uint32_t)j < len[q]) {
+              const double a = (double)pv[j], x = (double)xv[q][j];
+              if (MODE == ROW_AX)
+                t = (j == 0) ? a * x : fma(a, x, t);
+              else
+                t = fma(-a, x, t);
+            }
+          }
+          epi.row(ri, t, acc);
+        }
+        pidv[q] = pnext[q];
+      }
+    }
+    return;
+  }
+#pragma unroll 1
+  for (uint32_t i = tid; i < nr; i += kThreads) {
+    const uint32_t ri = r0 + i, p = in.pid[ri], len = lds.rp[p];
+    const int32_t* pd = lds.dict + p * in.vstride;
+    const MT* pv = lds.va + p * in.vstride;
+    double t = (MODE == ROW_AX) ? 0.0 : (double)bf(ri);
+    for (uint32_t base = 0; base < len; base += 8) {
+      std::decay_t<decltype(xf(0u))> xv[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) xv[j] = xf(ri + (uint32_t)pd[min(base + j, len - 1)]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const uint32_t k = base + j;
+        if (k < len) {
+          const double a = (double)pv[k], x = (double)xv[j];
+          if (MODE == ROW_AX)
+            t = (k == 0) ? a * x : fma(a, x, t);
+          else
+            t = fma(-a, x, t);
+        }
+      }
+    }
+    epi.row(ri, t, acc);
+  }
+}
+
 // Rows longer than this in a sliced-row window are summed by the whole
 // workgroup rather than by one wave.
 #ifndef FX_SELL_HUGE
@@ -580,7 +721,7 @@ __device__ __forceinline__ void emit_row(const Epi& epi, uint32_t pos, uint32_t 
 //   void fin(double (&sum)[NRED])          run by k_finish after the kernel
 template <class MT, class VT, int MODE, int NRED, unsigned MAXMASK, class XF, class BF, class Epi,
           int CF>
-__global__ __launch_bounds__(kThreads) void k_spmv(SpmvIn<MT, VT> in, XF xf0, BF bf, Epi epi0,
+__global__ __launch_bounds__(kThreads, CF == CF_ROWVAL ? 8 : 1) void k_spmv(SpmvIn<MT, VT> in, XF xf0, BF bf, Epi epi0,
                                                    double* partials) {
   if (epi0.skip()) return;
   XF xf = xf0;
@@ -596,6 +737,11 @@ __global__ __launch_bounds__(kThreads) void k_spmv(SpmvIn<MT, VT> in, XF xf0, BF
   const int tid = threadIdx.x;
   if constexpr (CF == CF_SELL) {
     if (bid < in.nblk) sell_block<MODE, NRED>(in, bid, tid, xf, bf, epi, acc);
+  } else if constexpr (CF == CF_ROWVAL) {
+    const uint32_t r0 = bid * kRowValRows;  // row blocks of their own
+    if (r0 < in.nrow)
+      row_value_block<MODE, NRED>(in, lds, r0, min(kRowValRows, in.nrow - r0), tid, xf, bf, epi,
+                                  acc);
   } else if (bid < in.nblk) {
     const uint32_t r0 = in.blk[2 * bid], k0 = in.blk[2 * bid + 1];
     const uint32_t r1 = in.blk[2 * bid + 2], k1 = in.blk[2 * bid + 3];
@@ -816,7 +962,10 @@ template <class MT, class VT, int MODE, int NRED, unsigned MAXMASK, class XF, cl
 inline int launch_spmv(fx_csr A, hipStream_t st, XF xf, BF bf, Epi epi, double* partials,
                        hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, bool finisher = true) {
   const unsigned g = spmv_grid_of<MT>(A, A->ctx->sms);
-  if (A->pid && sizeof(MT) == 4 && A->pat_rows == kPat2Rows)  // f32 copies only
+  if (has_row_values<MT>(A))
+    launch_spmv_k<MT, VT, MODE, NRED, MAXMASK, XF, BF, Epi, CF_ROWVAL>(A, st, xf, bf, epi,
+                                                                       partials, e0, e1, g);
+  else if (A->pid && sizeof(MT) == 4 && A->pat_rows == kPat2Rows)  // f32 copies only
     launch_spmv_k<MT, VT, MODE, NRED, MAXMASK, XF, BF, Epi,
                   sizeof(MT) == 4 ? CF_PAT2 : CF_PAT>(A, st, xf, bf, epi, partials, e0, e1, g);
   else if (A->pid)

@@ -186,7 +186,10 @@ int fx_csr_info(fx_csr A, uint32_t* nrow, uint32_t* mcol, uint32_t* nnz);
  * all: one pattern byte per row instead), 2 when every row block's columns
  * lie within 32K of the block's first row (16-bit deltas), else 4.
  * Environment at creation: FASPXX_FX_NOPAT=1 disables row patterns,
- * FASPXX_FX_COL32=1 keeps 4.  All forms give the same bits.  No reference
+ * FASPXX_FX_NOROWVAL=1 the row values (a row-pattern matrix of more than
+ * 262144 rows whose rows of one pattern hold the same values is read from a
+ * dictionary until its values change), FASPXX_FX_COL32=1 keeps 4.  All forms
+ * give the same bits.  No reference
  * counterpart (the reference stores u32 columns only, src/MAT.hxx:43-47). */
 int fx_csr_index_bytes(fx_csr A, int* bytes);
 /* How the SpMV kernels read the matrix: FX_LAYOUT_U32 (row blocks, u32
@@ -217,7 +220,9 @@ int fx_csr_download(fx_csr A, uint32_t* rowPtr, uint32_t* colInd, double* values
 /* Replace the f64 values from device memory (nnz doubles) on the context
  * stream; refreshes the f32 copy if one exists. */
 int fx_csr_set_values_dev(fx_csr A, const double* dev_values);
-/* Device pointer to the f64 values (nnz doubles). */
+/* Device pointer to the f64 values (nnz doubles).  Values written through it
+ * are seen by the f64 SpMV of a matrix without sorted or sliced rows; call
+ * fx_csr_set_values_dev with it to refresh every copy. */
 double* fx_csr_values_dev(fx_csr A);
 /* Build (or rebuild) the f32 value copy used by f32 SpMV / mixed precision. */
 int fx_csr_make_f32(fx_csr A);
