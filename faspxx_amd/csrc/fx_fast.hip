@@ -26,6 +26,7 @@
 #include <cstring>
 
 #include "fx_fast.hpp"
+#include "fx_resident.hpp"
 
 namespace fx {
 
@@ -91,9 +92,27 @@ __device__ __forceinline__ void cg_loop_top(CgState* S, const CgPrm& P, double r
   }
 }
 
+// The quotients and roots of the end-of-iteration logic, formed where they
+// are asked for (one thread taking the decision).
+struct CgQuotients {
+  __device__ __forceinline__ double resAbs(double rr) const { return sqrt(rr); }
+  __device__ __forceinline__ double resRel(double ra, const CgState* S) const {
+    return ra / S->denAbs;
+  }
+  __device__ __forceinline__ double ratio(double ra, const CgState* S) const {
+    return ra / S->resAbsOld;
+  }
+  __device__ __forceinline__ double xRelDiff(const CgState* S, const double (&a)[5]) const {
+    return fabs(S->alpha) * sqrt(a[4]) / sqrt(a[3]);
+  }
+  __device__ __forceinline__ double beta(double rz, const CgState* S) const { return rz / S->tmpa; }
+};
+
 // End-of-iteration logic of src/CG.cxx:130-234 for the common case; any rare
 // branch hands the whole step to the host (which recomputes it from S).
-__device__ __forceinline__ void cg_after_update(CgState* S, const CgPrm& P, const double (&a)[5], double* hist) {
+template <class Q = CgQuotients>
+__device__ __forceinline__ void cg_after_update(CgState* S, const CgPrm& P, const double (&a)[5],
+                                                double* hist, const Q& quot = Q{}) {
   S->rr = a[0];
   S->rz = a[1];
   S->xinf = a[2];
@@ -101,14 +120,14 @@ __device__ __forceinline__ void cg_after_update(CgState* S, const CgPrm& P, cons
   S->pp = a[4];
   const uint32_t it = S->numIter;
   if (it >= P.minIter) {
-    const double resAbs = sqrt(a[0]);
-    const double resRel = resAbs / S->denAbs;
-    const double ratio = resAbs / S->resAbsOld;
+    const double resAbs = quot.resAbs(a[0]);
+    const double resRel = quot.resRel(resAbs, S);
+    const double ratio = quot.ratio(resAbs, S);
     bool host = false;
     if (it >= P.savIter && resAbs < S->resAbsOld) host = true;
     if (ratio > kChkRatio) {
       if (a[2] < kCloseZero) host = true;
-      const double xRelDiff = fabs(S->alpha) * sqrt(a[4]) / sqrt(a[3]);
+      const double xRelDiff = quot.xRelDiff(S, a);
       if (S->stagStep <= kMaxStag && xRelDiff < P.solStagTol) host = true;
     }
     if (resRel < P.relTol) host = true;
@@ -123,7 +142,7 @@ __device__ __forceinline__ void cg_after_update(CgState* S, const CgPrm& P, cons
   }
   if (it < P.maxIter) {
     S->resAbsOld = S->resAbs;
-    S->beta = a[1] / S->tmpa;
+    S->beta = quot.beta(a[1], S);
     S->tmpa = a[1];
   } else {
     S->status = ST_DONE;
@@ -386,6 +405,163 @@ __global__ __launch_bounds__(kWideThreads) void k_cg_pupdate_w(
   if (blockIdx.x == 0 && threadIdx.x < n - nc * W) {
     const uint32_t i = nc * W + threadIdx.x;
     p[i] = fma(beta, p[i], (JAC && !SW) ? r[i] * dinv[i] : r[i]);
+  }
+}
+
+// ---- the resident iteration ---------------------------------------------------
+// The same iteration with x, r, dinv in registers and p in LDS, up to
+// max_it of them per launch (fx_resident.hpp).  p is exported after each
+// update for the gathers of other workgroups; the two reductions are
+// exchanges.  Per element the arithmetic, and per iteration the decisions,
+// are those of the three kernels above; every workgroup takes the decisions
+// for itself from the same sums.  On leaving, x, r, q and the state are where
+// the three kernels would have left them.
+
+// The quotients of cg_after_update formed by the lanes of one wave at once:
+// one square root and one division of latency instead of four of each.
+struct CgQuotientsWave {
+  double ra, rel, rat, xrel, bet;
+  __device__ __forceinline__ CgQuotientsWave(const CgState* S, const double (&a)[5], int lane) {
+    const double a1 = res_value(a[1]), a3 = res_value(a[3]), a4 = res_value(a[4]);
+    double square = res_value(a[0]);
+    if (lane == 1) square = a4;
+    if (lane == 2) square = a3;
+    const double root = sqrt(square);
+    ra = res_lane(root, 0);
+    double num = ra, den = S->denAbs;
+    if (lane == 1) den = S->resAbsOld;
+    if (lane == 2) {
+      num = fabs(S->alpha) * res_lane(root, 1);
+      den = res_lane(root, 2);
+    }
+    if (lane == 3) {
+      num = a1;
+      den = S->tmpa;
+    }
+    const double q = num / den;
+    rel = res_lane(q, 0);
+    rat = res_lane(q, 1);
+    xrel = res_lane(q, 2);
+    bet = res_lane(q, 3);
+  }
+  __device__ __forceinline__ double resAbs(double) const { return ra; }
+  __device__ __forceinline__ double resRel(double, const CgState*) const { return rel; }
+  __device__ __forceinline__ double ratio(double, const CgState*) const { return rat; }
+  __device__ __forceinline__ double xRelDiff(const CgState*, const double (&)[5]) const {
+    return xrel;
+  }
+  __device__ __forceinline__ double beta(double, const CgState*) const { return bet; }
+};
+
+template <int R, int MM>
+__global__ __launch_bounds__(kResThreads) void k_cg_resident(
+    ResMat A, double* __restrict__ x, double* __restrict__ r, double* p, double* __restrict__ q,
+    const double* __restrict__ dinv, CgState* st, CgState* hout, CgPrm P, double* hist,
+    ResComm cm, uint32_t max_it) {
+  constexpr bool kRl = R == 8;  // r in LDS too: eight rows' vectors do not fit the registers
+  __shared__ double pl[R * kResThreads];
+  __shared__ double rl[kRl ? R * kResThreads : 1];
+  __shared__ typename ResRows<double, R, MM>::Lds ml;
+  __shared__ ResShared sh;
+  __shared__ CgState S;
+  __shared__ int run;
+  const uint32_t tid = threadIdx.x, base = blockIdx.x * R * kResThreads, n = A.n;
+  const int lane = tid & 63;
+  ResRows<double, R, MM> rows;
+  uint32_t wlo, whi;
+  if (tid == 0) {
+    S = *st;
+    run = S.status == ST_RUN;
+  }
+  rows.load(A, ml, wlo, whi);
+  if (!run) {  // uniform over the launch
+    if (blockIdx.x == 0 && tid == 0) *hout = S;
+    return;
+  }
+  double xv[R], rv[kRl ? 1 : R], dv[R], qv[R];
+  auto rr = [&](int k) -> double& {
+    if constexpr (kRl) return rl[k * kResThreads + tid];
+    else return rv[k];
+  };
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const uint32_t i = base + k * kResThreads + tid;
+    const bool has = i < n;
+    xv[k] = has ? x[i] : 0.0;
+    rr(k) = has ? r[i] : 0.0;
+    dv[k] = has && dinv ? dinv[i] : 1.0;  // r * 1 = r: the identity
+    qv[k] = 0.0;
+    pl[k * kResThreads + tid] = has ? p[i] : 0.0;
+  }
+  __syncthreads();
+  uint32_t t = 0;  // reductions so far
+  bool ok = true;
+  for (uint32_t it = 0; it < max_it; ++it) {
+    rows.template product<false>(A, ml, pl, (const double*)p, qv);
+    double pq[1] = {0.0};
+#pragma unroll
+    for (int k = 0; k < R; ++k) pq[0] = fma(qv[k], pl[k * kResThreads + tid], pq[0]);
+    ok = res_allreduce<1, 0u>(pq, cm, t++, sh);
+    if (!ok) break;
+    if (!(fabs(pq[0]) > kCloseZero * kCloseZero)) {  // src/CG.cxx:114-119
+      if (tid == 0) {
+        S.numIter += 1;
+        S.pq = pq[0];
+        S.status = ST_HOST;
+        S.reason = R_BREAKDOWN;
+      }
+      break;
+    }
+    const double alpha = S.tmpa / pq[0];
+    const CgUpd<double, true> u{alpha};
+    double a[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      double rk = rr(k);
+      u.elem(pl[k * kResThreads + tid], qv[k], xv[k], rk, dv[k], a);
+      rr(k) = rk;
+    }
+    ok = res_allreduce<5, 4u>(a, cm, t++, sh);
+    if (!ok) break;
+    if (tid < 64) {
+      if (tid == 0) {
+        S.numIter += 1;
+        S.pq = pq[0];
+        S.alpha = alpha;
+      }
+      __builtin_amdgcn_wave_barrier();
+      const CgQuotientsWave quot(&S, a, lane);
+      if (tid == 0) {
+        cg_after_update(&S, P, a, blockIdx.x == 0 ? hist : nullptr, quot);
+        run = S.status == ST_RUN;
+      }
+    }
+    __syncthreads();
+    if (!run) break;
+    const double beta = S.beta;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const uint32_t i = base + k * kResThreads + tid;
+      const double pv = fma(beta, pl[k * kResThreads + tid], rr(k) * dv[k]);
+      pl[k * kResThreads + tid] = pv;
+      if (i < n) res_store(p + i, pv);
+    }
+    ok = res_exchange(cm, it + 1, wlo, whi, sh);
+    if (!ok) break;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const uint32_t i = base + k * kResThreads + tid;
+    if (i < n) {
+      x[i] = xv[k];
+      r[i] = rr(k);
+      q[i] = qv[k];
+    }
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    *st = S;
+    *hout = S;
   }
 }
 
@@ -1293,6 +1469,51 @@ struct CgRun {
     return 0;
   }
 
+  // One launch of the resident loop (f64) and the state it left; *held =
+  // false when the device cannot hold it.  A wait that gave up is an error of the device.
+  int run_resident(bool* held, CgState* out) {
+    if constexpr (std::is_same_v<VT, double>) {
+      const ResShape rs = res_shape(W.n, W.ctx->sms);
+      const int mode = res_mode<double>(A, rs.rows);
+      const void* k = nullptr;
+      auto pick = [&](auto R) {
+        constexpr int r = decltype(R)::value;
+        if constexpr (r <= 2)
+          if (mode == RM_REG) k = (const void*)&k_cg_resident<r, RM_REG>;
+        if constexpr (r >= 2) {
+          if (mode == RM_VAL) k = (const void*)&k_cg_resident<r, RM_VAL>;
+        }
+        if (mode == RM_MEM) k = (const void*)&k_cg_resident<r, RM_MEM>;
+      };
+      if (rs.rows == 1) pick(std::integral_constant<int, 1>{});
+      if (rs.rows == 2) pick(std::integral_constant<int, 2>{});
+      if (rs.rows == 4) pick(std::integral_constant<int, 4>{});
+      if (rs.rows == 8) pick(std::integral_constant<int, 8>{});
+      if (!k) {
+        *held = false;
+        return 0;
+      }
+      ResMat M = res_mat<double>(A);
+      ResComm cm = res_comm(W.comm);
+      double *x = (double*)W.x, *r = (double*)W.r, *p = (double*)W.p, *q = (double*)W.q;
+      const double* d = dinv;
+      CgState *ds = dstate(), *hs = hslot(0);
+      uint32_t most = kResLaunchIters;
+      void* args[] = {&M, &x, &r, &p, &q, &d, &ds, &hs, &P, &W.hist, &cm, &most};
+      const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args);
+      if (rc < 0) return rc;
+      *held = rc == 0;
+      if (*held) {
+        unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
+        FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
+        FX_HIP(hipStreamSynchronize(st));
+        FX_CHECK(*fail == 0, FX_ERROR_DEVICE, "a wait of the resident CG loop gave up");
+        *out = *hslot(0);
+      }
+    }
+    return 0;
+  }
+
   // x_user (in/out), b_user: device pointers of dtype VT.
   int run(const VT* b, VT* x_user, fx_result* res, const fx_params& PP, int pc_dtype) {
     const uint32_t n = W.n;
@@ -1356,8 +1577,27 @@ struct CgRun {
     // kChunk replays; every host step is preceded by at least one iteration,
     // so there are at most maxIter of them.
     const uint64_t max_chunks = (uint64_t)PP.maxIter / kChunk + 4;
-    uint64_t host_steps = 0;
+    uint64_t host_steps = 0, launches = 0;
+    bool resident = W.resident;
     for (;;) {
+      if (resident) {
+        bool held = true;
+        FX_TRY(run_resident(&held, &s));
+        if (!held) {  // the launch does not fit this device: kernel by kernel
+          W.resident = resident = false;
+          continue;
+        }
+        if (s.status == ST_RUN) {  // a full launch: its iterations are done
+          FX_CHECK(++launches <= (uint64_t)PP.maxIter / kResLaunchIters + 4 + host_steps,
+                   FX_ERROR_DEVICE, "resident CG loop did not stop");
+          continue;
+        }
+        FX_CHECK(++host_steps <= (uint64_t)PP.maxIter + 2, FX_ERROR_DEVICE,
+                 "CG device loop did not stop");
+        if (s.status == ST_DONE || host_step(s, vb, vx, vr, vp, vq, vs, o, PP)) break;
+        FX_TRY(write_state(s));
+        continue;
+      }
       ReplayPace pace;
       pace.hint = host_steps == 0 ? W.last_iters : 0;
       // the iteration that hands the loop's end to the host is numbered
@@ -1598,6 +1838,13 @@ int fast_solve(fx_solver S, fx_vec b, fx_vec x, fx_result* res) {
     }
   }
   FastWs& W = *S->fast;
+  // resident loops: a banded matrix of short rows that fits the chip
+  if (!W.comm && !S->op && S->type == FX_SOLVER_CG && !resident_disabled() &&
+      !(S->pc->kind == 1 && S->pc->iters > 1) && res_matrix_ok(S->A) &&
+      res_shape(n, S->ctx->sms).rows) {
+    FX_HIP(hipMalloc(&W.comm, kResCommWords * sizeof(unsigned long long)));
+    W.resident = true;
+  }
   if (S->type == FX_SOLVER_JACOBI) return jacobi_run(S, W, (const double*)b->d, (double*)x->d, res);
   if (S->type == FX_SOLVER_BICGSTAB)
     return bicgstab_fast(S, W, (const double*)b->d, (double*)x->d, res);

@@ -157,6 +157,8 @@ struct FastWs {
   void* gm = nullptr;          // GMRES basis and cycle graphs (fx_gmres.hip)
   void* opy = nullptr;         // callback operator: apply's output
   void* opx = nullptr;         // callback operator: an operand formed before apply
+  void* comm = nullptr;        // exchanges of the resident loop (fx_resident.hpp)
+  bool resident = false;       // the loop runs resident
   size_t part2_off = 0;        // second partials region (doubles)
   uint32_t last_iters = 0;     // iterations of the last solve on this workspace
   hipGraphExec_t chunk[2] = {nullptr, nullptr};  // replay graphs, one per host state slot
@@ -172,7 +174,7 @@ inline FastWs::~FastWs() {
   {
     if (ctx) (void)hipStreamSynchronize(ctx->stream);
     gmres_ws_free(gm);
-    void* bufs[] = {x, x2, r, p, q, safe, s, t, partials, state, hist, dscal, side, opy, opx};
+    void* bufs[] = {x, x2, r, p, q, safe, s, t, partials, state, hist, dscal, side, opy, opx, comm};
     for (void* b : bufs) (void)hipFree(b);
     if (hstate) (void)hipHostFree(hstate);
     for (auto& c : chunk)
