@@ -501,19 +501,20 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
     double pq[1] = {0.0};
 #pragma unroll
     for (int k = 0; k < R; ++k) pq[0] = fma(qv[k], pl[k * kResThreads + tid], pq[0]);
-    ok = res_allreduce<1, 0u>(pq, cm, t++, sh);
-    if (!ok) break;
-    if (!(fabs(pq[0]) > kCloseZero * kCloseZero)) {  // src/CG.cxx:114-119
-      if (tid == 0) {
-        S.numIter += 1;
-        S.pq = pq[0];
+    ok = res_allreduce<1, 0u>(pq, cm, t++, sh, [&](const double (&tot)[1]) {
+      if (lane != 0) return;
+      S.numIter += 1;
+      S.pq = tot[0];
+      if (!(fabs(tot[0]) > kCloseZero * kCloseZero)) {  // src/CG.cxx:114-119
         S.status = ST_HOST;
         S.reason = R_BREAKDOWN;
+        run = 0;
+      } else {
+        S.alpha = S.tmpa / tot[0];
       }
-      break;
-    }
-    const double alpha = S.tmpa / pq[0];
-    const CgUpd<double, true> u{alpha};
+    });
+    if (!ok || !run) break;
+    const CgUpd<double, true> u{S.alpha};
     double a[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < R; ++k) {
@@ -521,23 +522,13 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
       u.elem(pl[k * kResThreads + tid], qv[k], xv[k], rk, dv[k], a);
       rr(k) = rk;
     }
-    ok = res_allreduce<5, 4u>(a, cm, t++, sh);
-    if (!ok) break;
-    if (tid < 64) {
-      if (tid == 0) {
-        S.numIter += 1;
-        S.pq = pq[0];
-        S.alpha = alpha;
-      }
-      __builtin_amdgcn_wave_barrier();
-      const CgQuotientsWave quot(&S, a, lane);
-      if (tid == 0) {
-        cg_after_update(&S, P, a, blockIdx.x == 0 ? hist : nullptr, quot);
-        run = S.status == ST_RUN;
-      }
-    }
-    __syncthreads();
-    if (!run) break;
+    ok = res_allreduce<5, 4u>(a, cm, t++, sh, [&](const double (&tot)[5]) {
+      const CgQuotientsWave quot(&S, tot, lane);
+      if (lane != 0) return;
+      cg_after_update(&S, P, tot, blockIdx.x == 0 ? hist : nullptr, quot);
+      run = S.status == ST_RUN;
+    });
+    if (!ok || !run) break;
     const double beta = S.beta;
 #pragma unroll
     for (int k = 0; k < R; ++k) {
@@ -1180,6 +1171,126 @@ __global__ __launch_bounds__(kWideThreads) void k_ir_update(
   }
 }
 
+// The same inner iteration with r in LDS and w, s, p, y in registers, up to
+// max_it per launch (fx_resident.hpp): r is exported after each update for
+// the gathers of other workgroups, and (w, r), (r, r) are one exchange.  p
+// and y are formed in every iteration (they cost no memory here), with
+// ir_elem's roundings in the same order, so that y is whole on leaving.
+template <int R, int MM>
+__global__ __launch_bounds__(kResThreads) void k_ir_resident(ResMat A, float* r, float* p,
+                                                             float* s, float* y, IrState* st,
+                                                             IrState* hout, ResComm cm,
+                                                             uint32_t max_it) {
+  __shared__ float rl[R * kResThreads];
+  __shared__ typename ResRows<float, R, MM>::Lds ml;
+  __shared__ ResShared sh;
+  __shared__ IrState S;
+  __shared__ float sa, sb;
+  __shared__ int run;
+  const uint32_t tid = threadIdx.x, base = blockIdx.x * R * kResThreads, n = A.n;
+  const int lane = tid & 63;
+  ResRows<float, R, MM> rows;
+  uint32_t wlo, whi;
+  if (tid == 0) {
+    S = *st;
+    run = S.status == ST_RUN;
+  }
+  rows.load(A, ml, wlo, whi);
+  if (!run) {  // uniform over the launch
+    if (blockIdx.x == 0 && tid == 0) *hout = S;
+    return;
+  }
+  const bool begun = S.numIter > 0;  // a launch that goes on from an earlier one
+  float pv[R], sv[R], yv[R];
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const uint32_t i = base + k * kResThreads + tid;
+    const bool has = i < n;
+    pv[k] = has && begun ? p[i] : 0.0f;
+    sv[k] = has && begun ? s[i] : 0.0f;
+    yv[k] = has && begun ? y[i] : 0.0f;
+    rl[k * kResThreads + tid] = has ? r[i] : 0.0f;
+  }
+  __syncthreads();
+  bool ok = true;
+  for (uint32_t it = 0; it < max_it; ++it) {
+    double wv[R];
+    rows.template product<false>(A, ml, rl, (const float*)r, wv);
+    double v[2] = {0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const double rk = (double)rl[k * kResThreads + tid];
+      wv[k] = (double)(float)wv[k];
+      v[0] = fma(wv[k], rk, v[0]);
+      v[1] = fma(rk, rk, v[1]);
+    }
+    ok = res_allreduce<2, 0u>(v, cm, it, sh, [&](const double (&tot)[2]) {
+      if (lane != 0) return;
+      const double delta = tot[0], gamma = S.numIter > 0 ? tot[1] : S.gamma0;
+      S.gamma = gamma;
+      S.delta = delta;
+      int stop = -1;
+      double alpha = 0.0, beta = 0.0;
+      if (gamma < S.thr || gamma == 0.0) {
+        stop = IR_CONVERGED;
+      } else if (S.numIter >= S.maxIter) {
+        stop = IR_MAXIT;
+      } else {
+        double den = delta;
+        if (S.numIter > 0) {
+          beta = gamma / S.gamma_prev;
+          den = delta - beta * gamma / S.alpha_prev;
+        }
+        alpha = gamma / den;
+        if (!(den > 0.0) || !(fabs(alpha) < INFINITY) || !(fabs(beta) < INFINITY))
+          stop = IR_BREAKDOWN;
+      }
+      if (stop >= 0) {
+        S.status = ST_DONE;
+        S.reason = stop;
+        run = 0;
+        return;
+      }
+      sa = (float)alpha;
+      sb = (float)beta;
+      S.gamma_prev = gamma;
+      S.alpha_prev = alpha;
+      S.beta_prev = beta;
+      S.numIter += 1;
+    });
+    if (!ok || !run) break;
+    const bool first = S.numIter == 1;
+    const float a = sa, b = sb;
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const uint32_t i = base + k * kResThreads + tid;
+      float rk = rl[k * kResThreads + tid];
+      pv[k] = first ? rk : fma(b, pv[k], rk);
+      yv[k] = first ? a * pv[k] : fma(a, pv[k], yv[k]);
+      sv[k] = first ? (float)wv[k] : fma(b, sv[k], (float)wv[k]);
+      rk = fma(-a, sv[k], rk);
+      rl[k * kResThreads + tid] = rk;
+      if (i < n) res_store(r + i, rk);
+    }
+    ok = res_exchange(cm, it + 1, wlo, whi, sh);
+    if (!ok) break;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const uint32_t i = base + k * kResThreads + tid;
+    if (i < n) {
+      p[i] = pv[k];
+      s[i] = sv[k];
+      y[i] = yv[k];
+    }
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    *st = S;
+    *hout = S;
+  }
+}
+
 // x += s_i d_i: the scaled correction back in the unscaled unknowns.
 // x += S y; with cs, only after an inner solve that ran at least one
 // iteration to its end (y holds that solve's increment).  fin: the inner
@@ -1187,18 +1298,19 @@ __global__ __launch_bounds__(kWideThreads) void k_ir_update(
 // forms p and y two iterations at a time) the last iteration's p and
 // alpha p are still to be formed, as ir_elem would: p_{m-1} =
 // fma(beta, p_{m-2}, r_{m-1}) with r_{m-1} in ra (r_0 when m == 1), then
-// y = fma(alpha, p_{m-1}, y) (alpha p_0 when m == 1).
+// y = fma(alpha, p_{m-1}, y) (alpha p_0 when m == 1).  whole: y is complete
+// (k_ir_resident).
 __global__ void k_ir_add_scaled(double* __restrict__ x, const double* __restrict__ sc,
                                 const float* __restrict__ y, const float* __restrict__ p,
                                 const float* __restrict__ ra, uint32_t n, const IrState* cs,
-                                const IrState* fin) {
+                                const IrState* fin, int whole) {
   if (cs && (ir_inner_open(cs) || cs->numIter == 0)) return;
   const uint32_t m = fin->numIter;
-  const bool pend = (m & 1u) != 0;
+  const bool pend = !whole && (m & 1u) != 0;
   const float ap = (float)fin->alpha_prev, bp = (float)fin->beta_prev;
   const uint32_t stride = gridDim.x * kThreads;
   for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
-    float yi = m == 1 ? 0.0f : y[i];
+    float yi = m == 1 && !whole ? 0.0f : y[i];
     if (pend) {
       const float pm = m == 1 ? ra[i] : fma(bp, p[i], ra[i]);
       yi = m == 1 ? ap * pm : fma(ap, pm, yi);
@@ -1474,21 +1586,9 @@ struct CgRun {
   int run_resident(bool* held, CgState* out) {
     if constexpr (std::is_same_v<VT, double>) {
       const ResShape rs = res_shape(W.n, W.ctx->sms);
-      const int mode = res_mode<double>(A, rs.rows);
-      const void* k = nullptr;
-      auto pick = [&](auto R) {
-        constexpr int r = decltype(R)::value;
-        if constexpr (r <= 2)
-          if (mode == RM_REG) k = (const void*)&k_cg_resident<r, RM_REG>;
-        if constexpr (r >= 2) {
-          if (mode == RM_VAL) k = (const void*)&k_cg_resident<r, RM_VAL>;
-        }
-        if (mode == RM_MEM) k = (const void*)&k_cg_resident<r, RM_MEM>;
-      };
-      if (rs.rows == 1) pick(std::integral_constant<int, 1>{});
-      if (rs.rows == 2) pick(std::integral_constant<int, 2>{});
-      if (rs.rows == 4) pick(std::integral_constant<int, 4>{});
-      if (rs.rows == 8) pick(std::integral_constant<int, 8>{});
+      const void* k = res_pick(rs.rows, res_mode<double>(A, rs.rows), [](auto r, auto m) {
+        return (const void*)&k_cg_resident<decltype(r)::value, decltype(m)::value>;
+      });
       if (!k) {
         *held = false;
         return 0;
@@ -1763,6 +1863,44 @@ struct IrInner {
     return 0;
   }
 
+  // The resident loop, a launch of kResLaunchIters iterations at a time; the
+  // work behind is queued behind the first launch, to act if that one ends
+  // the loop.  *held = false when the device cannot hold it.
+  int run_resident(uint32_t maxIter, IrState& out, const std::function<int()>& behind,
+                   bool* behind_ran, bool* held) {
+    const ResShape rs = res_shape(W.n, W.ctx->sms);
+    const void* k = res_pick(rs.rows, res_mode<float>(As, rs.rows), [](auto r, auto m) {
+      return (const void*)&k_ir_resident<decltype(r)::value, decltype(m)::value>;
+    });
+    ResMat M = res_mat<float>(As);
+    ResComm cm = res_comm(W.comm);
+    float *r = (float*)W.r, *p = (float*)W.p, *s = (float*)W.x2, *y = (float*)W.x;
+    IrState *ds = dstate(0), *hs = hslot(0);
+    uint32_t most = kResLaunchIters;
+    void* args[] = {&M, &r, &p, &s, &y, &ds, &hs, &cm, &most};
+    if (behind_ran) *behind_ran = false;
+    const uint64_t max_launches = (uint64_t)maxIter / kResLaunchIters + 4;
+    for (uint64_t l = 0;; ++l) {
+      FX_CHECK(l <= max_launches, FX_ERROR_DEVICE, "resident IR inner loop did not stop");
+      const int rc = k ? res_launch(W.ctx, k, rs.wgs, W.comm, args) : 1;
+      if (rc < 0) return rc;
+      FX_CHECK(rc == 0 || l == 0, FX_ERROR_DEVICE, "resident IR inner loop: no launch");
+      *held = rc == 0;
+      if (!*held) return 0;
+      unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
+      FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
+      FX_HIP(hipEventRecord(W.ev[0], st));
+      if (l == 0 && behind) FX_TRY(behind());
+      FX_HIP(hipEventSynchronize(W.ev[0]));
+      FX_CHECK(*fail == 0, FX_ERROR_DEVICE, "a wait of the resident IR inner loop gave up");
+      out = *hs;
+      if (out.status != ST_RUN) {
+        if (behind_ran) *behind_ran = l == 0 && (bool)behind;
+        return 0;
+      }
+    }
+  }
+
   // Replays until the device loop stops; out = the final state.  A replay
   // that finds the loop running advances it, so it stops within maxIter /
   // kChunk + 1 replays after the predicted ones.
@@ -1773,6 +1911,12 @@ struct IrInner {
   // behind / behind_ran: see replay_loop.
   int run(uint32_t maxIter, IrState& out, uint32_t hint,
           const std::function<int()>& behind = nullptr, bool* behind_ran = nullptr) {
+    if (W.resident) {
+      bool held = true;
+      FX_TRY(run_resident(maxIter, out, behind, behind_ran, &held));
+      if (held) return 0;
+      W.resident = false;  // the launch does not fit this device: kernel by kernel
+    }
     ReplayPace pace;
     pace.hint = hint;
     const uint64_t need = hint ? (uint64_t)hint + 1 : 0;
@@ -2053,6 +2197,18 @@ int fx_ir_create(fx_ctx ctx, int inner_type, fx_csr A, double weight, const fx_p
     const size_t sb = sizeof(CgState) > sizeof(IrState) ? sizeof(CgState) : sizeof(IrState);
     rc = ws_alloc(*ir->W, ctx, FX_F32, n, inner->maxIter, sb, spmv_grid_max<float>(A));
     if (rc) return fail(rc);
+    // resident inner loop; eight rows per thread whose values are re-read
+    // from memory spill too many registers (1400^2 variable coefficients:
+    // 41 against 28 us per iteration kernel by kernel)
+    const ResShape rs = res_shape(n, ctx->sms);
+    if (ir->scaled && !resident_disabled() && res_matrix_ok(A) && rs.rows &&
+        !(rs.rows == 8 && res_mode<float>(&ir->As, rs.rows) == RM_MEM)) {
+      if (hipMalloc(&ir->W->comm, kResCommWords * sizeof(unsigned long long))) {
+        set_error("IR workspace allocation failed");
+        return fail(FX_ERROR_ALLOC_MEM);
+      }
+      ir->W->resident = true;
+    }
     // the scaled inner solve's second r buffer (odd iterations' r)
     if (ir->scaled && hipMalloc(&ir->W->s, sizeof(float) * pack_round(n))) {
       set_error("IR workspace allocation failed");
@@ -2088,7 +2244,7 @@ int fx_ir_solve(fx_ir ir, fx_vec b, fx_vec x, fx_result* result, uint32_t* inner
       hipLaunchKernelGGL(k_ir_add_scaled, dim3(stream_blocks(n)), dim3(kThreads), 0, st,
                          (double*)x->d, (const double*)ir->sc, (const float*)ir->W->x,
                          (const float*)ir->W->p, (const float*)ir->W->r, n, cs,
-                         (const IrState*)ir->W->state);
+                         (const IrState*)ir->W->state, ir->W->resident ? 1 : 0);
       FX_HIP(hipGetLastError());
     }
     if (ir->bo)

@@ -149,15 +149,17 @@ struct ResShared {
 
 // The K per-thread values v summed (slot k: maximum when bit k of MaxMask is
 // set) over every thread of every workgroup; every thread gets the same
-// bits, in v.  Call t of a launch uses slot buffer t mod 8 and empties the
+// bits, in v.  post(tot) is run by the first wave (all its lanes hold the
+// same sums) before the others go on: scalars formed there and left in LDS
+// cost one wave's latency and no further barrier.  Call t of a launch uses slot buffer t mod 8 and empties the
 // one that call t + 4 will use: by then every workgroup has left call t - 4,
 // which used it last.  Up to 32 workgroups each reads all slots; more go in
 // groups of 32, the group's first workgroup publishing its sum (one more
 // hop, but 256 workgroups polling 256 lines took longer).  False when a wait
 // gave up.
-template <int K, unsigned MaxMask>
+template <int K, unsigned MaxMask, class Post>
 __device__ __forceinline__ bool res_allreduce(double (&v)[K], const ResComm& cm, uint32_t t,
-                                              ResShared& sh) {
+                                              ResShared& sh, const Post& post) {
   static_assert(K <= kResSlot, "one line per slot");
   const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
   const uint32_t G = gridDim.x, g = blockIdx.x;
@@ -253,6 +255,7 @@ __device__ __forceinline__ bool res_allreduce(double (&v)[K], const ResComm& cm,
         });
       }
     }
+    if (ok) post(tot);
     if (lane == 0) {
       res_for<K>([&](auto k) { sh.tot[k] = tot[k]; });
       sh.bad = ok ? 0 : 1;
@@ -526,6 +529,26 @@ inline int res_mode(const fx_csr_s* A, uint32_t rows) {
   if (rows > 1 && has_row_values<MT>(A) && A->vstride == 8) return RM_VAL;
   if (rows == 2 && A->max_row <= 8) return RM_REG;
   return RM_MEM;
+}
+
+// make(rows, mode) for the instantiations that res_shape and res_mode give.
+template <class F>
+inline const void* res_pick(uint32_t rows, int mode, const F& make) {
+  using std::integral_constant;
+  const void* k = nullptr;
+  auto pick = [&](auto r) {
+    constexpr int R = decltype(r)::value;
+    if constexpr (R <= 2)
+      if (mode == RM_REG) k = make(r, integral_constant<int, RM_REG>{});
+    if constexpr (R >= 2)
+      if (mode == RM_VAL) k = make(r, integral_constant<int, RM_VAL>{});
+    if (mode == RM_MEM) k = make(r, integral_constant<int, RM_MEM>{});
+  };
+  if (rows == 1) pick(integral_constant<int, 1>{});
+  if (rows == 2) pick(integral_constant<int, 2>{});
+  if (rows == 4) pick(integral_constant<int, 4>{});
+  if (rows == 8) pick(integral_constant<int, 8>{});
+  return k;
 }
 
 // One cooperative launch of `kernel` on a comm block that is cleared first;

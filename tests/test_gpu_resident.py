@@ -134,3 +134,34 @@ def test_cg_resident_breakdown_and_zero(ctx, monkeypatch, m):
         old = solve(ctx, monkeypatch, False, fx.CG, A, prm, b=b, x0=x0)
         assert new[0].retcode == old[0].retcode
         assert np.linalg.norm(new[1] - old[1]) <= 1e-12 * max(1.0, np.linalg.norm(old[1]))
+
+
+@pytest.mark.parametrize("dim,m", [(2, 1), (2, 32), (2, 33), (2, 45), (2, 46), (2, 200), (2, 513),
+                                   (3, 65), (3, 82), (3, 103)])
+def test_ir_resident(ctx, monkeypatch, dim, m):
+    """The refinement with its inner loop resident and kernel by kernel: both
+    reach the outer tolerance, so the solutions differ by at most twice the
+    condition number times it."""
+    A = P.poisson2d(m) if dim == 2 else P.poisson3d(m)
+    b = A.matvec(np.random.default_rng(m).uniform(-1, 1, A.nrow))
+    out = []
+    for off in (False, True):
+        if off:
+            monkeypatch.setenv("FASPXX_FX_NORESIDENT", "1")
+        ir = fx.IR(ctx, fx.Csr.from_problem(ctx, A), 1.0,
+                   fx.params(maxIter=50, relTol=1e-12, absTol=0.0),
+                   fx.params(maxIter=20000, relTol=1e-4, absTol=0.0))
+        monkeypatch.delenv("FASPXX_FX_NORESIDENT", raising=False)
+        vb, runs = fx.Vec.from_numpy(ctx, b), []
+        for _ in range(2):  # the second solve queues its outer steps ahead
+            x = fx.Vec(ctx, A.nrow)
+            res, inner = ir.Solve(vb, x)
+            assert res.retcode == 0
+            assert np.linalg.norm(b - A.matvec(x.numpy())) < 1.01e-12 * np.linalg.norm(b)
+            runs.append((x.numpy(), res.numIter, inner))
+        assert np.array_equal(runs[0][0], runs[1][0]) and runs[0][1:] == runs[1][1:]
+        out.append(runs[1])
+    cond = 1.0 / np.tan(np.pi / (2.0 * (m + 1))) ** 2
+    (x1, o1, i1), (x0, o0, i0) = out
+    assert abs(o1 - o0) <= 1 and abs(i1 - i0) <= 0.15 * i0 + 2
+    assert np.linalg.norm(x1 - x0) <= 2e-12 * cond * np.linalg.norm(x0) + 1e-12
