@@ -7,10 +7,8 @@
 //   for k = 0 .. m-1 (kernels skip once the cycle has ended):
 //     S_k     w = V[k+1] = A P V[k] (right) or P A V[k] (left);
 //             partials of (w, V[0])                     (k_spmv + EpiGmW)
-//     M_k,j   j = 0..k: h = (w, V[j]) from the partials (every workgroup
-//             sums them in the same order), H(j,k) = h, w = w - h V[j];
-//             partials of (w, V[j+1]), or of (w, w) after the last
-//                                                                (k_gm_mgs)
+//     modified Gram-Schmidt of w against V[0..k], the column H(.,k), and
+//             partials of (w, w): see "orthogonalisation" below
 //     G_k     t = ||w||, w *= 1/t, H(k+1,k) = t; the Givens update and the
 //             cycle's stopping test on the device (one thread); at the end of
 //             the cycle the triangular solve                     (k_gm_givens)
@@ -25,15 +23,16 @@
 // Z[k] (one Jacobi sweep, z + D^-1 (v - A z), with the reference's shortcut
 // v when ||z||_inf < 1e-20; identity: Z[k] = V[k]), w = A Z[k], and
 // x += sum_j y_j Z[j]; ||Z[k]||_inf rides along as a second reduction slot of
-// the SpMV that writes Z[k].  Modified Gram-Schmidt keeps its sequential order: one kernel
-// per step, as the method needs one reduction per step.  The Hessenberg
+// the SpMV that writes Z[k].  The Hessenberg
 // matrix, the rotations and the right-hand side g stay in f64 on the device;
 // the arithmetic is the reference's (src/GMRES.cxx:182-219).
+#include <algorithm>
 #include <cmath>
 #include <map>
 #include <vector>
 
 #include "fx_fast.hpp"
+#include "fx_resident.hpp"
 
 namespace fx {
 
@@ -124,6 +123,29 @@ __global__ __launch_bounds__(kWideThreads) void k_gm_start(VT* __restrict__ v0, 
   }
 }
 
+// ---- orthogonalisation ------------------------------------------------------
+// Modified Gram-Schmidt takes h_j = (V[j], w - sum_{i<j} h_i V[i]) one after
+// the other, a reduction per j.  Three forms:
+//   up to kGmOneRows rows (one workgroup): all steps and the Givens update in
+//     one kernel, w in registers (k_gm_orth_one);
+//   cycles of up to kGmLowMax: the same h_j by linearity from one pass over the
+//     basis, h_j = (V[j], w) - sum_{i<j} (V[j], V[i]) h_i, i.e. (I + L) h = V^T w
+//     with L the strictly lower part of V^T V, whose row k is formed in the
+//     pass of step k.  (Low-synchronization modified Gram-Schmidt:
+//     Swirydowicz, Langou, Ananthan, Yang, Thomas, Numer. Linear Algebra Appl.
+//     28, 2021; its loss of orthogonality is bounded as MGS's is.)  One pass
+//     for the dot products (k_gm_dots), one workgroup for the triangular solve
+//     (k_gm_lower), one pass for w - V h (k_gm_sub): the basis is read twice
+//     per column instead of w, V[j], V[j+1] read and w written for every j,
+//     and 3 kernels replace k + 1.  The second pass runs from V[k] down, so
+//     that it begins with what the first one read last;
+//   longer cycles: a kernel per j (k_gm_mgs).
+// Measured, this part of an iteration of GMRES(30): 1024^2 unknowns 41 us (18.6
+// + 4.6 + 17.9) against 79 us a kernel per j; 256^2 13.7 us in 3 kernels
+// against 56 us in 13 on average; 40^2 one kernel.
+constexpr uint32_t kGmLowMax = 63;   // one lane per column in the triangular solve
+constexpr uint32_t kGmLowLd = 64;    // row length of L
+
 // One MGS step: h = (w, V[j]) from the partials, w -= h V[j], partials of
 // (w, next) where next = V[j+1], or w itself after the last step.
 template <class VT>
@@ -193,6 +215,239 @@ __global__ __launch_bounds__(kWideThreads) void k_gm_mgs(
   block_partials_n<1, 0u, kWideThreads>(acc, pout);
 }
 
+// Partials of (V[j], w), j <= k, in slots 0 .. k, and of (V[j], V[k]), j < k,
+// in slots k + 1 .. 2 k (part[slot * gridDim.x + workgroup]).  Bound by the
+// read of the basis: one workgroup per CU at most, four vectors at a time, T
+// packs of each per thread.  While T packs per thread cover the vectors
+// (ONCE), w and V[k] stay in registers and the next four vectors' packs are
+// asked for before the sums of these.  Eight sums at a time go through the
+// lanes together, each step halving the values a lane holds, instead of one
+// by one.
+constexpr unsigned kGmDotWgs = 256;  // most workgroups (k_gm_lower sums four partials per lane)
+template <class VT, int T, bool ONCE>
+__global__ __launch_bounds__(kWideThreads) void k_gm_dots(const VT* const* __restrict__ V,
+                                                          const VT* __restrict__ w, uint32_t n,
+                                                          const GmState* st, uint32_t k,
+                                                          double* __restrict__ part) {
+  if (st->status != GM_RUN) return;
+  using PK = Pack16<VT>;
+  constexpr int W = PK::W, B = 4;
+  __shared__ double red[2][2 * B][4 * kWideThreads / 64];
+  const uint32_t nc = n / W, stride = gridDim.x * kWideThreads, tid = threadIdx.x;
+  const uint32_t cfirst = blockIdx.x * kWideThreads + tid;
+  const int lane = tid & 63, wid = tid >> 6;
+  const VT* vk = V[k];
+  const bool tail = blockIdx.x == 0 && tid < n - nc * W;
+  const uint32_t it = nc * W + tid;
+  PK wp[T], kp[T], jp[B][T];
+  auto at = [&](uint32_t c, int t) {  // past the end: pack 0 of the padded vectors, dropped
+    return c + t * stride < nc ? c + t * stride : 0u;
+  };
+  auto load_wk = [&](uint32_t c) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      wp[t] = ld16(w, at(c, t));
+      kp[t] = ld16(vk, at(c, t));
+    }
+  };
+  auto load_v = [&](uint32_t j0, uint32_t c) {
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const VT* vj = V[min(j0 + u, k)];
+#pragma unroll
+      for (int t = 0; t < T; ++t) jp[u][t] = ld16(vj, at(c, t));
+    }
+  };
+  double v[2 * B];  // 2 u: (V[j0 + u], w), 2 u + 1: (V[j0 + u], V[k])
+  auto add = [&](uint32_t c) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if (c + t * stride >= nc) continue;
+#pragma unroll
+      for (int u = 0; u < B; ++u)
+#pragma unroll
+        for (int e = 0; e < W; ++e) {
+          v[2 * u] = fma((double)jp[u][t].v[e], (double)wp[t].v[e], v[2 * u]);
+          v[2 * u + 1] = fma((double)jp[u][t].v[e], (double)kp[t].v[e], v[2 * u + 1]);
+        }
+    }
+  };
+  if constexpr (ONCE) {
+    load_wk(cfirst);
+    load_v(0, cfirst);
+  }
+  for (uint32_t j0 = 0, b = 0; j0 <= k; j0 += B, b ^= 1) {
+#pragma unroll
+    for (int u = 0; u < 2 * B; ++u) v[u] = 0.0;
+    if constexpr (ONCE) {
+      add(cfirst);
+      if (j0 + B <= k) load_v(j0 + B, cfirst);
+    } else {
+      for (uint32_t c = cfirst; c < nc; c += T * stride) {
+        load_wk(c);
+        load_v(j0, c);
+        add(c);
+      }
+    }
+    if (tail) {
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        const VT vj = V[min(j0 + u, k)][it];
+        v[2 * u] = fma((double)vj, (double)w[it], v[2 * u]);
+        v[2 * u + 1] = fma((double)vj, (double)vk[it], v[2 * u + 1]);
+      }
+    }
+    // lane l ends up with value l & 7 summed over its row of 16 lanes
+    double h4[4], h2[2], h1;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const double even = v[2 * i], odd = v[2 * i + 1];
+      h4[i] = (lane & 1 ? odd : even) + dpp_move<0xB1>(lane & 1 ? even : odd);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      const double even = h4[2 * i], odd = h4[2 * i + 1];
+      h2[i] = (lane & 2 ? odd : even) + dpp_move<0x4E>(lane & 2 ? even : odd);
+    }
+    {
+      const double even = h2[0], odd = h2[1];
+      h1 = (lane & 4 ? odd : even) + __shfl_xor(lane & 4 ? even : odd, 4, 64);
+    }
+    h1 += dpp_move<0x128>(h1);  // row_ror 8
+    if ((lane & 8) == 0) red[b][lane & 7][wid * 4 + (lane >> 4)] = h1;
+    __syncthreads();  // (red[b] is written again only after the next barrier)
+    if (tid < 2 * B) {
+      double s = 0.0;
+#pragma unroll
+      for (int i = 0; i < 4 * kWideThreads / 64; ++i) s += red[b][tid][i];
+      const uint32_t j = j0 + tid / 2, slot = (tid & 1) ? k + 1 + j : j;
+      if (j < k || (j == k && !(tid & 1))) part[(size_t)slot * gridDim.x + blockIdx.x] = s;
+    }
+  }
+}
+
+// Its grid: a pack per thread while that gives at most a workgroup per CU.
+inline unsigned gm_dot_wgs(uint32_t n, int cus) {
+  const unsigned most = std::min<unsigned>(kGmDotWgs, (unsigned)cus);
+  const unsigned g = (n / 2 + kWideThreads - 1) / kWideThreads;
+  return g < 1 ? 1 : g > most ? most : g;
+}
+
+// One workgroup: the sums of k_gm_dots's partials (at most 256 each), row k
+// of L, the column h of (I + L) h = V^T w into H and hv; FGMRES: max |Z[k]|
+// from the SpMV's partials (slot 1 of pz).
+__global__ __launch_bounds__(1024) void k_gm_lower(const GmState* st,
+                                                   const double* __restrict__ part, unsigned g,
+                                                   uint32_t k, double* __restrict__ Lm, GmLsq L,
+                                                   double* __restrict__ hv,
+                                                   const double* __restrict__ pz, unsigned gz,
+                                                   double* zinf_out) {
+  if (st->status != GM_RUN) return;
+  __shared__ double sum[2 * kGmLowMax + 1];
+  __shared__ double low[kGmLowMax][kGmLowLd];
+  const uint32_t tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  for (uint32_t e = tid; e < k * kGmLowLd; e += 1024) low[e / kGmLowLd][e % kGmLowLd] = Lm[e];
+  if (zinf_out) {
+    double z[1];
+    partials_thread<1, 1u, 1024>(pz + gz, gz, tid, z);
+    partials_combine<1, 1u, 1024>(z);
+    if (tid == 0) *zinf_out = z[0];
+  }
+  for (uint32_t s = wid; s <= 2 * k; s += 16) {
+    double x[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const uint32_t b = lane + 64 * i;
+      const double y = part[(size_t)s * g + min(b, g - 1)];
+      x[i] = b < g ? y : 0.0;
+    }
+    const double t = res_wave<false>((x[0] + x[1]) + (x[2] + x[3]));
+    if (lane == 0) sum[s] = t;
+  }
+  __syncthreads();
+  if (wid == 0) {
+    double r = lane <= k ? sum[lane] : 0.0;
+    const uint32_t row = min(lane, k);
+    for (uint32_t i = 0; i < k; ++i) {
+      const double hi = res_lane(r, (int)i);
+      const double lji = row < k ? low[row][i] : sum[k + 1 + i];
+      if (lane > i && lane <= k) r = fma(-lji, hi, r);
+    }
+    if (lane <= k) {
+      hv[lane] = r;
+      L.H[(size_t)lane * L.ld + k] = r;
+    }
+    if (lane < k) Lm[(size_t)k * kGmLowLd + lane] = sum[k + 1 + lane];
+  }
+}
+
+// w = w - sum_j h_j V[j], from V[k] down; partials of (w, w).
+template <class VT>
+__global__ __launch_bounds__(kWideThreads) void k_gm_sub(VT* __restrict__ w,
+                                                         const VT* const* __restrict__ V,
+                                                         uint32_t n, const GmState* st, uint32_t k,
+                                                         const double* __restrict__ hv,
+                                                         double* __restrict__ pout) {
+  if (st->status != GM_RUN) return;
+  using PK = Pack16<VT>;
+  constexpr int W = PK::W, T = 2, B = 4;
+  const uint32_t nc = n / W, stride = gridDim.x * kWideThreads;
+  const uint32_t cfirst = blockIdx.x * kWideThreads + threadIdx.x;
+  double acc[1] = {0.0};
+  for (uint32_t c = cfirst; c < nc; c += T * stride) {
+    uint32_t ct[T];
+    PK wp[T];
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      ct[t] = c + t * stride < nc ? c + t * stride : c;
+      wp[t] = ld16(w, ct[t]);
+    }
+    int j = (int)k;
+    for (; j >= B - 1; j -= B) {
+      PK jp[B][T];
+      VT h[B];
+#pragma unroll
+      for (int u = 0; u < B; ++u) {
+        h[u] = (VT)(-hv[j - u]);
+        const VT* vj = V[j - u];
+#pragma unroll
+        for (int t = 0; t < T; ++t) jp[u][t] = ld16(vj, ct[t]);
+      }
+#pragma unroll
+      for (int u = 0; u < B; ++u)
+#pragma unroll
+        for (int t = 0; t < T; ++t)
+#pragma unroll
+          for (int e = 0; e < W; ++e) wp[t].v[e] = fma(h[u], jp[u][t].v[e], wp[t].v[e]);
+    }
+    for (; j >= 0; --j) {
+      const VT h = (VT)(-hv[j]);
+      const VT* vj = V[j];
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        const PK jp = ld16(vj, ct[t]);
+#pragma unroll
+        for (int e = 0; e < W; ++e) wp[t].v[e] = fma(h, jp.v[e], wp[t].v[e]);
+      }
+    }
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      if (c + t * stride >= nc) continue;
+      st16(w, ct[t], wp[t]);
+#pragma unroll
+      for (int e = 0; e < W; ++e) acc[0] = fma((double)wp[t].v[e], (double)wp[t].v[e], acc[0]);
+    }
+  }
+  if (blockIdx.x == 0 && threadIdx.x < n - nc * W) {
+    const uint32_t i = nc * W + threadIdx.x;
+    VT wi = w[i];
+    for (int j = (int)k; j >= 0; --j) wi = fma((VT)(-hv[j]), V[j][i], wi);
+    w[i] = wi;
+    acc[0] = fma((double)wi, (double)wi, acc[0]);
+  }
+  block_partials_n<1, 0u, kWideThreads>(acc, pout);
+}
+
 // Givens update of column cnt - 1 (src/GMRES.cxx:182-203)
 __device__ __forceinline__ void givens_column(const GmLsq& L, uint32_t cnt) {
   const uint32_t c1 = cnt - 1;
@@ -253,18 +508,12 @@ __device__ __forceinline__ void givens_column_lds(double* __restrict__ col,
   gc1 = hc[c1] * gc1;
 }
 
-// G_k: t = ||w||, w *= 1/t, H(k+1,k) = t, Givens, stopping test (workgroup
-// 0; it stages column k, the rotations and g[k] in LDS while every
+// G_k: t = ||w||, w *= 1/t (scale), H(k+1,k) = t, Givens, stopping test
+// (workgroup 0; it stages column k, the rotations and g[k] in LDS while every
 // workgroup scales w), and at the end of the cycle the triangular solve.
-template <class VT>
-__global__ __launch_bounds__(kWideThreads) void k_gm_givens(
-    VT* __restrict__ w, uint32_t n, GmState* st, const double* __restrict__ pin, unsigned gin,
-    GmLsq L, GmPrm P, uint32_t k, double* hist) {
-  if (st->status != GM_RUN) return;
-  double t2[1];
-  partials_thread<1, 0u, kWideThreads>(pin, gin, threadIdx.x, t2);
-  partials_combine<1, 0u, kWideThreads>(t2);
-  const double t = sqrt(t2[0]);  // VEC::Norm2
+template <class Scale>
+__device__ __forceinline__ void givens_step(double t, GmState* st, const GmLsq& L, const GmPrm& P,
+                                            uint32_t k, double* hist, const Scale& scale) {
   const double a = 1.0 / t;      // src/GMRES.cxx:177-178 (t > SMALL_DBL always holds)
   const uint32_t cnt = k + 1;
   const bool staged = cnt < kGivLds;
@@ -280,9 +529,7 @@ __global__ __launch_bounds__(kWideThreads) void k_gm_givens(
     }
     if (threadIdx.x == 0) sg[0] = L.g[k];
   }
-  const uint32_t stride = gridDim.x * kWideThreads;
-  for (uint32_t i = blockIdx.x * kWideThreads + threadIdx.x; i < n; i += stride)
-    w[i] = w[i] * (VT)a;
+  scale(a);
   if (blockIdx.x != 0) return;
   __syncthreads();
   if (threadIdx.x == 0) {
@@ -347,6 +594,121 @@ __global__ __launch_bounds__(kWideThreads) void k_gm_givens(
   }
 }
 
+template <class VT>
+__global__ __launch_bounds__(kWideThreads) void k_gm_givens(
+    VT* __restrict__ w, uint32_t n, GmState* st, const double* __restrict__ pin, unsigned gin,
+    GmLsq L, GmPrm P, uint32_t k, double* hist) {
+  if (st->status != GM_RUN) return;
+  double t2[1];
+  partials_thread<1, 0u, kWideThreads>(pin, gin, threadIdx.x, t2);
+  partials_combine<1, 0u, kWideThreads>(t2);
+  givens_step(sqrt(t2[0]), st, L, P, k, hist, [&](double a) {  // VEC::Norm2
+    const uint32_t stride = gridDim.x * kWideThreads;
+    for (uint32_t i = blockIdx.x * kWideThreads + threadIdx.x; i < n; i += stride)
+      w[i] = w[i] * (VT)a;
+  });
+}
+
+// All of column k in one workgroup (n <= kGmOneRows): the steps of k_gm_mgs
+// with w in registers and V[j + 1] kept for the next step, then G_k; the same
+// sums in the same order as kernel by kernel.  A step costs a reduction of one
+// workgroup in place of a kernel (4 us with its gap).
+constexpr uint32_t kGmOneRows = 2 * kGmPer * kWideThreads;
+template <class VT>
+__global__ __launch_bounds__(kWideThreads) void k_gm_orth_one(
+    VT* __restrict__ w, const VT* const* __restrict__ V, uint32_t n, GmState* st,
+    const double* __restrict__ pin, unsigned gin, GmLsq L, GmPrm P, uint32_t k, double* hist,
+    double* zinf_out) {
+  if (st->status != GM_RUN) return;
+  using PK = Pack16<VT>;
+  constexpr int W = PK::W;
+  static_assert(W * 2 * kWideThreads >= kGmOneRows, "two packs per thread hold w");
+  const uint32_t nc = n / W, tid = threadIdx.x;
+  const bool one = tid < nc, two = tid + kWideThreads < nc, odd = tid < n - nc * W;
+  const uint32_t c0 = one ? tid : 0u, c1 = two ? tid + kWideThreads : c0, it = nc * W + tid;
+  PK wa = ld16(w, c0), wb = ld16(w, c1), va = ld16(V[0], c0), vb = ld16(V[0], c1);
+  VT wt = odd ? w[it] : (VT)0, vt = odd ? V[0][it] : (VT)0;
+  double h[1];
+  if (zinf_out) {  // FGMRES: the partials also hold max |Z[k]| (slot 1)
+    double hz[2];
+    partials_thread<2, 2u, kWideThreads>(pin, gin, tid, hz);
+    partials_combine<2, 2u, kWideThreads>(hz);
+    h[0] = hz[0];
+    if (tid == 0) *zinf_out = hz[1];
+  } else {
+    partials_thread<1, 0u, kWideThreads>(pin, gin, tid, h);
+    partials_combine<1, 0u, kWideThreads>(h);
+  }
+  for (uint32_t j = 0; j <= k; ++j) {
+    const bool self = j == k;
+    PK na{}, nb{};
+    VT nt = (VT)0;
+    if (!self) {
+      na = ld16(V[j + 1], c0);
+      nb = ld16(V[j + 1], c1);
+      if (odd) nt = V[j + 1][it];
+    }
+    if (tid == 0) L.H[(size_t)j * L.ld + k] = h[0];
+    const VT b = (VT)(-h[0]);
+    const bool bone = -h[0] == 1.0;
+    double a0 = 0.0, a1 = 0.0, acc[1] = {0.0};
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      wa.v[e] = bone ? wa.v[e] + va.v[e] : fma(b, va.v[e], wa.v[e]);
+      wb.v[e] = bone ? wb.v[e] + vb.v[e] : fma(b, vb.v[e], wb.v[e]);
+      a0 = fma((double)wa.v[e], (double)(self ? wa.v[e] : na.v[e]), a0);
+      a1 = fma((double)wb.v[e], (double)(self ? wb.v[e] : nb.v[e]), a1);
+    }
+    acc[0] += (one ? a0 : 0.0) + (two ? a1 : 0.0);
+    if (odd) {
+      wt = bone ? wt + vt : fma(b, vt, wt);
+      acc[0] = fma((double)wt, (double)(self ? wt : nt), acc[0]);
+    }
+    partials_combine<1, 0u, kWideThreads>(acc);
+    h[0] = acc[0];
+    va = na;
+    vb = nb;
+    vt = nt;
+  }
+  __syncthreads();  // column k of H, for the Givens step's staging
+  givens_step(sqrt(h[0]), st, L, P, k, hist, [&](double a) {
+#pragma unroll
+    for (int e = 0; e < W; ++e) {
+      wa.v[e] = wa.v[e] * (VT)a;
+      wb.v[e] = wb.v[e] * (VT)a;
+    }
+    if (one) st16(w, c0, wa);
+    if (two) st16(w, c1, wb);
+    if (odd) w[it] = wt * (VT)a;
+  });
+}
+
+// sum_j y_j V[j]_i from j = cnt - 1 down (copy, Scale(y), then AXPBY(1, y_j,
+// V[j], wk)); eight vectors' entries are asked for before the first is used
+// (one by one the 30 loads of a row came one latency after the other: 27 us at
+// 65536 unknowns, whatever the bandwidth).
+template <class VT>
+__device__ __forceinline__ VT combine_basis(const VT* const* __restrict__ V,
+                                            const double* __restrict__ y, uint32_t cnt,
+                                            uint32_t i) {
+  VT wk = V[cnt - 1][i] * (VT)y[cnt - 1];
+  constexpr int B = 8;
+  for (int j = (int)cnt - 2; j >= 0; j -= B) {
+    VT x[B];
+    double g[B];
+#pragma unroll
+    for (int u = 0; u < B; ++u) {
+      const int ju = j - u >= 0 ? j - u : 0;
+      x[u] = V[ju][i];
+      g[u] = y[ju];
+    }
+#pragma unroll
+    for (int u = 0; u < B; ++u)
+      if (j - u >= 0) wk = g[u] == 1.0 ? wk + x[u] : fma((VT)g[u], x[u], wk);
+  }
+  return wk;
+}
+
 // X: wk = sum_j y_j V[j] in the reference's order, then x += P wk (right) or
 // x += wk (left).
 template <class VT, bool RIGHTJAC>
@@ -359,11 +721,7 @@ __global__ __launch_bounds__(kWideThreads) void k_gm_update(VT* __restrict__ x,
   if (cnt == 0) return;
   const uint32_t stride = gridDim.x * kWideThreads;
   for (uint32_t i = blockIdx.x * kWideThreads + threadIdx.x; i < n; i += stride) {
-    VT wk = V[cnt - 1][i] * (VT)L.g[cnt - 1];  // copy, then Scale(g[count-1])
-    for (int j = (int)cnt - 2; j >= 0; --j) {  // AXPBY(1, g[j], V[j], wk)
-      const double gj = L.g[j];
-      wk = gj == 1.0 ? wk + V[j][i] : fma((VT)gj, V[j][i], wk);
-    }
+    const VT wk = combine_basis(V, L.g, cnt, i);
     const VT d = RIGHTJAC ? wk * dinv[i] : wk;  // P wk from zero
     x[i] = fma((VT)1, d, x[i]);                 // x.AXPY(1, .)
   }
@@ -460,11 +818,7 @@ __global__ __launch_bounds__(kWideThreads) void k_fgm_update(VT* __restrict__ x,
   if (cnt == 0) return;
   const uint32_t stride = gridDim.x * kWideThreads;
   for (uint32_t i = blockIdx.x * kWideThreads + threadIdx.x; i < n; i += stride) {
-    VT wk = Z[cnt - 1][i] * (VT)L.g[cnt - 1];
-    for (int j = (int)cnt - 2; j >= 0; --j) {
-      const double gj = L.g[j];
-      wk = gj == 1.0 ? wk + Z[j][i] : fma((VT)gj, Z[j][i], wk);
-    }
+    const VT wk = combine_basis(Z, L.g, cnt, i);
     x[i] = fma((VT)1, wk, x[i]);
   }
 }
@@ -504,6 +858,9 @@ struct GmWs {
   double* zpart = nullptr;   // FGMRES: (maxR + 1) x kMaxRedBlocks partial maxima
   void* tmp = nullptr;
   double* lsq = nullptr;     // H, hc, hs, g
+  // low-synchronization orthogonalisation: the dot products' partials, L and h
+  double* dots = nullptr;
+  double* low = nullptr;
   std::map<uint32_t, hipGraphExec_t> cycles;
   ~GmWs() {
     for (auto& c : cycles) (void)hipGraphExecDestroy(c.second);
@@ -514,6 +871,8 @@ struct GmWs {
     (void)hipFree(zpart);
     (void)hipFree(tmp);
     (void)hipFree(lsq);
+    (void)hipFree(dots);
+    (void)hipFree(low);
   }
 };
 
@@ -612,18 +971,44 @@ struct GmRun {
         FX_TRY((fused_spmv<VT, ROW_AX, 1, 0u>(A, op, W, st, XLoad<VT>{vec(k)}, BNone{},
                                               EpiGmW<VT, false>{w, vec(0), dinv, cst}, pa)));
       }
+      double* zinf = flex ? G.zinf + k : nullptr;  // S_k's partials carry max |Z[k]|
+      const VT* const* Vd = (const VT* const*)G.Vdev;
+      if (n <= kGmOneRows) {
+        hipLaunchKernelGGL((k_gm_orth_one<VT>), dim3(1), dim3(kWideThreads), 0, st, w, Vd, n,
+                           dstate(), (const double*)pa, gs, L, P, k, W.hist, zinf);
+        FX_HIP(hipGetLastError());
+        continue;
+      }
       const double* pin = pa;
       unsigned gin = gs;
-      for (uint32_t j = 0; j <= k; ++j) {
-        double* pout = (pin == pa) ? pb : pa;
-        const VT* next = (j < k) ? vec(j + 1) : nullptr;
-        const bool zslot = flex && j == 0;  // S_k's partials carry max |Z[k]|
-        hipLaunchKernelGGL((k_gm_mgs<VT>), dim3(g), dim3(kWideThreads), 0, st, w,
-                           (const VT*)vec(j), next, n, cst, pin, gin, pout, L, j, k,
-                           zslot ? G.zinf + k : nullptr);
+      if (m <= kGmLowMax) {
+        double* hv = G.low + (size_t)kGmLowMax * kGmLowLd;
+        static_assert(Pack16<VT>::W == 2, "the dot products' grid counts f64 packs");
+        const unsigned gd = gm_dot_wgs(n, cus);
+        const uint64_t held = (uint64_t)gd * kWideThreads * Pack16<VT>::W;  // by a pack per thread
+        auto dots = n <= held + 1       ? k_gm_dots<VT, 1, true>
+                    : n <= 4 * held + 1 ? k_gm_dots<VT, 4, true>
+                                        : k_gm_dots<VT, 4, false>;
+        hipLaunchKernelGGL(dots, dim3(gd), dim3(kWideThreads), 0, st, Vd, (const VT*)w, n, cst, k,
+                           G.dots);
+        hipLaunchKernelGGL(k_gm_lower, dim3(1), dim3(1024), 0, st, cst, (const double*)G.dots, gd,
+                           k, G.low, L, hv, (const double*)pa, gs, zinf);
+        hipLaunchKernelGGL((k_gm_sub<VT>), dim3(g), dim3(kWideThreads), 0, st, w, Vd, n, cst, k,
+                           (const double*)hv, pb);
         FX_HIP(hipGetLastError());
-        pin = pout;
+        pin = pb;
         gin = g;
+      } else {
+        for (uint32_t j = 0; j <= k; ++j) {
+          double* pout = (pin == pa) ? pb : pa;
+          const VT* next = (j < k) ? vec(j + 1) : nullptr;
+          hipLaunchKernelGGL((k_gm_mgs<VT>), dim3(g), dim3(kWideThreads), 0, st, w,
+                             (const VT*)vec(j), next, n, cst, pin, gin, pout, L, j, k,
+                             j == 0 ? zinf : nullptr);
+          FX_HIP(hipGetLastError());
+          pin = pout;
+          gin = g;
+        }
       }
       hipLaunchKernelGGL((k_gm_givens<VT>), dim3(g), dim3(kWideThreads), 0, st, w, n, dstate(),
                          pin, gin, L, P, k, W.hist);
@@ -765,6 +1150,10 @@ int gmres_fast(fx_solver S, FastWs& W, const double* b, double* x, fx_result* re
     const size_t nl = (size_t)(maxR + 1) * maxR + (maxR + 1) + maxR + (maxR + 2);
     FX_HIP(hipMalloc(&N.lsq, sizeof(double) * nl));
     FX_HIP(hipMemset(N.lsq, 0, sizeof(double) * nl));
+    if (W.n > kGmOneRows) {
+      FX_HIP(hipMalloc(&N.dots, sizeof(double) * (2 * kGmLowMax + 1) * kGmDotWgs));
+      FX_HIP(hipMalloc(&N.low, sizeof(double) * (kGmLowMax + 1) * kGmLowLd));
+    }
   }
   GmWs& GG = *(GmWs*)W.gm;
   const bool flex = S->type == FX_SOLVER_FGMRES;

@@ -52,7 +52,7 @@ inline ResComm res_comm(void* mem) {
 }
 
 // Empty slots and zero flags, before each launch.
-__global__ __launch_bounds__(kThreads) void k_res_clear(unsigned long long* w) {
+static __global__ __launch_bounds__(kThreads) void k_res_clear(unsigned long long* w) {
   for (size_t i = blockIdx.x * kThreads + threadIdx.x; i < kResCommWords;
        i += (size_t)gridDim.x * kThreads)
     w[i] = i < kResSlotWords + kResGsumWords ? kResEmpty : 0ull;
