@@ -1354,6 +1354,8 @@ int ws_alloc(FastWs& W, fx_ctx ctx, int dt, uint32_t n, uint32_t hist_cap, size_
   FX_HIP(hipHostMalloc(&W.hstate, 2 * state_bytes, hipHostMallocDefault));
   W.hist_cap = hist_cap + 2;
   FX_HIP(hipMalloc(&W.hist, sizeof(double) * W.hist_cap));
+  // nothing is recorded before minIter: those entries read as zero
+  FX_HIP(hipMemsetAsync(W.hist, 0, sizeof(double) * W.hist_cap, ctx->stream));
   FX_HIP(hipMalloc(&W.dscal, sizeof(double) * 8));
   FX_HIP(hipEventCreateWithFlags(&W.ev[0], hipEventDisableTiming));
   FX_HIP(hipEventCreateWithFlags(&W.ev[1], hipEventDisableTiming));
