@@ -103,36 +103,153 @@ __global__ __launch_bounds__(kThreads) void k_convert(const S* __restrict__ s, D
 // (from LARGE_DBL = 1e60, VEC::Min, :403-421; computed as -max(-x)).  Optional
 // fused update before the reduction (kinds 0/1): upd 1 y += a x (AXPY),
 // upd 2 y = a y + x (XPAY).
-// Products are formed in double; sums accumulate in double with fma.  Each
-// workgroup writes one partial; k_finish combines them.
-template <class T>
-__global__ __launch_bounds__(kThreads) void k_reduce(int kind, int upd, double a,
-                                                     const T* __restrict__ x, T* __restrict__ y,
-                                                     const T* __restrict__ z, uint32_t n,
-                                                     double* partials) {
-  double acc[1] = {kind >= 3 ? -1e60 : 0.0};
-  const uint32_t stride = gridDim.x * kThreads;
-  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) {
-    if (kind == 2) {
-      acc[0] = fmax(acc[0], fabs((double)x[i]));
-    } else if (kind == 3) {
-      acc[0] = fmax(acc[0], (double)x[i]);
-    } else if (kind == 4) {
-      acc[0] = fmax(acc[0], -(double)x[i]);
-    } else if (upd) {
-      const T yn = upd == 1 ? fma((T)a, x[i], y[i]) : fma((T)a, y[i], x[i]);
-      y[i] = yn;
-      const double u = (double)yn;
-      acc[0] = fma(u, kind == 0 ? (double)z[i] : u, acc[0]);
-    } else {
-      const double u = (double)x[i];
-      acc[0] = fma(u, kind == 0 ? (double)y[i] : u, acc[0]);
+// Products are formed in double; sums accumulate in double with fma.
+//
+// One launch: each workgroup publishes its partial and counts itself done;
+// the one that counts last combines the partials (in k_finish's order: 1024
+// threads' worth of sums, each wave's butterfly, the waves in order) and
+// stores the result, to the device, to the host, or both.  Partials and count
+// pass through relaxed agent-scope atomics, each store waited for before the
+// count, so no cache is written back.  A finisher kernel, a copy to the host
+// and a wait for the stream were three more round trips: 13 us of 20 for a
+// dot product of 10^6 f64.
+struct RedOut {
+  double* dev;   // device result, or null
+  double* host;  // pinned host result, or null
+  int post;      // 1: square root, 2: negated
+  unsigned* count;
+};
+constexpr unsigned long long kRedPending = 0x7ff4f00d5eed0001ull;  // hpin before the result
+
+// Workgroups are counted in groups, whose last ones are counted in turn: one
+// address takes an increment every 12 ns or so, 12 us for 1000 workgroups.
+constexpr unsigned kRedGroup = 32;
+constexpr unsigned kRedStride = 32;  // words between two counts: a line each
+constexpr unsigned kRedCounts = 1 + (kMaxRedBlocks + kRedGroup - 1) / kRedGroup;
+
+// One more of `members`; true for the last, which leaves the count at zero.
+__device__ __forceinline__ bool red_count(unsigned* c, unsigned members) {
+  if (__hip_atomic_fetch_add(c, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != members - 1)
+    return false;
+  __hip_atomic_store(c, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  return true;
+}
+
+template <bool MAX>
+__device__ __forceinline__ double red_combine(const double* partials, unsigned G) {
+  static_assert(kMaxRedBlocks <= 2 * kFinThreads, "two partials per summing thread at most");
+  __shared__ double red[kFinThreads / 64];
+  const double ident = MAX ? -INFINITY : 0.0;
+  const int tid = threadIdx.x, lane = tid & 63, wid = tid >> 6;
+  constexpr int V = kFinThreads / kThreads;
+  double p[V][2];
+#pragma unroll
+  for (int v = 0; v < V; ++v)
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+      const unsigned i = tid + v * kThreads + h * kFinThreads;
+      const unsigned long long x = __hip_atomic_load(
+          reinterpret_cast<const unsigned long long*>(partials) + (i < G ? i : 0u),
+          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      p[v][h] = i < G ? __longlong_as_double((long long)x) : ident;
     }
+#pragma unroll
+  for (int v = 0; v < V; ++v) {
+    double a = ident;
+    a = MAX ? fmax(a, p[v][0]) : a + p[v][0];
+    if (G > (unsigned)kFinThreads) a = MAX ? fmax(a, p[v][1]) : a + p[v][1];
+    a = MAX ? wave_max(a) : wave_sum(a);
+    if (lane == 0) red[v * kWaves + wid] = a;
+  }
+  __syncthreads();
+  double a = red[0];
+#pragma unroll
+  for (int w = 1; w < kFinThreads / 64; ++w) a = MAX ? fmax(a, red[w]) : a + red[w];
+  return a;
+}
+
+template <bool MAX>
+__device__ __forceinline__ void red_finish(double (&acc)[1], double* partials, const RedOut& o) {
+  block_reduce<1, MAX ? 1u : 0u>(acc);
+  const unsigned G = gridDim.x;
+  double s = acc[0];
+  if (G > 1) {
+    __shared__ bool last;
+    if (threadIdx.x == 0) {
+      const unsigned g = blockIdx.x / kRedGroup, ng = (G + kRedGroup - 1) / kRedGroup;
+      const unsigned members = g + 1 < ng ? kRedGroup : G - g * kRedGroup;
+      __hip_atomic_store(reinterpret_cast<unsigned long long*>(partials) + blockIdx.x,
+                         (unsigned long long)__double_as_longlong(s), __ATOMIC_RELAXED,
+                         __HIP_MEMORY_SCOPE_AGENT);
+      asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the partial is there before the count
+      last = red_count(o.count + kRedStride * (g + 1), members) && red_count(o.count, ng);
+    }
+    __syncthreads();
+    if (!last) return;
+    s = red_combine<MAX>(partials, G);
+  }
+  if (threadIdx.x != 0) return;
+  s = o.post == 1 ? sqrt(s) : o.post == 2 ? -s : s;
+  if (o.dev) *o.dev = s;
+  if (o.host)
+    __hip_atomic_store(reinterpret_cast<unsigned long long*>(o.host),
+                       (unsigned long long)__double_as_longlong(s), __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
+// Four strided elements at a time: their loads are all in flight before the
+// first is used (a thread has up to four below 2^21 elements).
+template <class Load, class Use>
+__device__ __forceinline__ void red_loop(uint32_t i, uint32_t n, uint32_t stride, Load load,
+                                         Use use) {
+  for (; i < n; i = stride * 4u < n - i ? i + stride * 4u : n) {
+    decltype(load(i)) v[4];
+    const uint32_t left = (n - 1 - i) / stride;  // elements of this thread after i
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k) v[k] = load(i + stride * (k < left ? k : left));
+#pragma unroll
+    for (uint32_t k = 0; k < 4; ++k)
+      if (k <= left) use(i + stride * k, v[k]);
+  }
+}
+template <class T>
+struct Two {
+  T a, b;
+};
+
+template <class T>
+__global__ __launch_bounds__(kThreads) void k_reduce(int kind, int upd, double a, const T* x, T* y,
+                                                     const T* z, uint32_t n, double* partials,
+                                                     RedOut o) {
+  double acc[1] = {kind >= 3 ? -1e60 : 0.0};
+  const uint32_t stride = gridDim.x * kThreads, i = blockIdx.x * kThreads + threadIdx.x;
+  if (kind == 0 && !upd) {
+    red_loop(i, n, stride, [&](uint32_t j) { return Two<T>{x[j], y[j]}; },
+             [&](uint32_t, const Two<T>& v) { acc[0] = fma((double)v.a, (double)v.b, acc[0]); });
+  } else if (kind == 1 && !upd) {
+    red_loop(i, n, stride, [&](uint32_t j) { return x[j]; },
+             [&](uint32_t, T v) { acc[0] = fma((double)v, (double)v, acc[0]); });
+  } else if (kind >= 2) {
+    red_loop(i, n, stride, [&](uint32_t j) { return x[j]; }, [&](uint32_t, T v) {
+      acc[0] = fmax(acc[0], kind == 2 ? fabs((double)v) : kind == 3 ? (double)v : -(double)v);
+    });
+  } else {
+    // The updates (y may be z).  y is in memory, for any stream to read,
+    // before its workgroup counts itself done: stored at agent scope, past
+    // the L2, and waited for.
+    red_loop(i, n, stride, [&](uint32_t j) { return Two<T>{x[j], y[j]}; },
+             [&](uint32_t j, const Two<T>& v) {
+               const T yn = upd == 1 ? fma((T)a, v.a, v.b) : fma((T)a, v.b, v.a);
+               __hip_atomic_store(y + j, yn, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+               const double u = (double)yn;
+               acc[0] = fma(u, kind != 0 ? u : z == y ? u : (double)z[j], acc[0]);
+             });
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
   }
   if (kind >= 2)
-    block_partials<1, 1u>(acc, partials);
+    red_finish<true>(acc, partials, o);
   else
-    block_partials<1, 0u>(acc, partials);
+    red_finish<false>(acc, partials, o);
 }
 
 template <class T>
@@ -156,33 +273,55 @@ int elem_dispatch(fx_ctx ctx, int op, int form, double a, double b, fx_vec x, fx
   return launch_elem<float>(ctx, op, form, a, b, xp, y->d, y->n);
 }
 
+template <class T>
+int launch_reduce(fx_ctx ctx, int kind, int upd, double a, const void* x, void* y, const void* z,
+                  uint32_t n, double* dev_out, double* host_out) {
+  const RedOut o{dev_out, host_out, kind == 4 ? 2 : kind == 1 ? 1 : 0, ctx->rcount};
+  hipLaunchKernelGGL(k_reduce<T>, dim3(stream_blocks(n)), dim3(kThreads), 0, ctx->stream, kind,
+                     upd, a, (const T*)x, (T*)y, (const T*)z, n, ctx->ws.partials, o);
+  FX_HIP(hipGetLastError());
+  return 0;
+}
+
 int reduce_dispatch(fx_ctx ctx, int kind, int upd, double a, fx_vec x, fx_vec y, fx_vec z,
-                    double* dev_out) {
+                    double* dev_out, double* host_out = nullptr) {
   FX_CHECK(x, FX_ERROR_INPUT_PAR, "null vector");
   if (y) FX_CHECK(y->n == x->n && y->dtype == x->dtype, FX_ERROR_NONMATCH_SIZE, "vector mismatch");
   if (z) FX_CHECK(z->n == x->n && z->dtype == x->dtype, FX_ERROR_NONMATCH_SIZE, "vector mismatch");
-  const unsigned g = stream_blocks(x->n);
+  void* yd = y ? y->d : nullptr;
+  const void* zd = z ? z->d : nullptr;
   if (x->dtype == FX_F64)
-    hipLaunchKernelGGL(k_reduce<double>, dim3(g), dim3(kThreads), 0, ctx->stream, kind, upd, a,
-                       (const double*)x->d, (double*)(y ? y->d : nullptr),
-                       (const double*)(z ? z->d : nullptr), x->n, ctx->ws.partials);
-  else
-    hipLaunchKernelGGL(k_reduce<float>, dim3(g), dim3(kThreads), 0, ctx->stream, kind, upd, a,
-                       (const float*)x->d, (float*)(y ? y->d : nullptr),
-                       (const float*)(z ? z->d : nullptr), x->n, ctx->ws.partials);
-  FX_HIP(hipGetLastError());
-  if (kind >= 2)
-    return launch_finish<1, 1u>(ctx->stream, ctx->ws.partials, g,
-                                FinStore<1>{dev_out, kind == 4 ? 2 : 0});
-  return launch_finish<1, 0u>(ctx->stream, ctx->ws.partials, g, FinStore<1>{dev_out, kind == 1});
+    return launch_reduce<double>(ctx, kind, upd, a, x->d, yd, zd, x->n, dev_out, host_out);
+  return launch_reduce<float>(ctx, kind, upd, a, x->d, yd, zd, x->n, dev_out, host_out);
 }
 
-int fetch_scalar(fx_ctx ctx, int slot, double* out) {
-  FX_HIP(hipMemcpyAsync(ctx->hpin + slot, ctx->dscal + slot, sizeof(double),
-                        hipMemcpyDeviceToHost, ctx->stream));
-  FX_HIP(hipStreamSynchronize(ctx->stream));
-  *out = ctx->hpin[slot];
+// A reduction whose result the host waits for.  The last workgroup stores it
+// to pinned memory, where the host looks for it: the stream's own completion
+// is seen some 8 to 16 us later.  By then all the work queued before it is
+// done, x and y are read and an updated y is stored.  Whatever does not show
+// up soon (a long kernel queue, an error) is waited for on the stream.
+int reduce_host(fx_ctx ctx, int kind, int upd, double a, fx_vec x, fx_vec y, fx_vec z,
+                double* out) {
+  unsigned long long* slot = reinterpret_cast<unsigned long long*>(ctx->hpin);
+  __atomic_store_n(slot, kRedPending, __ATOMIC_RELEASE);
+  FX_TRY(reduce_dispatch(ctx, kind, upd, a, x, y, z, nullptr, ctx->hpin));
+  unsigned long long bits = kRedPending;
+  for (int spin = 0; spin < 200000; ++spin) {
+    bits = __atomic_load_n(slot, __ATOMIC_ACQUIRE);
+    if (bits != kRedPending) break;
+  }
+  if (bits == kRedPending) {
+    FX_HIP(hipStreamSynchronize(ctx->stream));
+    bits = __atomic_load_n(slot, __ATOMIC_ACQUIRE);
+  }
+  std::memcpy(out, &bits, sizeof(double));
   return 0;
+}
+
+int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, double* dev_out) {
+  if (dtype == FX_F64)
+    return launch_reduce<double>(ctx, 2, 0, 0.0, x, nullptr, nullptr, n, dev_out, nullptr);
+  return launch_reduce<float>(ctx, 2, 0, 0.0, x, nullptr, nullptr, n, dev_out, nullptr);
 }
 
 int convert_copy(fx_ctx ctx, const void* s, int sdt, void* d, int ddt, uint32_t n) {
@@ -227,6 +366,8 @@ void fx_params_default(fx_params* p) {
 static int ctx_init(fx_ctx c) {
   FX_HIP(hipMalloc(&c->ws.partials, sizeof(double) * 16 * 65536));
   FX_HIP(hipMalloc(&c->dscal, sizeof(double) * 64));
+  FX_HIP(hipMalloc(&c->rcount, sizeof(unsigned) * kRedStride * kRedCounts));
+  FX_HIP(hipMemset(c->rcount, 0, sizeof(unsigned) * kRedStride * kRedCounts));
   FX_HIP(hipHostMalloc(&c->hpin, sizeof(double) * 64, hipHostMallocDefault));
   hipDeviceProp_t prop;
   FX_HIP(hipGetDeviceProperties(&prop, c->device));
@@ -278,6 +419,7 @@ int fx_ctx_destroy(fx_ctx c) {
   if (c->stream) (void)hipStreamSynchronize(c->stream);
   (void)hipFree(c->ws.partials);
   (void)hipFree(c->dscal);
+  (void)hipFree(c->rcount);
   if (c->hpin) (void)hipHostFree(c->hpin);
   for (auto& e : c->tev)
     if (e) (void)hipEventDestroy(e);
@@ -438,27 +580,25 @@ int fx_norm2_dev(fx_ctx ctx, fx_vec x, double* dev_out) {
   return reduce_dispatch(ctx, 1, 0, 0.0, x, nullptr, nullptr, dev_out);
 }
 int fx_dot(fx_ctx ctx, fx_vec x, fx_vec y, double* out) {
-  FX_TRY(fx_dot_dev(ctx, x, y, ctx->dscal));
-  return fetch_scalar(ctx, 0, out);
+  clear_error();
+  FX_CHECK(y, FX_ERROR_INPUT_PAR, "null vector");
+  return reduce_host(ctx, 0, 0, 0.0, x, y, nullptr, out);
 }
 int fx_norm2(fx_ctx ctx, fx_vec x, double* out) {
-  FX_TRY(fx_norm2_dev(ctx, x, ctx->dscal));
-  return fetch_scalar(ctx, 0, out);
+  clear_error();
+  return reduce_host(ctx, 1, 0, 0.0, x, nullptr, nullptr, out);
 }
 int fx_norminf(fx_ctx ctx, fx_vec x, double* out) {
   clear_error();
-  FX_TRY(reduce_dispatch(ctx, 2, 0, 0.0, x, nullptr, nullptr, ctx->dscal));
-  return fetch_scalar(ctx, 0, out);
+  return reduce_host(ctx, 2, 0, 0.0, x, nullptr, nullptr, out);
 }
 int fx_max(fx_ctx ctx, fx_vec x, double* out) {
   clear_error();
-  FX_TRY(reduce_dispatch(ctx, 3, 0, 0.0, x, nullptr, nullptr, ctx->dscal));
-  return fetch_scalar(ctx, 0, out);
+  return reduce_host(ctx, 3, 0, 0.0, x, nullptr, nullptr, out);
 }
 int fx_min(fx_ctx ctx, fx_vec x, double* out) {
   clear_error();
-  FX_TRY(reduce_dispatch(ctx, 4, 0, 0.0, x, nullptr, nullptr, ctx->dscal));
-  return fetch_scalar(ctx, 0, out);
+  return reduce_host(ctx, 4, 0, 0.0, x, nullptr, nullptr, out);
 }
 int fx_shift(fx_ctx ctx, double a, fx_vec y) {
   clear_error();
@@ -480,20 +620,17 @@ int fx_sub(fx_ctx ctx, fx_vec v, fx_vec y) {
 int fx_axpy_norm2(fx_ctx ctx, double a, fx_vec x, fx_vec y, double* out) {
   clear_error();
   FX_CHECK(y, FX_ERROR_INPUT_PAR, "null vector");
-  FX_TRY(reduce_dispatch(ctx, 1, 1, a, x, y, nullptr, ctx->dscal));
-  return fetch_scalar(ctx, 0, out);
+  return reduce_host(ctx, 1, 1, a, x, y, nullptr, out);
 }
 int fx_xpay_norm2(fx_ctx ctx, double a, fx_vec x, fx_vec y, double* out) {
   clear_error();
   FX_CHECK(y, FX_ERROR_INPUT_PAR, "null vector");
-  FX_TRY(reduce_dispatch(ctx, 1, 2, a, x, y, nullptr, ctx->dscal));
-  return fetch_scalar(ctx, 0, out);
+  return reduce_host(ctx, 1, 2, a, x, y, nullptr, out);
 }
 int fx_axpy_dot(fx_ctx ctx, double a, fx_vec x, fx_vec y, fx_vec z, double* out) {
   clear_error();
   FX_CHECK(y && z, FX_ERROR_INPUT_PAR, "null vector");
-  FX_TRY(reduce_dispatch(ctx, 0, 1, a, x, y, z, ctx->dscal));
-  return fetch_scalar(ctx, 0, out);
+  return reduce_host(ctx, 0, 1, a, x, y, z, out);
 }
 
 }  // extern "C"

@@ -93,17 +93,6 @@ __global__ void k_f64_to_f32(const double* __restrict__ s, float* __restrict__ d
   for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += stride) d[i] = (float)s[i];
 }
 
-// max |x_i| into *out (one reduction)
-template <class T>
-__global__ __launch_bounds__(kThreads) void k_norminf(const T* __restrict__ x, uint32_t n,
-                                                      double* partials) {
-  double acc[1] = {0.0};
-  const uint32_t stride = gridDim.x * kThreads;
-  for (uint32_t i = blockIdx.x * kThreads + threadIdx.x; i < n; i += stride)
-    acc[0] = fmax(acc[0], fabs((double)x[i]));
-  block_partials<1, 1u>(acc, partials);
-}
-
 // r = b if ||x||_inf < CLOSE_ZERO, else the row chain b - A x
 // (MAT::Residual, src/MAT.cxx:459-469).
 template <class VT>
@@ -1065,20 +1054,15 @@ int fx_residual(fx_ctx ctx, fx_csr A, fx_vec b, fx_vec x, fx_vec r) {
   FX_CHECK(r->d != x->d, FX_ERROR_INPUT_PAR, "Residual with r aliasing x is not supported");
   if (A->nrow == 0) return 0;
   hipStream_t st = ctx->stream;
-  const unsigned g = stream_blocks(x->n);
   double* xinf = ctx->dscal + 1;
   if (x->dtype == FX_F64) {
-    hipLaunchKernelGGL(k_norminf<double>, dim3(g), dim3(kThreads), 0, st, (const double*)x->d, x->n,
-                       ctx->ws.partials);
-    FX_TRY((launch_finish<1, 1u>(st, ctx->ws.partials, g, FinStore<1>{xinf, 0})));
+    FX_TRY(norminf_dev(ctx, x->d, FX_F64, x->n, xinf));
     return launch_spmv<double, double, ROW_B_MINUS_AX, 0, 0u>(
         A, st, XLoad<double>{(const double*)x->d}, BLoad<double>{(const double*)b->d},
         EpiResidual<double>{(double*)r->d, (const double*)b->d, xinf}, nullptr);
   }
   FX_CHECK(A->va32 || !A->has_values, FX_ERROR_INPUT_PAR, "f32 residual needs fx_csr_make_f32");
-  hipLaunchKernelGGL(k_norminf<float>, dim3(g), dim3(kThreads), 0, st, (const float*)x->d, x->n,
-                     ctx->ws.partials);
-  FX_TRY((launch_finish<1, 1u>(st, ctx->ws.partials, g, FinStore<1>{xinf, 0})));
+  FX_TRY(norminf_dev(ctx, x->d, FX_F32, x->n, xinf));
   return launch_spmv<float, float, ROW_B_MINUS_AX, 0, 0u>(
       A, st, XLoad<float>{(const float*)x->d}, BLoad<float>{(const float*)b->d},
       EpiResidual<float>{(float*)r->d, (const float*)b->d, xinf}, nullptr);

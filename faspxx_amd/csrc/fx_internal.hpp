@@ -82,7 +82,8 @@ struct fx_ctx_s {
   bool own_stream = false;
   fx_red_ws ws;
   double* dscal = nullptr;  // device scalar slots for standalone reductions
-  double* hpin = nullptr;   // pinned host mirror of dscal
+  double* hpin = nullptr;   // pinned: the scalar a reduction hands to the host
+  unsigned* rcount = nullptr;  // workgroups done, of the reduction that runs (fx_core.hip)
   hipEvent_t tev[2] = {nullptr, nullptr};  // dispatch-attached timing events (fx_spmv_timed)
   int sms = 256;
   double* scratch = nullptr;  // this device's fx_pc_apply_noalloc scratch (fx_noalloc.hip)
@@ -240,6 +241,8 @@ constexpr uint32_t kSellRows = kThreads;
 constexpr uint32_t kSellMax = FX_SELL_MAX;
 constexpr uint32_t kSellNoRow = 0xFFFFFFFFu;
 
+// ||x||_inf of n elements into *dev_out (no synchronisation; fx_core.hip).
+int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, double* dev_out);
 int csr_spmv_dispatch(fx_ctx ctx, fx_csr A, const void* x, void* y, int dtype,
                       hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 int ensure_dinv32(fx_pc pc);
