@@ -300,16 +300,20 @@ int reduce_dispatch(fx_ctx ctx, int kind, int upd, double a, fx_vec x, fx_vec y,
 // is seen some 8 to 16 us later.  By then all the work queued before it is
 // done, x and y are read and an updated y is stored.  Whatever does not show
 // up soon (a long kernel queue, an error) is waited for on the stream.
+unsigned long long wait_pinned(const unsigned long long* slot, unsigned long long pending) {
+  for (int spin = 0; spin < 200000; ++spin) {
+    const unsigned long long bits = __atomic_load_n(slot, __ATOMIC_ACQUIRE);
+    if (bits != pending) return bits;
+  }
+  return pending;
+}
+
 int reduce_host(fx_ctx ctx, int kind, int upd, double a, fx_vec x, fx_vec y, fx_vec z,
                 double* out) {
   unsigned long long* slot = reinterpret_cast<unsigned long long*>(ctx->hpin);
   __atomic_store_n(slot, kRedPending, __ATOMIC_RELEASE);
   FX_TRY(reduce_dispatch(ctx, kind, upd, a, x, y, z, nullptr, ctx->hpin));
-  unsigned long long bits = kRedPending;
-  for (int spin = 0; spin < 200000; ++spin) {
-    bits = __atomic_load_n(slot, __ATOMIC_ACQUIRE);
-    if (bits != kRedPending) break;
-  }
+  unsigned long long bits = wait_pinned(slot, kRedPending);
   if (bits == kRedPending) {
     FX_HIP(hipStreamSynchronize(ctx->stream));
     bits = __atomic_load_n(slot, __ATOMIC_ACQUIRE);
@@ -318,10 +322,35 @@ int reduce_host(fx_ctx ctx, int kind, int upd, double a, fx_vec x, fx_vec y, fx_
   return 0;
 }
 
+__global__ void k_words_to_host(const uint32_t* __restrict__ src, int n,
+                                unsigned long long* __restrict__ host) {
+  if ((int)threadIdx.x < n)
+    __hip_atomic_store(host + threadIdx.x, (unsigned long long)src[threadIdx.x], __ATOMIC_RELAXED,
+                       __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, double* dev_out) {
   if (dtype == FX_F64)
     return launch_reduce<double>(ctx, 2, 0, 0.0, x, nullptr, nullptr, n, dev_out, nullptr);
   return launch_reduce<float>(ctx, 2, 0, 0.0, x, nullptr, nullptr, n, dev_out, nullptr);
+}
+
+// A copy of a few words to pageable memory and a wait took some 30 us.
+int read_words(fx_ctx ctx, const uint32_t* dev, int n, uint32_t* out) {
+  constexpr unsigned long long pending = ~0ull;  // no 32-bit word
+  unsigned long long* slots = reinterpret_cast<unsigned long long*>(ctx->hpin) + 8;
+  for (int i = 0; i < n; ++i) __atomic_store_n(slots + i, pending, __ATOMIC_RELEASE);
+  hipLaunchKernelGGL(k_words_to_host, dim3(1), dim3(64), 0, ctx->stream, dev, n, slots);
+  FX_HIP(hipGetLastError());
+  for (int i = 0; i < n; ++i) {
+    unsigned long long v = wait_pinned(slots + i, pending);
+    if (v == pending) {
+      FX_HIP(hipStreamSynchronize(ctx->stream));
+      v = __atomic_load_n(slots + i, __ATOMIC_ACQUIRE);
+    }
+    out[i] = (uint32_t)v;
+  }
+  return 0;
 }
 
 int convert_copy(fx_ctx ctx, const void* s, int sdt, void* d, int ddt, uint32_t n) {
@@ -367,7 +396,11 @@ static int ctx_init(fx_ctx c) {
   FX_HIP(hipMalloc(&c->ws.partials, sizeof(double) * 16 * 65536));
   FX_HIP(hipMalloc(&c->dscal, sizeof(double) * 64));
   FX_HIP(hipMalloc(&c->rcount, sizeof(unsigned) * kRedStride * kRedCounts));
-  FX_HIP(hipMemset(c->rcount, 0, sizeof(unsigned) * kRedStride * kRedCounts));
+  const size_t cb = sizeof(unsigned) * kRedStride * kRedCounts;
+  if (c->own_stream)  // a caller's stream may be one that is captured
+    FX_HIP(hipMemsetAsync(c->rcount, 0, cb, c->stream));
+  else
+    FX_HIP(hipMemset(c->rcount, 0, cb));
   FX_HIP(hipHostMalloc(&c->hpin, sizeof(double) * 64, hipHostMallocDefault));
   hipDeviceProp_t prop;
   FX_HIP(hipGetDeviceProperties(&prop, c->device));

@@ -71,12 +71,12 @@ __global__ void k_get_diag(const double* __restrict__ va, const uint32_t* __rest
 }
 
 // cd[k] = ci[k] - r0 for the entries of row block b (one workgroup per
-// block); *bad is set when a delta does not fit in 16 bits.
+// block; *nblk of them); *bad is set when a delta does not fit in 16 bits.
 __global__ void k_col_delta(const uint32_t* __restrict__ ci, const uint32_t* __restrict__ blk,
-                            uint32_t nblk,
+                            const uint32_t* __restrict__ nblk,
                             int16_t* __restrict__ cd, uint32_t* bad) {
   const uint32_t b = blockIdx.x;
-  if (b >= nblk) return;
+  if (b >= *nblk) return;
   const uint32_t r0 = blk[2 * b];
   const uint32_t k0 = blk[2 * b + 1], k1 = blk[2 * b + 3];
   bool fits = true;
@@ -255,6 +255,181 @@ __global__ void k_pattern_grad(const uint32_t* __restrict__ rp, const uint32_t* 
   if (i >= nrow) return;
   const double li = lam[i];
   for (uint32_t k = rp[i]; k < rp[i + 1]; ++k) g[k] = -(li * x[ci[k]]);
+}
+
+// ---- row blocks on the device ----------------------------------------------
+// build_row_blocks for a matrix whose row pointers are in HBM.  Where a block
+// ends depends on where it starts, a chain over all rows; it is followed per
+// tile of rows from every row that a block coming out of the tile before can
+// end at (a block has at most kBlockRows rows), and the tiles' answers are
+// then strung together.  (The chain on the host, with the copies of the row
+// pointers there and of the tables back, took 0.6 ms at 262144 rows.)
+constexpr uint32_t kBlkTile = 2048;
+
+struct BlkStage {
+  uint32_t rp[kBlkTile + kBlockRows + 1];
+  uint16_t next[kBlkTile];  // the row after the block that starts here, from the tile's start
+};
+
+__device__ __forceinline__ void blk_stage(const uint32_t* __restrict__ rp, uint32_t nrow,
+                                          BlkStage& s) {
+  const uint32_t t0 = blockIdx.x * kBlkTile;
+  for (uint32_t i = threadIdx.x; i <= kBlkTile + kBlockRows; i += kThreads)
+    s.rp[i] = rp[i < nrow - t0 ? t0 + i : nrow];
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < kBlkTile && i < nrow - t0; i += kThreads) {
+    const uint32_t base = s.rp[i];
+    uint32_t lo = 1, hi = min(kBlockRows, nrow - t0 - i);
+    if (s.rp[i + 1] - base <= kBlockNnz) {
+      while (lo < hi) {  // the most rows whose entries fit
+        const uint32_t mid = (lo + hi + 1) / 2;
+        if (s.rp[i + mid] - base <= kBlockNnz)
+          lo = mid;
+        else
+          hi = mid - 1;
+      }
+    }
+    s.next[i] = (uint16_t)(i + lo);
+  }
+  __syncthreads();
+}
+
+// walk[tile * kBlockRows + e]: for a first block at the tile's row e, the
+// blocks that start in the tile (low half) and the row of the next tile that
+// the last of them ends at (high half).  longest[tile]: its longest row.
+__global__ __launch_bounds__(kThreads) void k_blk_walk(const uint32_t* __restrict__ rp,
+                                                       uint32_t nrow, uint32_t* __restrict__ walk,
+                                                       uint32_t* __restrict__ longest) {
+  __shared__ BlkStage s;
+  __shared__ uint32_t mx;
+  if (threadIdx.x == 0) mx = 0;
+  blk_stage(rp, nrow, s);
+  const uint32_t left = min(kBlkTile, nrow - blockIdx.x * kBlkTile);
+  uint32_t m = 0;
+  for (uint32_t i = threadIdx.x; i < left; i += kThreads) m = max(m, s.rp[i + 1] - s.rp[i]);
+  atomicMax(&mx, m);
+  for (uint32_t e = threadIdx.x; e < kBlockRows; e += kThreads) {
+    uint32_t at = e, c = 0;
+    while (at < left) {
+      at = s.next[at];
+      ++c;
+    }
+    walk[(size_t)blockIdx.x * kBlockRows + e] = c | (at > kBlkTile ? at - kBlkTile : 0u) << 16;
+  }
+  __syncthreads();
+  if (threadIdx.x == 0) longest[blockIdx.x] = mx;
+}
+
+// Tile by tile: its first block's row and the blocks before it.  out: the
+// number of blocks, the longest row, and a zero.
+__global__ __launch_bounds__(kThreads) void k_blk_chain(const uint32_t* __restrict__ walk,
+                                                        const uint32_t* __restrict__ longest,
+                                                        uint32_t ntile, uint32_t* __restrict__ entry,
+                                                        uint32_t* __restrict__ before,
+                                                        uint32_t* __restrict__ out) {
+  constexpr uint32_t kAt = 32;  // tiles staged at a time
+  __shared__ uint32_t w[kAt * kBlockRows];
+  __shared__ uint32_t mx;
+  if (threadIdx.x == 0) mx = 0;
+  uint32_t e = 0, c = 0, m = 0;
+  for (uint32_t t0 = 0; t0 < ntile; t0 += kAt) {
+    const uint32_t nt = min(kAt, ntile - t0);
+    for (uint32_t i = threadIdx.x; i < nt * kBlockRows; i += kThreads)
+      w[i] = walk[(size_t)t0 * kBlockRows + i];
+    if (threadIdx.x < nt) m = max(m, longest[t0 + threadIdx.x]);
+    __syncthreads();
+    if (threadIdx.x == 0) {
+      for (uint32_t t = 0; t < nt; ++t) {
+        entry[t0 + t] = e;
+        before[t0 + t] = c;
+        const uint32_t v = w[t * kBlockRows + e];
+        c += v & 0xffffu;
+        e = v >> 16;
+      }
+    }
+    __syncthreads();
+  }
+  atomicMax(&mx, m);
+  __syncthreads();
+  if (threadIdx.x == 0) out[0] = c, out[1] = mx, out[2] = 0;
+}
+
+__global__ __launch_bounds__(kThreads) void k_blk_fill(const uint32_t* __restrict__ rp,
+                                                       uint32_t nrow,
+                                                       const uint32_t* __restrict__ entry,
+                                                       const uint32_t* __restrict__ before,
+                                                       uint32_t* __restrict__ blk,
+                                                       const uint32_t* __restrict__ nblk,
+                                                       uint16_t* __restrict__ rpb) {
+  __shared__ BlkStage s;
+  __shared__ uint16_t start[kBlkTile + 1];
+  __shared__ uint32_t count;
+  blk_stage(rp, nrow, s);
+  const uint32_t t0 = blockIdx.x * kBlkTile, left = min(kBlkTile, nrow - t0);
+  if (threadIdx.x == 0) {
+    uint32_t at = entry[blockIdx.x], c = 0;
+    while (at < left) {
+      start[c++] = (uint16_t)at;
+      at = s.next[at];
+    }
+    start[c] = (uint16_t)at;
+    count = c;
+  }
+  __syncthreads();
+  const uint32_t lane = threadIdx.x & 63, b0 = before[blockIdx.x];
+  for (uint32_t b = threadIdx.x >> 6; b < count; b += kWaves) {
+    const uint32_t r0 = start[b], r1 = start[b + 1], k0 = s.rp[r0];
+    if (lane == 0) {
+      blk[2 * (b0 + b)] = t0 + r0;
+      blk[2 * (b0 + b) + 1] = k0;
+    }
+    for (uint32_t r = r0 + lane; r < r1; r += 64) rpb[t0 + r] = (uint16_t)(s.rp[r] - k0);
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    blk[2 * *nblk] = nrow;
+    blk[2 * *nblk + 1] = rp[nrow];
+  }
+}
+
+// A->blk, rpb, cd (where all deltas fit, unless col32), nblk and max_row from
+// A->rp and ci.  A block is full, or it and the next row hold more than
+// kBlockNnz entries; so there are at most nrow / kBlockRows + 2 nnz /
+// kBlockNnz + 2 of them, and the host need not wait for their number.
+int device_blocks(fx_csr A, bool col32) {
+  hipStream_t st = A->ctx->stream;
+  const uint32_t nt = (A->nrow + kBlkTile - 1) / kBlkTile;
+  const size_t most = (size_t)A->nrow / kBlockRows + 2 * ((size_t)A->nnz / kBlockNnz) + 2;
+  uint32_t* tmp = nullptr;  // {blocks, longest row, bad}, entry[nt], before[nt], longest[nt], walk
+  FX_HIP(hipMalloc(&tmp, sizeof(uint32_t) * (3 + (size_t)nt * (3 + kBlockRows))));
+  uint32_t *entry = tmp + 3, *before = entry + nt, *longest = before + nt, *walk = longest + nt;
+  uint32_t got[3] = {0, 0, 0};
+  auto run = [&]() -> int {
+    FX_HIP(hipMalloc(&A->rpb, sizeof(uint16_t) * A->nrow));
+    FX_HIP(hipMalloc(&A->blk, sizeof(uint32_t) * 2 * (most + 1)));
+    hipLaunchKernelGGL(k_blk_walk, dim3(nt), dim3(kThreads), 0, st, A->rp, A->nrow, walk, longest);
+    hipLaunchKernelGGL(k_blk_chain, dim3(1), dim3(kThreads), 0, st, walk, longest, nt, entry,
+                       before, tmp);
+    hipLaunchKernelGGL(k_blk_fill, dim3(nt), dim3(kThreads), 0, st, A->rp, A->nrow, entry, before,
+                       A->blk, tmp, A->rpb);
+    if (!col32) {
+      FX_HIP(hipMalloc(&A->cd, sizeof(int16_t) * A->nnz));
+      hipLaunchKernelGGL(k_col_delta, dim3((unsigned)most), dim3(kThreads), 0, st, A->ci, A->blk,
+                         tmp, A->cd, tmp + 2);
+    }
+    FX_HIP(hipGetLastError());
+    FX_TRY(read_words(A->ctx, tmp, 3, got));
+    A->nblk = got[0];
+    A->max_row = got[1];
+    return 0;
+  };
+  const int rc = run();
+  if (rc) (void)hipStreamSynchronize(st);
+  (void)hipFree(tmp);
+  if (got[2]) {
+    (void)hipFree(A->cd);
+    A->cd = nullptr;
+  }
+  return rc;
 }
 
 int csr_alloc(fx_csr A) {
@@ -629,6 +804,7 @@ int build_sorted(fx_csr A, const uint32_t* hrp, const uint32_t* hci) {
   return 0;
 }
 
+// host_rp null: the row pointers are A->rp alone (and host_ci is null too).
 int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
   // Row patterns for a matrix given on the host (FASPXX_FX_NOPAT=1: none;
   // FASPXX_FX_COL32=1 keeps u32 columns); they get their own row blocks.
@@ -639,6 +815,7 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
   const char* e = std::getenv("FASPXX_FX_COL32");
   const bool col32_env = e && e[0] == '1';
   const bool col32 = col32_env || sell == 2;
+  if (!host_rp) return device_blocks(A, col32);
   std::vector<uint8_t> pid;
   std::vector<int32_t> dict;
   std::vector<uint32_t> first;
@@ -649,6 +826,7 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
     for (uint32_t r = 0; r < A->nrow; ++r) longest = std::max(longest, host_rp[r + 1] - host_rp[r]);
     pat = build_patterns(A->nrow, host_rp, host_ci, longest, pid, dict, first, plen, npat);
   }
+  hipStream_t st = A->ctx->stream;
   uint32_t mx = 0;
   const std::vector<uint32_t> rows =
       pat ? build_row_blocks(A->nrow, host_rp, &mx, kPatRows, kPatNnz)
@@ -661,7 +839,6 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
     blk[2 * b + 1] = host_rp[rows[b]];
   }
   FX_HIP(hipMalloc(&A->blk, sizeof(uint32_t) * blk.size()));
-  hipStream_t st = A->ctx->stream;
   FX_HIP(hipMemcpyAsync(A->blk, blk.data(), sizeof(uint32_t) * blk.size(), hipMemcpyHostToDevice,
                         st));
   std::vector<uint16_t> rpb(A->nrow ? A->nrow : 1, 0);
@@ -708,21 +885,24 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
   if (A->nnz && A->nblk && !col32) {
     uint32_t* bad = nullptr;
     FX_HIP(hipMalloc(&A->cd, sizeof(int16_t) * A->nnz));
-    FX_HIP(hipMalloc(&bad, sizeof(uint32_t)));
+    FX_HIP(hipMalloc(&bad, 2 * sizeof(uint32_t)));  // the flag, and the number of blocks
     uint32_t hbad = 0;
-    hipError_t err = hipMemsetAsync(bad, 0, sizeof(uint32_t), st);
+    const uint32_t words[2] = {0, A->nblk};
+    hipError_t err = hipMemcpyAsync(bad, words, sizeof(words), hipMemcpyHostToDevice, st);
     if (err == hipSuccess) {
       hipLaunchKernelGGL(k_col_delta, dim3(A->nblk), dim3(kThreads), 0, st, A->ci, A->blk,
-                         A->nblk, A->cd, bad);
+                         (const uint32_t*)(bad + 1), A->cd, bad);
       err = hipGetLastError();
     }
-    if (err == hipSuccess) err = hipMemcpyAsync(&hbad, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, st);
-    if (err == hipSuccess) err = hipStreamSynchronize(st);
+    int rc = 0;
+    if (err == hipSuccess) rc = read_words(A->ctx, bad, 1, &hbad);
+    if (err != hipSuccess || rc) (void)hipStreamSynchronize(st);
     (void)hipFree(bad);
-    if (err != hipSuccess || hbad) {
+    if (err != hipSuccess || rc || hbad) {
       (void)hipFree(A->cd);
       A->cd = nullptr;
       FX_HIP(err);
+      FX_TRY(rc);
     }
   }
   if (host_ci && !A->cd && sell != 2 && !col32_env && sort_enabled() && A->nrow && A->nnz) {
@@ -730,7 +910,7 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
   } else if (!A->cd && (sell == 2 || (sell == 1 && !col32_env))) {
     FX_TRY(build_sell(A, host_rp, host_ci));
   }
-  FX_HIP(hipStreamSynchronize(st));
+  FX_HIP(hipStreamSynchronize(st));  // the host vectors go out of scope
   return 0;
 }
 
@@ -790,8 +970,8 @@ int csr_pattern_blocks512(fx_csr A, uint32_t** blk, uint16_t** rpb, uint32_t* nb
 void csr_release(fx_csr A) { csr_free(A); }
 
 int scan_u32(hipStream_t st, const uint32_t* cnt, uint32_t m, uint32_t* out) {
-  if (m <= kScanTile) {
-    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, cnt, m, out);
+  if (m <= kScanTile) {  // one tile, whose total is out[m]
+    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, st, cnt, m, out, out + m);
     FX_HIP(hipGetLastError());
     return 0;
   }
@@ -800,7 +980,11 @@ int scan_u32(hipStream_t st, const uint32_t* cnt, uint32_t m, uint32_t* out) {
   uint32_t* tmp = nullptr;  // tile totals [0, nt), their scan [nt, 2 nt + 1)
   FX_HIP(hipMallocAsync((void**)&tmp, sizeof(uint32_t) * (2 * (size_t)nt + 1), st));
   hipLaunchKernelGGL(k_scan_tiles, dim3(nt), dim3(1024), 0, st, cnt, m, out, tmp);
-  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, (const uint32_t*)tmp, nt, tmp + nt);
+  if (nt <= kScanTile)
+    hipLaunchKernelGGL(k_scan_tiles, dim3(1), dim3(1024), 0, st, (const uint32_t*)tmp, nt,
+                       tmp + nt, tmp + 2 * (size_t)nt);
+  else
+    hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, (const uint32_t*)tmp, nt, tmp + nt);
   hipLaunchKernelGGL(k_scan_add, dim3(nt), dim3(1024), 0, st, out, m, (const uint32_t*)(tmp + nt),
                      nt);
   const hipError_t e = hipGetLastError();
@@ -816,11 +1000,11 @@ int csr_finish_device(fx_csr A) {
                        0, st, A->rp, A->ci, A->dp, A->nrow);
     FX_HIP(hipGetLastError());
   }
-  std::vector<uint32_t> hrp((size_t)A->nrow + 1);
-  FX_HIP(hipMemcpyAsync(hrp.data(), A->rp, sizeof(uint32_t) * hrp.size(), hipMemcpyDeviceToHost,
-                        st));
-  FX_HIP(hipStreamSynchronize(st));
-  return csr_set_blocks(A, hrp.data(), nullptr);
+  if (!A->nrow) {
+    const uint32_t rp0 = 0;
+    return csr_set_blocks(A, &rp0, nullptr);
+  }
+  return csr_set_blocks(A, nullptr, nullptr);
 }
 
 int csr_spmv_dispatch(fx_ctx ctx, fx_csr A, const void* x, void* y, int dtype, hipEvent_t e0,
@@ -1109,18 +1293,21 @@ int fx_csr_transpose(fx_ctx ctx, fx_csr A, fx_csr* At) {
   const uint32_t m = A->mcol, nnz = A->nnz;
   uint32_t *cnt = nullptr, *perm = nullptr, *sorted = nullptr, *rid = nullptr;
   auto cleanup = [&]() {
-    (void)hipStreamSynchronize(st);
-    (void)hipFree(cnt);
-    (void)hipFree(perm);
-    (void)hipFree(sorted);
-    (void)hipFree(rid);
+    for (uint32_t* p : {cnt, perm, rid})
+      if (p) (void)hipFreeAsync(p, st);
+    if (sorted) {
+      (void)hipStreamSynchronize(st);
+      (void)hipFree(sorted);
+    }
   };
   auto keep_sorted = [&]() {  // becomes T->src
     T->src = sorted;
     sorted = nullptr;
   };
-  if (hipMalloc(&cnt, sizeof(uint32_t) * (m + 1)) || hipMalloc(&perm, sizeof(uint32_t) * nnz) ||
-      hipMalloc(&sorted, sizeof(uint32_t) * nnz) || hipMalloc(&rid, sizeof(uint32_t) * nnz)) {
+  if (hipMallocAsync((void**)&cnt, sizeof(uint32_t) * ((size_t)m + 1), st) ||
+      hipMallocAsync((void**)&perm, sizeof(uint32_t) * nnz, st) ||
+      hipMallocAsync((void**)&rid, sizeof(uint32_t) * nnz, st) ||
+      hipMalloc(&sorted, sizeof(uint32_t) * nnz)) {
     cleanup();
     csr_free(T);
     set_error("transpose: allocation failed");
@@ -1129,7 +1316,12 @@ int fx_csr_transpose(fx_ctx ctx, fx_csr A, fx_csr* At) {
   const unsigned gz = stream_blocks(nnz);
   (void)hipMemsetAsync(cnt, 0, sizeof(uint32_t) * (m + 1), st);
   hipLaunchKernelGGL(k_col_count, dim3(gz), dim3(kThreads), 0, st, A->ci, nnz, cnt);
-  hipLaunchKernelGGL(k_scan, dim3(1), dim3(1024), 0, st, cnt, m, T->rp);
+  rc = scan_u32(st, cnt, m, T->rp);
+  if (rc) {
+    cleanup();
+    csr_free(T);
+    return rc;
+  }
   (void)hipMemcpyAsync(cnt, T->rp, sizeof(uint32_t) * m, hipMemcpyDeviceToDevice, st);
   hipLaunchKernelGGL(k_scatter, dim3(gz), dim3(kThreads), 0, st, A->ci, nnz, cnt, perm);
   hipLaunchKernelGGL(k_rank_rows, dim3((m + kWaves - 1) / kWaves), dim3(kThreads), 0, st, T->rp, m,
@@ -1147,17 +1339,9 @@ int fx_csr_transpose(fx_ctx ctx, fx_csr A, fx_csr* At) {
     set_error("transpose kernels: %s", hipGetErrorString(e));
     return FX_ERROR_DEVICE;
   }
-  std::vector<uint32_t> hrp(m + 1);
-  if (hipMemcpyAsync(hrp.data(), T->rp, sizeof(uint32_t) * (m + 1), hipMemcpyDeviceToHost, st) ||
-      hipStreamSynchronize(st)) {
-    cleanup();
-    csr_free(T);
-    set_error("transpose: download failed");
-    return FX_ERROR_DEVICE;
-  }
   keep_sorted();
   cleanup();
-  rc = csr_set_blocks(T, hrp.data(), nullptr);
+  rc = csr_set_blocks(T, nullptr, nullptr);
   if (rc) {
     csr_free(T);
     return rc;

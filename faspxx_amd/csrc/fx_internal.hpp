@@ -241,6 +241,9 @@ constexpr uint32_t kSellRows = kThreads;
 constexpr uint32_t kSellMax = FX_SELL_MAX;
 constexpr uint32_t kSellNoRow = 0xFFFFFFFFu;
 
+// The first n (at most 8) of the 32-bit words at dev, once the work queued
+// before is done (fx_core.hip).
+int read_words(fx_ctx ctx, const uint32_t* dev, int n, uint32_t* out);
 // ||x||_inf of n elements into *dev_out (no synchronisation; fx_core.hip).
 int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, double* dev_out);
 int csr_spmv_dispatch(fx_ctx ctx, fx_csr A, const void* x, void* y, int dtype,

@@ -17,9 +17,10 @@
 // diagonal entry).  Structure-only operands (no values) give a structure-
 // only result for the triangular parts and the product; a + b needs values.
 //
-// These run once per setup, so each kernel gives a row to a thread.  The
-// product accumulates each row in an open-addressing table (twice the
-// row's candidate count, so every probe sequence ends) kept in HBM scratch.
+// The kernels give a row to a thread; the product gives it to a few lanes.  It
+// accumulates each row in an open-addressing table (at least twice as many
+// slots as the row has distinct columns, so every probe sequence ends) kept in
+// LDS, or in HBM scratch for matrices with longer rows.
 #include <vector>
 
 #include "fx_internal.hpp"
@@ -155,24 +156,179 @@ __global__ void k_shift_diag(const uint32_t* __restrict__ dp, double* __restrict
 
 // ---- L R ------------------------------------------------------------------
 // Candidate products of row i: the summed lengths of the rows of R that row
-// i of L selects.
-__global__ void k_mult_count(const uint32_t* __restrict__ lrp, const uint32_t* __restrict__ lci,
-                             const uint32_t* __restrict__ rrp, uint32_t nrow,
-                             uint32_t* __restrict__ cand) {
+// i of L selects.  Per workgroup their sum (two words) and the largest.
+__global__ __launch_bounds__(kThreads) void k_mult_count(
+    const uint32_t* __restrict__ lrp, const uint32_t* __restrict__ lci,
+    const uint32_t* __restrict__ rrp, uint32_t nrow, uint32_t* __restrict__ cand,
+    unsigned long long* __restrict__ sums, uint32_t* __restrict__ most) {
+  __shared__ unsigned long long total;
+  __shared__ uint32_t top;
+  if (threadIdx.x == 0) total = 0, top = 0;
+  __syncthreads();
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  if (i >= nrow) return;
   uint32_t c = 0;
-  for (uint32_t k = lrp[i]; k < lrp[i + 1]; ++k) {
-    const uint32_t r = lci[k];
-    c += rrp[r + 1] - rrp[r];
+  if (i < nrow) {
+    for (uint32_t k = lrp[i]; k < lrp[i + 1]; ++k) {
+      const uint32_t r = lci[k];
+      c += rrp[r + 1] - rrp[r];
+    }
+    cand[i] = c;
   }
-  cand[i] = c;
+  atomicAdd(&total, (unsigned long long)c);
+  atomicMax(&top, c);
+  __syncthreads();
+  if (threadIdx.x == 0) sums[blockIdx.x] = total, most[blockIdx.x] = top;
+}
+
+// out: the matrix's sum of candidates (low and high word) and the largest.
+__global__ __launch_bounds__(1024) void k_mult_total(const unsigned long long* __restrict__ sums,
+                                                     const uint32_t* __restrict__ most,
+                                                     uint32_t nb, uint32_t* __restrict__ out) {
+  __shared__ unsigned long long total;
+  __shared__ uint32_t top;
+  if (threadIdx.x == 0) total = 0, top = 0;
+  __syncthreads();
+  unsigned long long t = 0;
+  uint32_t m = 0;
+  for (uint32_t b = threadIdx.x; b < nb; b += 1024) t += sums[b], m = max(m, most[b]);
+  atomicAdd(&total, t);
+  atomicMax(&top, m);
+  __syncthreads();
+  if (threadIdx.x == 0) out[0] = (uint32_t)total, out[1] = (uint32_t)(total >> 32), out[2] = top;
+}
+
+// Rows of up to kMultMost candidates: a row's table stays in LDS, and G lanes
+// take a row, the entries of one row of R side by side.  The first pass counts
+// the distinct columns, the second writes them, in order of first appearance,
+// and their values; no scratch, no copy.  (A thread per row with its table in
+// HBM, compacted afterwards, took 1.15 ms and 360 MB of scratch for A A of
+// the 7-point stencil on 64^3 points; these take 0.13 ms.)  What bounds them is the
+// chain of LDS operations per row of R, so a batch of those rows is loaded
+// before the first is entered.
+constexpr uint32_t kMultShort = 64, kMultMost = 512;
+
+__device__ __forceinline__ void wave_order() {  // LDS operations of a wave, in program order
+  __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+}
+
+template <uint32_t CAP>
+__device__ __forceinline__ uint32_t mult_slot(uint32_t* keys, uint32_t col, bool& fresh) {
+  static_assert((CAP & (CAP - 1)) == 0, "a power of two");
+  uint32_t h = (col * 2654435761u) >> (32 - __builtin_ctz(CAP));
+  for (;;) {  // at most CAP / 2 keys: an empty slot ends it
+    const uint32_t key = atomicCAS(keys + h, kEmpty, col);
+    fresh = key == kEmpty;
+    if (fresh || key == col) return h;
+    h = (h + 1) & (CAP - 1);
+  }
+}
+
+template <uint32_t G, uint32_t MORE, uint32_t MOST, bool FILL>
+__global__ __launch_bounds__(kThreads) void k_mult_lds(
+    const uint32_t* __restrict__ lrp, const uint32_t* __restrict__ lci,
+    const double* __restrict__ lva, const uint32_t* __restrict__ rrp,
+    const uint32_t* __restrict__ rci, const double* __restrict__ rva, uint32_t nrow,
+    const uint32_t* __restrict__ cand, uint32_t* __restrict__ cnt,
+    const uint32_t* __restrict__ orp, uint32_t* __restrict__ oci, double* __restrict__ ova) {
+  constexpr uint32_t ROWS = kThreads / G, CAP = 2 * MOST, BATCH = 4;
+  __shared__ uint4 keys4[ROWS * CAP / 4];
+  __shared__ uint4 tags4[FILL ? ROWS * CAP / 4 : 1];  // claiming lane << 16 | place in the row
+  __shared__ double vals_[FILL ? ROWS * MOST : 1];
+  const uint32_t lane = threadIdx.x & 63, gl = lane % G, grp = threadIdx.x / G;
+  const uint32_t i = blockIdx.x * ROWS + grp;
+  if (i >= nrow) return;
+  const uint32_t P = cand[i];
+  if (P > MOST || (MORE && P <= MORE)) return;
+  const unsigned long long mine = G == 64 ? ~0ull : ((1ull << (G % 64)) - 1) << (lane - gl);
+  for (uint32_t j = gl; j < CAP / 4; j += G) {
+    const uint4 e = {kEmpty, kEmpty, kEmpty, kEmpty};
+    keys4[grp * (CAP / 4) + j] = e;
+    if constexpr (FILL) tags4[grp * (CAP / 4) + j] = e;
+  }
+  wave_order();
+  uint32_t* keys = reinterpret_cast<uint32_t*>(keys4) + grp * CAP;
+  uint32_t* tags = reinterpret_cast<uint32_t*>(tags4) + (FILL ? grp * CAP : 0);
+  double* vals = vals_ + (FILL ? grp * MOST : 0);
+  const uint32_t o = FILL ? orp[i] : 0;
+  uint32_t c = 0;  // distinct columns so far
+
+  auto enter = [&](bool on, uint32_t col, double a, double b) {
+    bool fresh = false;
+    uint32_t h = 0;
+    if (on) h = mult_slot<CAP>(keys, col, fresh);
+    if constexpr (!FILL) {
+      c += __popcll(__ballot(fresh) & mine);
+    } else {
+      // of lanes with one column (a row of R may repeat one) the first leads
+      wave_order();
+      const uint32_t place = on ? tags[h] & 0xffffu : 0u;  // 0xffff: not yet placed
+      wave_order();
+      if (on) atomicMin(tags + h, gl << 16 | place);
+      wave_order();
+      const bool lead = on && tags[h] >> 16 == gl;
+      const bool first = lead && place == 0xffffu;
+      const unsigned long long firsts = __ballot(first) & mine;
+      const uint32_t p = first ? c + __popcll(firsts & ((1ull << lane) - 1)) : place;
+      c += __popcll(firsts);
+      wave_order();
+      if (lead) {
+        tags[h] = 0xffff0000u | p;
+        vals[p] = fma(a, b, first ? 0.0 : vals[p]);
+        if (first) oci[o + p] = col;
+      }
+      unsigned long long rest = __ballot(on && !lead) & mine;
+      while (rest) {  // repeats, in their order
+        wave_order();
+        if (lane == (uint32_t)__builtin_ctzll(rest)) {
+          const uint32_t q = tags[h] & 0xffffu;
+          vals[q] = fma(a, b, vals[q]);
+        }
+        rest &= rest - 1;
+      }
+      wave_order();
+    }
+  };
+
+  const uint32_t le = lrp[i + 1];
+  for (uint32_t k0 = lrp[i]; k0 < le; k0 += BATCH) {
+    uint32_t s[BATCH], e[BATCH], col[BATCH];
+    double a[BATCH], b[BATCH];
+#pragma unroll
+    for (uint32_t j = 0; j < BATCH; ++j) {
+      const uint32_t k = min(k0 + j, le - 1), r = lci[k];
+      a[j] = FILL && lva ? lva[k] : 1.0;
+      s[j] = rrp[r];
+      e[j] = k0 + j < le ? rrp[r + 1] : s[j];
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < BATCH; ++j) {
+      const bool on = s[j] + gl < e[j];
+      col[j] = on ? rci[s[j] + gl] : 0u;
+      b[j] = FILL && on && rva ? rva[s[j] + gl] : 1.0;
+    }
+#pragma unroll
+    for (uint32_t j = 0; j < BATCH; ++j) {
+      if (s[j] < e[j]) enter(s[j] + gl < e[j], col[j], a[j], b[j]);
+      for (uint32_t l0 = s[j] + G; l0 < e[j]; l0 += G) {
+        const bool on = l0 + gl < e[j];
+        const uint32_t cl = on ? rci[l0 + gl] : 0u;
+        enter(on, cl, a[j], FILL && on && rva ? rva[l0 + gl] : 1.0);
+      }
+    }
+  }
+  if constexpr (!FILL) {
+    if (gl == 0) cnt[i] = c;
+  } else if (ova) {
+    for (uint32_t j = gl; j < c; j += G) ova[o + j] = vals[j];
+  }
 }
 
 __device__ __forceinline__ uint32_t col_hash(uint32_t c, uint32_t cap) {
   return (uint32_t)(((uint64_t)(c * 2654435761u) * cap) >> 32);
 }
 
+// Matrices with a row of more than kMultMost candidates.
 // Row i: its candidates (L's entries in order, then each R row in order)
 // through an open-addressing table of 2 * cand_i slots at keys[2 * off_i];
 // a column's first candidate appends it to the row's list at tcol/tval +
@@ -240,32 +396,35 @@ __global__ void k_mult_copy(const uint32_t* __restrict__ off, const uint32_t* __
   }
 }
 
-// Device scratch released on every exit path.
+// Device scratch released on every exit path: small buffers by hipMalloc (1 us
+// each here, and freed after a wait), large ones in the stream's order.
+// (hipMalloc and hipFree of tables of 100 MB took 1.8 of the 8.8 ms of a
+// product, a sum, a triangular part and a transpose at 262144 rows.)
 struct Scratch {
   hipStream_t st;
-  std::vector<void*> bufs;
+  std::vector<void*> small, large;
   explicit Scratch(hipStream_t s) : st(s) {}
   template <class T>
   T* get(size_t count) {
     void* p = nullptr;
-    if (hipMalloc(&p, sizeof(T) * (count ? count : 1)) != hipSuccess) return nullptr;
-    bufs.push_back(p);
+    const size_t bytes = sizeof(T) * (count ? count : 1);
+    const bool lg = bytes > (2u << 20);
+    if ((lg ? hipMallocAsync(&p, bytes, st) : hipMalloc(&p, bytes)) != hipSuccess) return nullptr;
+    (lg ? large : small).push_back(p);
     return (T*)p;
   }
   ~Scratch() {
-    (void)hipStreamSynchronize(st);
-    for (void* p : bufs) (void)hipFree(p);
+    for (void* p : large) (void)hipFreeAsync(p, st);
+    if (!small.empty()) (void)hipStreamSynchronize(st);
+    for (void* p : small) (void)hipFree(p);
   }
 };
 
 // A new matrix handle of the given shape whose rp is `rp` (device, nrow + 1
-// entries, already scanned): reads nnz = rp[nrow], allocates the rest.
+// entries, already scanned): allocates the rest.
 int new_from_rowptr(fx_ctx ctx, uint32_t nrow, uint32_t mcol, bool values, uint32_t* rp,
-                    fx_csr* out) {
+                    uint32_t nnz, fx_csr* out) {
   hipStream_t st = ctx->stream;
-  uint32_t nnz = 0;
-  FX_HIP(hipMemcpyAsync(&nnz, rp + nrow, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  FX_HIP(hipStreamSynchronize(st));
   fx_csr C = new fx_csr_s();
   C->ctx = ctx;
   if (nnz == 0) {  // MAT::Empty, src/MAT.cxx:26-29
@@ -309,7 +468,7 @@ int finish(fx_csr C, fx_csr* out) {
 
 int scaled_copy(fx_ctx ctx, double s, fx_csr X, fx_csr* out) {
   fx_csr C = nullptr;
-  FX_TRY(new_from_rowptr(ctx, X->nrow, X->mcol, true, X->rp, &C));
+  FX_TRY(new_from_rowptr(ctx, X->nrow, X->mcol, true, X->rp, X->nnz, &C));
   hipLaunchKernelGGL(k_scaled_copy, dim3(stream_blocks(X->nnz)), dim3(kThreads), 0, ctx->stream,
                      X->ci, X->va, s, X->nnz, C->ci, C->va);
   return finish(C, out);
@@ -329,20 +488,19 @@ int tri_part(fx_ctx ctx, fx_csr A, int upper, fx_csr* out) {
   const uint32_t n = A->nrow;
   Scratch S(st);
   uint32_t* cnt = S.get<uint32_t>(n);
-  uint32_t* orp = S.get<uint32_t>((size_t)n + 1);
-  uint32_t* bad = S.get<uint32_t>(1);
-  FX_CHECK(cnt && orp && bad, FX_ERROR_ALLOC_MEM, "triangular part: allocation failed");
+  uint32_t* orp = S.get<uint32_t>((size_t)n + 2);
+  FX_CHECK(cnt && orp, FX_ERROR_ALLOC_MEM, "triangular part: allocation failed");
+  uint32_t* bad = orp + n + 1;  // read with the number of entries
   FX_HIP(hipMemsetAsync(bad, 0, sizeof(uint32_t), st));
   hipLaunchKernelGGL(k_tri_count, dim3(row_blocks(n)), dim3(kThreads), 0, st, A->rp, A->ci, A->dp,
                      n, upper, cnt, bad);
   FX_HIP(hipGetLastError());
-  uint32_t hbad = 0;
-  FX_HIP(hipMemcpyAsync(&hbad, bad, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-  FX_HIP(hipStreamSynchronize(st));
-  FX_CHECK(!hbad, FX_ERROR_MAT_DATA, "triangular part needs a diagonal entry in every row");
   FX_TRY(scan_u32(st, cnt, n, orp));
+  uint32_t got[2];
+  FX_TRY(read_words(ctx, orp + n, 2, got));
+  FX_CHECK(!got[1], FX_ERROR_MAT_DATA, "triangular part needs a diagonal entry in every row");
   fx_csr C = nullptr;
-  FX_TRY(new_from_rowptr(ctx, n, A->mcol, A->has_values, orp, &C));
+  FX_TRY(new_from_rowptr(ctx, n, A->mcol, A->has_values, orp, got[0], &C));
   hipLaunchKernelGGL(k_tri_copy, dim3(row_blocks(n)), dim3(kThreads), 0, st, A->rp, A->ci,
                      A->has_values ? A->va : nullptr, A->dp, n, upper, C->rp, C->ci,
                      C->has_values ? C->va : nullptr);
@@ -389,8 +547,10 @@ int fx_csr_add(fx_ctx ctx, double a, fx_csr A, double b, fx_csr B, fx_csr* C) {
                      B->ci, n, cnt);
   FX_HIP(hipGetLastError());
   FX_TRY(scan_u32(st, cnt, n, orp));
+  uint32_t nnz = 0;
+  FX_TRY(read_words(ctx, orp + n, 1, &nnz));
   fx_csr R = nullptr;
-  FX_TRY(new_from_rowptr(ctx, n, A->mcol, true, orp, &R));
+  FX_TRY(new_from_rowptr(ctx, n, A->mcol, true, orp, nnz, &R));
   hipLaunchKernelGGL(k_add_fill, dim3(row_blocks(n)), dim3(kThreads), 0, st, a, A->rp, A->ci,
                      A->va, b, B->rp, B->ci, B->va, n, R->rp, R->ci, R->va);
   return finish(R, C);
@@ -421,23 +581,53 @@ int fx_csr_mult(fx_ctx ctx, fx_csr L, fx_csr R, fx_csr* C) {
   const uint32_t n = L->nrow;
   const bool values = L->has_values && R->has_values;
   Scratch S(st);
+  const unsigned nb = row_blocks(n);
   uint32_t* cand = S.get<uint32_t>(n);
-  uint32_t* off = S.get<uint32_t>((size_t)n + 1);
   uint32_t* cnt = S.get<uint32_t>(n);
   uint32_t* orp = S.get<uint32_t>((size_t)n + 1);
-  FX_CHECK(cand && off && cnt && orp, FX_ERROR_ALLOC_MEM, "L R: allocation failed");
-  hipLaunchKernelGGL(k_mult_count, dim3(row_blocks(n)), dim3(kThreads), 0, st, L->rp, L->ci, R->rp,
-                     n, cand);
+  auto* sums = S.get<unsigned long long>(nb);
+  uint32_t* most = S.get<uint32_t>((size_t)nb + 3);
+  FX_CHECK(cand && cnt && orp && sums && most, FX_ERROR_ALLOC_MEM, "L R: allocation failed");
+  hipLaunchKernelGGL(k_mult_count, dim3(nb), dim3(kThreads), 0, st, L->rp, L->ci, R->rp, n, cand,
+                     sums, most);
+  hipLaunchKernelGGL(k_mult_total, dim3(1), dim3(1024), 0, st, sums, most, nb, most + nb);
   FX_HIP(hipGetLastError());
+  uint32_t got[3];
+  FX_TRY(read_words(ctx, most + nb, 3, got));
   // the candidate total must fit the u32 offsets
-  std::vector<uint32_t> hc(n);
-  FX_HIP(hipMemcpyAsync(hc.data(), cand, sizeof(uint32_t) * n, hipMemcpyDeviceToHost, st));
-  FX_HIP(hipStreamSynchronize(st));
-  uint64_t total = 0;
-  for (uint32_t v : hc) total += v;
+  const uint64_t total = got[0] | (uint64_t)got[1] << 32;
   FX_CHECK(total < 0x80000000ull, FX_ERROR_ALLOC_MEM,
            "L R: %llu candidate products exceed the 2^31 scratch limit",
            (unsigned long long)total);
+  fx_csr P = nullptr;
+  uint32_t nnz = 0;
+  if (got[2] <= kMultMost) {
+    const double *lv = values ? L->va : nullptr, *rv = values ? R->va : nullptr;
+    const dim3 gs((n + kThreads / 8 - 1) / (kThreads / 8)), gw((n + kWaves - 1) / kWaves);
+    hipLaunchKernelGGL((k_mult_lds<8, 0, kMultShort, false>), gs, dim3(kThreads), 0, st, L->rp,
+                       L->ci, lv, R->rp, R->ci, rv, n, cand, cnt, nullptr, nullptr, nullptr);
+    if (got[2] > kMultShort)
+      hipLaunchKernelGGL((k_mult_lds<64, kMultShort, kMultMost, false>), gw, dim3(kThreads), 0, st,
+                         L->rp, L->ci, lv, R->rp, R->ci, rv, n, cand, cnt, nullptr, nullptr,
+                         nullptr);
+    FX_HIP(hipGetLastError());
+    FX_TRY(scan_u32(st, cnt, n, orp));
+    FX_TRY(read_words(ctx, orp + n, 1, &nnz));
+    FX_TRY(new_from_rowptr(ctx, n, R->mcol, values, orp, nnz, &P));
+    if (P->nnz == 0) {  // R's rows that L selects are all empty
+      *C = P;
+      return 0;
+    }
+    double* ov = values ? P->va : nullptr;
+    hipLaunchKernelGGL((k_mult_lds<8, 0, kMultShort, true>), gs, dim3(kThreads), 0, st, L->rp,
+                       L->ci, lv, R->rp, R->ci, rv, n, cand, nullptr, P->rp, P->ci, ov);
+    if (got[2] > kMultShort)
+      hipLaunchKernelGGL((k_mult_lds<64, kMultShort, kMultMost, true>), gw, dim3(kThreads), 0, st,
+                         L->rp, L->ci, lv, R->rp, R->ci, rv, n, cand, nullptr, P->rp, P->ci, ov);
+    return finish(P, C);
+  }
+  uint32_t* off = S.get<uint32_t>((size_t)n + 1);
+  FX_CHECK(off, FX_ERROR_ALLOC_MEM, "L R: allocation failed");
   FX_TRY(scan_u32(st, cand, n, off));
   uint32_t* keys = S.get<uint32_t>(2 * total);
   uint32_t* slot = S.get<uint32_t>(2 * total);
@@ -451,8 +641,8 @@ int fx_csr_mult(fx_ctx ctx, fx_csr L, fx_csr R, fx_csr* C) {
                      keys, slot, tcol, tval, cnt);
   FX_HIP(hipGetLastError());
   FX_TRY(scan_u32(st, cnt, n, orp));
-  fx_csr P = nullptr;
-  FX_TRY(new_from_rowptr(ctx, n, R->mcol, values, orp, &P));
+  FX_TRY(read_words(ctx, orp + n, 1, &nnz));
+  FX_TRY(new_from_rowptr(ctx, n, R->mcol, values, orp, nnz, &P));
   const uint64_t copy_threads = (uint64_t)n * kCopyLanes;
   hipLaunchKernelGGL(k_mult_copy, dim3((unsigned)((copy_threads + kThreads - 1) / kThreads)),
                      dim3(kThreads), 0, st, off, tcol, tval, n, P->rp, P->ci,
