@@ -26,6 +26,7 @@
 #include <utility>
 
 #include "fx_fast.hpp"
+#include "fx_resident.hpp"
 
 namespace fx {
 
@@ -285,19 +286,37 @@ __device__ __forceinline__ void bi_loop_top(BiState* S, const CgPrm& P, double r
   }
 }
 
+// The quotients and roots of the end-of-iteration logic, formed where they
+// are asked for (one thread taking the decision).
+struct BiQuotients {
+  __device__ __forceinline__ double resAbs(const BiState* S) const { return sqrt(S->rr); }
+  __device__ __forceinline__ double resRel(const BiState* S, double ra) const {
+    return ra / S->denAbs;
+  }
+  __device__ __forceinline__ double ratio(const BiState* S, double ra) const {
+    return ra / S->resAbsOld;
+  }
+  __device__ __forceinline__ double xRelDiff(const BiState* S) const {
+    return fabs(S->alpha) * sqrt(S->pp) / sqrt(S->xx);
+  }
+  __device__ __forceinline__ double rr0(const BiState* S) const { return S->rr0n / S->rr0; }
+};
+
 // End of iteration, src/BiCGStab.cxx:148-206, for the common case; a rare
 // branch hands the step to the host, which recomputes it from the state.
-__device__ __forceinline__ void bi_after_update(BiState* S, const CgPrm& P, double* hist) {
+template <class Q = BiQuotients>
+__device__ __forceinline__ void bi_after_update(BiState* S, const CgPrm& P, double* hist,
+                                                const Q& quot = Q{}) {
   const uint32_t it = S->numIter;
   if (it >= P.minIter) {
-    const double resAbs = sqrt(S->rr);
-    const double resRel = resAbs / S->denAbs;
-    const double ratio = resAbs / S->resAbsOld;
+    const double resAbs = quot.resAbs(S);
+    const double resRel = quot.resRel(S, resAbs);
+    const double ratio = quot.ratio(S, resAbs);
     bool host = false;
     if (it >= P.savIter && resAbs < S->resAbsOld) host = true;
     if (ratio > kChkRatio && it > P.minIter) {
       if (S->xinf < P.solStagTol) host = true;
-      const double xRelDiff = fabs(S->alpha) * sqrt(S->pp) / sqrt(S->xx);
+      const double xRelDiff = quot.xRelDiff(S);
       if (S->stagStep <= kMaxStag && xRelDiff < P.solStagTol) host = true;
     }
     if (resRel < P.relTol) host = true;
@@ -312,14 +331,213 @@ __device__ __forceinline__ void bi_after_update(BiState* S, const CgPrm& P, doub
   }
   if (it < P.maxIter) {
     S->resAbsOld = S->resAbs;
-    const double rr0old = S->rr0;
+    const double q = quot.rr0(S);
     S->rr0 = S->rr0n;
-    S->beta = S->rr0 / rr0old * S->alpha / S->omega;
+    S->beta = q * S->alpha / S->omega;
   } else {
     S->status = ST_DONE;
     return;
   }
   bi_loop_top(S, P, S->rr, hist);
+}
+
+// ---- the resident iteration ---------------------------------------------------
+// The same iteration with x, t, dinv in registers, p, r (s in its place), pt
+// and r0* in LDS, up to max_it of them per launch (fx_resident.hpp).  p and s
+// are exported for the gathers of other workgroups; the three reductions are
+// exchanges.  Per element the arithmetic, and per iteration the decisions,
+// are those of the five kernels; every workgroup takes the decisions for
+// itself from the same sums.  On leaving, x, r, p, pt and the state are where
+// the five kernels would have left them.  Bound by the exchanges' latency:
+// three reductions and two halos; us per iteration, with the five kernels'
+// in parentheses: 1024 unknowns 7.4 (22.3), 256^2 16.1 (24.5), 1024^2 27.6
+// (54.0), 95^3 37.5 (52.8).  Up to four rows per thread: eight rows' vectors
+// do not fit the registers.  The two dot products sum a thread's even and odd
+// rows apart, half the chain.  (At 1024^2 the upwind system's count is set by
+// rounding: 1240 to 1522 over right-hand sides an ulp apart, mean 1379, and
+// 1268 to 1462, mean 1361, with the five kernels.)
+
+// The quotients above formed by the lanes of one wave at once.
+struct BiQuotientsWave {
+  double ra, rel, rat, xrel, q;
+  __device__ __forceinline__ BiQuotientsWave(const BiState* S, const double (&a)[5], int lane) {
+    const double a1 = res_value(a[1]), a3 = res_value(a[3]), a4 = res_value(a[4]);
+    double square = res_value(a[0]);
+    if (lane == 1) square = a3;
+    if (lane == 2) square = a4;
+    const double root = sqrt(square);
+    ra = res_lane(root, 0);
+    double num = ra, den = S->denAbs;
+    if (lane == 1) den = S->resAbsOld;
+    if (lane == 2) {
+      num = fabs(S->alpha) * res_lane(root, 1);
+      den = res_lane(root, 2);
+    }
+    if (lane == 3) {
+      num = a1;
+      den = S->rr0;
+    }
+    const double quo = num / den;
+    rel = res_lane(quo, 0);
+    rat = res_lane(quo, 1);
+    xrel = res_lane(quo, 2);
+    q = res_lane(quo, 3);
+  }
+  __device__ __forceinline__ double resAbs(const BiState*) const { return ra; }
+  __device__ __forceinline__ double resRel(const BiState*, double) const { return rel; }
+  __device__ __forceinline__ double ratio(const BiState*, double) const { return rat; }
+  __device__ __forceinline__ double xRelDiff(const BiState*) const { return xrel; }
+  __device__ __forceinline__ double rr0(const BiState*) const { return q; }
+};
+
+constexpr uint32_t kBiResRows = 4;  // most rows per thread
+
+template <int R, int MM>
+__global__ __launch_bounds__(kResThreads) void k_bi_resident(
+    ResMat A, double* __restrict__ x, double* __restrict__ r, double* p, double* s,
+    double* __restrict__ pt, const double* __restrict__ r0s, const double* __restrict__ dinv,
+    BiState* st, BiState* hout, CgPrm P, double* hist, ResComm cm, uint32_t max_it) {
+  __shared__ double pl[R * kResThreads];
+  __shared__ double sl[R * kResThreads];
+  __shared__ double ql[R * kResThreads];  // pt
+  __shared__ double zl[R * kResThreads];  // r0*
+  __shared__ typename ResRows<double, R, MM>::Lds ml;
+  __shared__ ResShared sh;
+  __shared__ BiState S;
+  __shared__ int run;
+  const uint32_t tid = threadIdx.x, base = blockIdx.x * R * kResThreads, n = A.n;
+  const int lane = tid & 63;
+  const bool others = gridDim.x > 1;
+  ResRows<double, R, MM> rows;
+  uint32_t wlo, whi;
+  if (tid == 0) {
+    S = *st;
+    run = S.status == ST_RUN;
+  }
+  rows.load(A, ml, wlo, whi);
+  if (!run) {  // uniform over the launch
+    if (blockIdx.x == 0 && tid == 0) *hout = S;
+    return;
+  }
+  double xv[R], dv[R], tv[R];  // tv: A p, then t
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const uint32_t i = base + k * kResThreads + tid;
+    const bool has = i < n;
+    xv[k] = has ? x[i] : 0.0;
+    zl[k * kResThreads + tid] = has ? r0s[i] : 0.0;
+    dv[k] = has && dinv ? dinv[i] : 1.0;  // a * 1 = a: the identity
+    tv[k] = 0.0;
+    ql[k * kResThreads + tid] = 0.0;
+    pl[k * kResThreads + tid] = has ? p[i] : 0.0;
+    sl[k * kResThreads + tid] = has ? r[i] : 0.0;
+  }
+  __syncthreads();
+  uint32_t t = 0;  // reductions so far
+  bool ok = true;
+  for (uint32_t it = 0; it < max_it; ++it) {
+    rows.fresh();
+    rows.template product<false>(A, ml, pl, (const double*)p, tv);
+    double a1[1] = {0.0}, b1 = 0.0;  // even and odd rows: half the chain
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      tv[k] = tv[k] * dv[k];
+      ql[k * kResThreads + tid] = tv[k];
+      double& sum = k & 1 ? b1 : a1[0];
+      sum = fma(tv[k], zl[k * kResThreads + tid], sum);
+    }
+    if constexpr (R > 1) a1[0] += b1;
+    ok = res_allreduce<1, 0u>(a1, cm, t++, sh, [&](const double (&tot)[1]) {
+      if (lane != 0) return;
+      S.numIter += 1;
+      S.t12 = tot[0];
+      if (!(fabs(tot[0]) > 1e-40)) {  // src/BiCGStab.cxx:119-124
+        S.err = FX_ERROR_DIVIDE_ZERO;
+        S.status = ST_DONE;
+        run = 0;
+      } else {
+        S.alpha = S.rr0 / tot[0];
+      }
+    });
+    if (!ok || !run) break;
+    const double alpha = S.alpha;
+    const int fs = waxpby_form(1.0, -alpha);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const uint32_t i = base + k * kResThreads + tid;
+      const double sv = waxpby_e(fs, 1.0, sl[k * kResThreads + tid], -alpha, tv[k]);
+      sl[k * kResThreads + tid] = sv;
+      if (others && i < n) res_store(s + i, sv);
+    }
+    ok = res_exchange(cm, 2 * (unsigned long long)it + 1, wlo, whi, sh);
+    if (!ok) break;
+    rows.fresh();
+    rows.template product<false>(A, ml, sl, (const double*)s, tv);
+    double a2[2] = {0.0, 0.0}, b2[2] = {0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      tv[k] = tv[k] * dv[k];
+      double(&sum)[2] = k & 1 ? b2 : a2;
+      sum[0] = fma(tv[k], sl[k * kResThreads + tid], sum[0]);
+      sum[1] = fma(tv[k], tv[k], sum[1]);
+    }
+    if constexpr (R > 1) a2[0] += b2[0], a2[1] += b2[1];
+    ok = res_allreduce<2, 0u>(a2, cm, t++, sh, [&](const double (&tot)[2]) {
+      if (lane == 0) S.omega = tot[0] / tot[1];  // src/BiCGStab.cxx:134 (no guard there)
+    });
+    if (!ok) break;
+    const double omega = S.omega;
+    const BiUpd<double, true> u{alpha, omega, waxpby_form(alpha, omega),
+                                waxpby_form(1.0, -omega)};
+    double a[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const uint32_t l = k * kResThreads + tid;
+      double ri;
+      u.elem(pl[l], sl[l], tv[k], dv[k], zl[l], xv[k], ri, a);
+      sl[l] = ri;
+    }
+    ok = res_allreduce<5, 4u>(a, cm, t++, sh, [&](const double (&tot)[5]) {
+      const BiQuotientsWave quot(&S, tot, lane);
+      if (lane != 0) return;
+      S.rr = tot[0];
+      S.rr0n = tot[1];
+      S.xinf = tot[2];
+      S.pp = tot[3];
+      S.xx = tot[4];
+      bi_after_update(&S, P, blockIdx.x == 0 ? hist : nullptr, quot);
+      run = S.status == ST_RUN;
+    });
+    if (!ok || !run) break;
+    const double beta = S.beta;
+    const int f1 = waxpby_form(1.0, -omega), f2 = waxpby_form(1.0, beta);
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      const uint32_t i = base + k * kResThreads + tid;
+      // tmp = p - omega pt; p = r + beta tmp   (src/BiCGStab.cxx:214-215)
+      const double pv = waxpby_e(f2, 1.0, sl[k * kResThreads + tid], beta,
+                                 waxpby_e(f1, 1.0, pl[k * kResThreads + tid], -omega, ql[k * kResThreads + tid]));
+      pl[k * kResThreads + tid] = pv;
+      if (others && i < n) res_store(p + i, pv);
+    }
+    ok = res_exchange(cm, 2 * (unsigned long long)it + 2, wlo, whi, sh);
+    if (!ok) break;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int k = 0; k < R; ++k) {
+    const uint32_t i = base + k * kResThreads + tid;
+    if (i < n) {
+      x[i] = xv[k];
+      r[i] = sl[k * kResThreads + tid];
+      pt[i] = ql[k * kResThreads + tid];
+      if (!others) p[i] = pl[k * kResThreads + tid];
+    }
+  }
+  if (blockIdx.x == 0 && tid == 0) {
+    *st = S;
+    *hout = S;
+  }
 }
 
 template <class VT>
@@ -624,6 +842,42 @@ struct BiRun {
     return 0;
   }
 
+  // One launch of the resident loop and the state it left; *held = false when
+  // the device cannot hold it.  A wait that gave up is an error of the device.
+  int run_resident(bool* held, BiState* out) {
+    *held = false;
+    if constexpr (std::is_same_v<VT, double>) {
+      const ResShape rs = res_shape(W.n, W.ctx->sms);
+      const void* k = nullptr;
+      if (rs.rows && rs.rows <= kBiResRows)
+        k = res_pick(rs.rows, res_mode<double>(A, rs.rows), [](auto r, auto m) -> const void* {
+          if constexpr (decltype(r)::value <= (int)kBiResRows)
+            return (const void*)&k_bi_resident<decltype(r)::value, decltype(m)::value>;
+          else
+            return nullptr;
+        });
+      if (!k) return 0;
+      ResMat M = res_mat<double>(A);
+      ResComm cm = res_comm(W.comm);
+      double *x = vx(), *r = vr(), *p = vp(), *s = vs(), *pt = vpt();
+      const double *r0s = vr0s(), *d = dinv;
+      BiState *ds = dstate(0), *hs = hslot(0);
+      uint32_t most = kResLaunchIters;
+      void* args[] = {&M, &x, &r, &p, &s, &pt, &r0s, &d, &ds, &hs, &P, &W.hist, &cm, &most};
+      const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args);
+      if (rc < 0) return rc;
+      *held = rc == 0;
+      if (*held) {
+        unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
+        FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
+        FX_HIP(hipStreamSynchronize(st));
+        FX_CHECK(*fail == 0, FX_ERROR_DEVICE, "a wait of the resident BiCGStab loop gave up");
+        *out = *hslot(0);
+      }
+    }
+    return 0;
+  }
+
   int run(const VT* b, VT* x_user, fx_result* res, const fx_params& PP, int pc_dtype) {
     const uint32_t n = W.n;
     FX_HIP(hipMemcpyAsync(vx(), x_user, sizeof(VT) * n, hipMemcpyDeviceToDevice, st));
@@ -659,8 +913,29 @@ struct BiRun {
     // as for CG: a stretch of replays stops within maxIter / kChunk of them,
     // and there are at most maxIter host steps
     const uint64_t max_chunks = (uint64_t)PP.maxIter / kChunk + 4;
-    uint64_t host_steps = 0;
+    uint64_t host_steps = 0, launches = 0;
+    bool resident = W.resident;
     for (;;) {
+      if (resident) {
+        bool held = true;
+        FX_TRY(run_resident(&held, &s));
+        if (!held) {  // the launch does not fit this device: kernel by kernel
+          W.resident = resident = false;
+          continue;
+        }
+        if (s.status == ST_RUN) {  // a full launch: its iterations are done
+          FX_CHECK(++launches <= (uint64_t)PP.maxIter / kResLaunchIters + 4 + host_steps,
+                   FX_ERROR_DEVICE, "resident BiCGStab loop did not stop");
+          continue;
+        }
+        FX_CHECK(++host_steps <= (uint64_t)PP.maxIter + 2, FX_ERROR_DEVICE,
+                 "BiCGStab device loop did not stop");
+        if (s.status == ST_DONE ||
+            host_step(s, vb_, vx_, vr_, vp_, vpt_, vr0s_, vtmp, vsafe, o, PP))
+          break;
+        FX_TRY(write_state(s));
+        continue;
+      }
       ReplayPace pace;
       pace.hint = host_steps == 0 ? W.last_iters : 0;
       // the iteration that ends the loop is numbered numIter - 1: a

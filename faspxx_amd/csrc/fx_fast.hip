@@ -1985,7 +1985,8 @@ int fast_solve(fx_solver S, fx_vec b, fx_vec x, fx_result* res) {
   }
   FastWs& W = *S->fast;
   // resident loops: a banded matrix of short rows that fits the chip
-  if (!W.comm && !S->op && S->type == FX_SOLVER_CG && !resident_disabled() &&
+  if (!W.comm && !S->op && (S->type == FX_SOLVER_CG || S->type == FX_SOLVER_BICGSTAB) &&
+      !resident_disabled() &&
       !(S->pc->kind == 1 && S->pc->iters > 1) && res_matrix_ok(S->A) &&
       res_shape(n, S->ctx->sms).rows) {
     FX_HIP(hipMalloc(&W.comm, kResCommWords * sizeof(unsigned long long)));

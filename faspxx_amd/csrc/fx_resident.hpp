@@ -335,6 +335,22 @@ struct ResRows {
   __device__ __forceinline__ uint32_t len(int q) const { return (len4[q / 4] >> (8 * (q % 4))) & 255u; }
   __device__ __forceinline__ uint32_t pid(int q) const { return (pid4[q / 4] >> (8 * (q % 4))) & 255u; }
 
+  // The places of the entries as values of this moment: addresses formed from
+  // them are not kept from one product to the next (two products per
+  // iteration kept more of them than there are registers).
+  __device__ __forceinline__ void fresh() {
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      if constexpr (MM == RM_REG) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) asm volatile("" : "+v"(at[q][j]));
+      }
+      if constexpr (MM == RM_MEM) asm volatile("" : "+v"(start[q]));
+    }
+#pragma unroll
+    for (int w = 0; w < kPack; ++w) asm volatile("" : "+v"(len4[w]), "+v"(pid4[w]));
+  }
+
   // lo .. hi: the workgroups whose rows this one's rows gather from.
   __device__ __forceinline__ void load(const ResMat& A, Lds& l, uint32_t& lo, uint32_t& hi) {
     const uint32_t tid = threadIdx.x, base = blockIdx.x * kRows;
