@@ -456,8 +456,12 @@ struct CgQuotientsWave {
 template <int R, int MM>
 __global__ __launch_bounds__(kResThreads) void k_cg_resident(
     ResMat A, double* __restrict__ x, double* __restrict__ r, double* p, double* __restrict__ q,
-    const double* __restrict__ dinv, CgState* st, CgState* hout, CgPrm P, double* hist,
+    double* zx, const double* __restrict__ dinv, CgState* st, CgState* hout, CgPrm P, double* hist,
     ResComm cm, uint32_t max_it) {
+  // One exchange less per iteration: z is exported before the second
+  // reduction, which then announces it, and each thread keeps the p it gathers
+  // from other workgroups (at most 8 of them) up to date for itself.
+  constexpr bool kOwn = MM == RM_REG && R == 1;
   constexpr bool kRl = R == 8;  // r in LDS too: eight rows' vectors do not fit the registers
   __shared__ double pl[R * kResThreads];
   __shared__ double rl[kRl ? R * kResThreads : 1];
@@ -493,11 +497,23 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
     qv[k] = 0.0;
     pl[k * kResThreads + tid] = has ? p[i] : 0.0;
   }
+  double po[kOwn ? 8 * R : 1];  // p at the entries outside the workgroup's rows
+  const bool others = gridDim.x > 1;
+  if constexpr (kOwn) {
+#pragma unroll
+    for (int e = 0; e < 8 * R; ++e) po[e] = 0.0;
+    rows.outside([&](int e, uint32_t c) { po[e] = p[c]; });
+  }
   __syncthreads();
   uint32_t t = 0;  // reductions so far
   bool ok = true;
   for (uint32_t it = 0; it < max_it; ++it) {
-    rows.template product<false>(A, ml, pl, (const double*)p, qv);
+    if constexpr (kOwn) {
+      rows.fresh();
+      rows.product_of(pl, po, qv);
+    } else {
+      rows.template product<false>(A, ml, pl, (const double*)p, qv);
+    }
     double pq[1] = {0.0};
 #pragma unroll
     for (int k = 0; k < R; ++k) pq[0] = fma(qv[k], pl[k * kResThreads + tid], pq[0]);
@@ -521,8 +537,10 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
       double rk = rr(k);
       u.elem(pl[k * kResThreads + tid], qv[k], xv[k], rk, dv[k], a);
       rr(k) = rk;
+      const uint32_t i = base + k * kResThreads + tid;
+      if (kOwn && others && i < n) res_store(zx + i, rk * dv[k]);
     }
-    ok = res_allreduce<5, 4u>(a, cm, t++, sh, [&](const double (&tot)[5]) {
+    ok = res_allreduce<5, 4u, kOwn>(a, cm, t++, sh, [&](const double (&tot)[5]) {
       const CgQuotientsWave quot(&S, tot, lane);
       if (lane != 0) return;
       cg_after_update(&S, P, tot, blockIdx.x == 0 ? hist : nullptr, quot);
@@ -535,10 +553,20 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
       const uint32_t i = base + k * kResThreads + tid;
       const double pv = fma(beta, pl[k * kResThreads + tid], rr(k) * dv[k]);
       pl[k * kResThreads + tid] = pv;
-      if (i < n) res_store(p + i, pv);
+      if (!kOwn && i < n) res_store(p + i, pv);
     }
-    ok = res_exchange(cm, it + 1, wlo, whi, sh);
-    if (!ok) break;
+    if constexpr (kOwn) {
+      double zo[8 * R];  // all asked for before the first is used
+#pragma unroll
+      for (int e = 0; e < 8 * R; ++e) zo[e] = 0.0;
+      rows.outside([&](int e, uint32_t c) { zo[e] = res_load(zx + c); });
+#pragma unroll
+      for (int e = 0; e < 8 * R; ++e) po[e] = fma(beta, po[e], zo[e]);
+      __syncthreads();
+    } else {
+      ok = res_exchange(cm, it + 1, wlo, whi, sh);
+      if (!ok) break;
+    }
   }
   __syncthreads();
 #pragma unroll
@@ -548,6 +576,7 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
       x[i] = xv[k];
       r[i] = rr(k);
       q[i] = qv[k];
+      if (kOwn) p[i] = pl[k * kResThreads + tid];
     }
   }
   if (blockIdx.x == 0 && tid == 0) {
@@ -1598,10 +1627,11 @@ struct CgRun {
       ResMat M = res_mat<double>(A);
       ResComm cm = res_comm(W.comm);
       double *x = (double*)W.x, *r = (double*)W.r, *p = (double*)W.p, *q = (double*)W.q;
+      double* z = (double*)W.x2;
       const double* d = dinv;
       CgState *ds = dstate(), *hs = hslot(0);
       uint32_t most = kResLaunchIters;
-      void* args[] = {&M, &x, &r, &p, &q, &d, &ds, &hs, &P, &W.hist, &cm, &most};
+      void* args[] = {&M, &x, &r, &p, &q, &z, &d, &ds, &hs, &P, &W.hist, &cm, &most};
       const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args);
       if (rc < 0) return rc;
       *held = rc == 0;

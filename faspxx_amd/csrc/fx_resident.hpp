@@ -157,7 +157,9 @@ struct ResShared {
 // groups of 32, the group's first workgroup publishing its sum (one more
 // hop, but 256 workgroups polling 256 lines took longer).  False when a wait
 // gave up.
-template <int K, unsigned MaxMask, class Post>
+// DRAIN: what this workgroup exported before the call is visible to every
+// workgroup that has left it.
+template <int K, unsigned MaxMask, bool DRAIN = false, class Post>
 __device__ __forceinline__ bool res_allreduce(double (&v)[K], const ResComm& cm, uint32_t t,
                                               ResShared& sh, const Post& post) {
   static_assert(K <= kResSlot, "one line per slot");
@@ -167,6 +169,7 @@ __device__ __forceinline__ bool res_allreduce(double (&v)[K], const ResComm& cm,
     const double s = res_wave<((MaxMask >> k) & 1u) != 0>(v[k]);
     if (lane == 0) sh.red[k][wid] = s;
   });
+  if constexpr (DRAIN) res_drain();
   __syncthreads();
   if (wid == 0) {
     double tot[K];
@@ -417,6 +420,42 @@ struct ResRows {
     __syncthreads();
     lo = min(l.lo, base) / kRows;
     hi = max(l.hi, base) / kRows;
+  }
+
+  // RM_REG: f(place, column) for each of the thread's entries outside the
+  // workgroup's rows.
+  template <class F>
+  __device__ __forceinline__ void outside(const F& f) const {
+    static_assert(MM == RM_REG, "places are in registers");
+#pragma unroll
+    for (int q = 0; q < R; ++q)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (at[q][j] < 0) f(8 * q + j, (uint32_t)~at[q][j]);
+  }
+
+  // RM_REG: the product below with the outside entries given in vo.
+  template <class VT>
+  __device__ __forceinline__ void product_of(const VT* vl, const VT (&vo)[8 * R],
+                                             double (&out)[R]) const {
+    static_assert(MM == RM_REG, "places are in registers");
+#pragma unroll
+    for (int q = 0; q < R; ++q) {
+      const uint32_t n = len(q);
+      VT x[8];
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int32_t d = at[q][j];
+        const VT in = vl[d < 0 ? 0 : d];
+        x[j] = d < 0 ? vo[8 * q + j] : in;
+      }
+      double t = 0.0;
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if ((uint32_t)j < n)
+          t = j == 0 ? (double)a[q][j] * (double)x[j] : fma((double)a[q][j], (double)x[j], t);
+      out[q] = t;
+    }
   }
 
   // (A v)_i of the thread's q-th row, left to right as in the SpMV kernels
