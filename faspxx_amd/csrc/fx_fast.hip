@@ -510,7 +510,10 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
   for (uint32_t it = 0; it < max_it; ++it) {
     if constexpr (kOwn) {
       rows.fresh();
-      rows.product_of(pl, po, qv);
+      if (others)
+        rows.product_of(pl, po, qv);
+      else
+        rows.product_within(pl, qv);
     } else {
       rows.template product<false>(A, ml, pl, (const double*)p, qv);
     }

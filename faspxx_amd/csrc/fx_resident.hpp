@@ -434,21 +434,17 @@ struct ResRows {
         if (at[q][j] < 0) f(8 * q + j, (uint32_t)~at[q][j]);
   }
 
-  // RM_REG: the product below with the outside entries given in vo.
-  template <class VT>
-  __device__ __forceinline__ void product_of(const VT* vl, const VT (&vo)[8 * R],
-                                             double (&out)[R]) const {
+  // RM_REG: the product below with the outside entries given in vo, or with
+  // none (one workgroup).
+  template <class VT, class At>
+  __device__ __forceinline__ void product_at(double (&out)[R], const At& entry) const {
     static_assert(MM == RM_REG, "places are in registers");
 #pragma unroll
     for (int q = 0; q < R; ++q) {
       const uint32_t n = len(q);
       VT x[8];
 #pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        const int32_t d = at[q][j];
-        const VT in = vl[d < 0 ? 0 : d];
-        x[j] = d < 0 ? vo[8 * q + j] : in;
-      }
+      for (int j = 0; j < 8; ++j) x[j] = entry(8 * q + j, at[q][j]);
       double t = 0.0;
 #pragma unroll
       for (int j = 0; j < 8; ++j)
@@ -456,6 +452,18 @@ struct ResRows {
           t = j == 0 ? (double)a[q][j] * (double)x[j] : fma((double)a[q][j], (double)x[j], t);
       out[q] = t;
     }
+  }
+  template <class VT>
+  __device__ __forceinline__ void product_of(const VT* vl, const VT (&vo)[8 * R],
+                                             double (&out)[R]) const {
+    product_at<VT>(out, [&](int e, int32_t d) {
+      const VT in = vl[d < 0 ? 0 : d];
+      return d < 0 ? vo[e] : in;
+    });
+  }
+  template <class VT>
+  __device__ __forceinline__ void product_within(const VT* vl, double (&out)[R]) const {
+    product_at<VT>(out, [&](int, int32_t d) { return vl[d]; });
   }
 
   // (A v)_i of the thread's q-th row, left to right as in the SpMV kernels
