@@ -1,6 +1,8 @@
 // fx_bicgstab.hip -- fused, graph-replayed BiCGStab (src/BiCGStab.cxx:68-270)
 // with the identity or a one-sweep Jacobi preconditioner on the system
-// matrix.
+// matrix.  Banded systems of up to 1048576 rows run their loop in one
+// cooperative launch (see "the resident iteration" below), others kernel by
+// kernel.
 //
 // The reference's recurrence is the preconditioned P.A form: the residual is
 // updated with P A p and P A s, the solution with P p and P s (:114-146).  One

@@ -14,6 +14,8 @@
 // a single-reduction form: 2 kernels and 11 vector passes per iteration
 // (see "the scaled inner solver of the refinement" below).
 //
+// Banded systems that fit the chip run the CG loop and the refinement's inner
+// loop in one cooperative launch (see "the resident iteration" below).  Else a
 // CG iteration = 3 kernels (see "the three-kernel iteration" below), replayed
 // as a hipGraph of kChunk iterations; the last iteration of a replay copies
 // the state to a pinned host slot.  Per iteration HBM traffic: the SpMV's
@@ -460,7 +462,8 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
     ResComm cm, uint32_t max_it) {
   // One exchange less per iteration: z is exported before the second
   // reduction, which then announces it, and each thread keeps the p it gathers
-  // from other workgroups (at most 8 of them) up to date for itself.
+  // from other workgroups (at most 8 of them) up to date for itself: 11.1 ->
+  // 9.0 us per iteration at 512^2.  Two rows' copies do not fit the registers.
   constexpr bool kOwn = MM == RM_REG && R == 1;
   constexpr bool kRl = R == 8;  // r in LDS too: eight rows' vectors do not fit the registers
   __shared__ double pl[R * kResThreads];
