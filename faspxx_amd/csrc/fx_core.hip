@@ -317,6 +317,7 @@ int reduce_host(fx_ctx ctx, int kind, int upd, double a, fx_vec x, fx_vec y, fx_
   if (bits == kRedPending) {
     FX_HIP(hipStreamSynchronize(ctx->stream));
     bits = __atomic_load_n(slot, __ATOMIC_ACQUIRE);
+    FX_CHECK(bits != kRedPending, FX_ERROR_DEVICE, "a reduction left no result");
   }
   std::memcpy(out, &bits, sizeof(double));
   return 0;
@@ -347,6 +348,7 @@ int read_words(fx_ctx ctx, const uint32_t* dev, int n, uint32_t* out) {
     if (v == pending) {
       FX_HIP(hipStreamSynchronize(ctx->stream));
       v = __atomic_load_n(slots + i, __ATOMIC_ACQUIRE);
+      FX_CHECK(v != pending, FX_ERROR_DEVICE, "a word from the device did not arrive");
     }
     out[i] = (uint32_t)v;
   }
