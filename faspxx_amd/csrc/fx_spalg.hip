@@ -156,7 +156,9 @@ __global__ void k_shift_diag(const uint32_t* __restrict__ dp, double* __restrict
 
 // ---- L R ------------------------------------------------------------------
 // Candidate products of row i: the summed lengths of the rows of R that row
-// i of L selects.  Per workgroup their sum (two words) and the largest.
+// i of L selects.  Per workgroup their sum (two words) and the largest.  A
+// row's own count stops at 2^32 - 1 (repeated entries of L can pass it); the
+// sum does not, and is refused from 2^31 on.
 __global__ __launch_bounds__(kThreads) void k_mult_count(
     const uint32_t* __restrict__ lrp, const uint32_t* __restrict__ lci,
     const uint32_t* __restrict__ rrp, uint32_t nrow, uint32_t* __restrict__ cand,
@@ -166,16 +168,17 @@ __global__ __launch_bounds__(kThreads) void k_mult_count(
   if (threadIdx.x == 0) total = 0, top = 0;
   __syncthreads();
   const uint32_t i = blockIdx.x * kThreads + threadIdx.x;
-  uint32_t c = 0;
+  unsigned long long c = 0;
   if (i < nrow) {
     for (uint32_t k = lrp[i]; k < lrp[i + 1]; ++k) {
       const uint32_t r = lci[k];
       c += rrp[r + 1] - rrp[r];
     }
-    cand[i] = c;
   }
-  atomicAdd(&total, (unsigned long long)c);
-  atomicMax(&top, c);
+  const uint32_t own = (uint32_t)(c < 0xffffffffull ? c : 0xffffffffull);
+  if (i < nrow) cand[i] = own;
+  atomicAdd(&total, c);
+  atomicMax(&top, own);
   __syncthreads();
   if (threadIdx.x == 0) sums[blockIdx.x] = total, most[blockIdx.x] = top;
 }

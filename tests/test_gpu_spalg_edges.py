@@ -54,6 +54,18 @@ def test_mult_without_entries(ctx, oracle):
     assert C.nnz == 0
 
 
+@pytest.mark.parametrize("k", [32768, 65537])
+def test_mult_refuses_too_many_candidates(ctx, k):
+    """One row of L that selects one row of 65536 entries k times: 2^31
+    candidates, and more than a 32-bit count holds."""
+    m = 65536
+    L = fx.Csr(ctx, 1, 1, np.array([0, k]), np.zeros(k, np.uint32), np.ones(k))
+    R = fx.Csr(ctx, 1, m, np.array([0, m]), np.arange(m), np.ones(m))
+    with pytest.raises(fx.FxError) as e:
+        fx.Csr.mult(L, R)
+    assert e.value.code == -20  # ERROR_ALLOC_MEM
+
+
 LENGTHS = {
     "short": lambda n, rng: rng.integers(0, 9, n),
     "empty but one": lambda n, rng: np.where(np.arange(n) == n // 2, 5, 0),
