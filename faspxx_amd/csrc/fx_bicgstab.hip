@@ -844,10 +844,9 @@ struct BiRun {
     return 0;
   }
 
-  // One launch of the resident loop and the state it left; *held = false when
-  // the device cannot hold it.  A wait that gave up is an error of the device.
-  int run_resident(bool* held, BiState* out) {
-    *held = false;
+  // One launch of the resident loop and the state it left.
+  int run_resident(uint64_t before, ResOutcome* how, BiState* out) {
+    *how = RES_REFUSED;
     if constexpr (std::is_same_v<VT, double>) {
       const ResShape rs = res_shape(W.n, W.ctx->sms);
       const void* k = nullptr;
@@ -866,16 +865,13 @@ struct BiRun {
       BiState *ds = dstate(0), *hs = hslot(0);
       uint32_t most = kResLaunchIters;
       void* args[] = {&M, &x, &r, &p, &s, &pt, &r0s, &d, &ds, &hs, &P, &W.hist, &cm, &most};
-      const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args);
-      if (rc < 0) return rc;
-      *held = rc == 0;
-      if (*held) {
-        unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
-        FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
-        FX_HIP(hipStreamSynchronize(st));
-        FX_CHECK(*fail == 0, FX_ERROR_DEVICE, "a wait of the resident BiCGStab loop gave up");
-        *out = *hslot(0);
-      }
+      const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args, before);
+      if (rc) return rc < 0 ? rc : 0;
+      unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
+      FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
+      FX_HIP(hipStreamSynchronize(st));
+      *out = *hslot(0);
+      *how = res_outcome(out->status == ST_RUN, *fail);
     }
     return 0;
   }
@@ -919,14 +915,19 @@ struct BiRun {
     bool resident = W.resident;
     for (;;) {
       if (resident) {
-        bool held = true;
-        FX_TRY(run_resident(&held, &s));
-        if (!held) {  // the launch does not fit this device: kernel by kernel
+        ResOutcome how;
+        FX_TRY(run_resident(launches, &how, &s));
+        ++launches;
+        if (how == RES_REFUSED) {  // on from here kernel by kernel
           W.resident = resident = false;
           continue;
         }
+        if (how == RES_LOST) {  // b and the caller's x are untouched
+          W.resident = false;
+          return run(b, x_user, res, PP, pc_dtype);
+        }
         if (s.status == ST_RUN) {  // a full launch: its iterations are done
-          FX_CHECK(++launches <= (uint64_t)PP.maxIter / kResLaunchIters + 4 + host_steps,
+          FX_CHECK(launches <= (uint64_t)PP.maxIter / kResLaunchIters + 4 + 2 * host_steps,
                    FX_ERROR_DEVICE, "resident BiCGStab loop did not stop");
           continue;
         }
@@ -958,6 +959,7 @@ struct BiRun {
       if (host_step(s, vb_, vx_, vr_, vp_, vpt_, vr0s_, vtmp, vsafe, o, PP)) break;
       FX_TRY(write_state(s));
     }
+    S->last_resident = resident;
     res->numIter = s.numIter;
     W.last_iters = host_steps == 1 ? s.numIter : 0;  // a prediction only for plain runs
     if (!(s.numIter == PP.minIter && s.numIter == PP.maxIter)) {

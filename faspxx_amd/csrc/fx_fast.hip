@@ -1618,18 +1618,15 @@ struct CgRun {
     return 0;
   }
 
-  // One launch of the resident loop (f64) and the state it left; *held =
-  // false when the device cannot hold it.  A wait that gave up is an error of the device.
-  int run_resident(bool* held, CgState* out) {
+  // One launch of the resident loop (f64) and the state it left.
+  int run_resident(uint64_t before, ResOutcome* how, CgState* out) {
+    *how = RES_REFUSED;
     if constexpr (std::is_same_v<VT, double>) {
       const ResShape rs = res_shape(W.n, W.ctx->sms);
       const void* k = res_pick(rs.rows, res_mode<double>(A, rs.rows), [](auto r, auto m) {
         return (const void*)&k_cg_resident<decltype(r)::value, decltype(m)::value>;
       });
-      if (!k) {
-        *held = false;
-        return 0;
-      }
+      if (!k) return 0;
       ResMat M = res_mat<double>(A);
       ResComm cm = res_comm(W.comm);
       double *x = (double*)W.x, *r = (double*)W.r, *p = (double*)W.p, *q = (double*)W.q;
@@ -1638,16 +1635,13 @@ struct CgRun {
       CgState *ds = dstate(), *hs = hslot(0);
       uint32_t most = kResLaunchIters;
       void* args[] = {&M, &x, &r, &p, &q, &z, &d, &ds, &hs, &P, &W.hist, &cm, &most};
-      const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args);
-      if (rc < 0) return rc;
-      *held = rc == 0;
-      if (*held) {
-        unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
-        FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
-        FX_HIP(hipStreamSynchronize(st));
-        FX_CHECK(*fail == 0, FX_ERROR_DEVICE, "a wait of the resident CG loop gave up");
-        *out = *hslot(0);
-      }
+      const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args, before);
+      if (rc) return rc < 0 ? rc : 0;
+      unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
+      FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
+      FX_HIP(hipStreamSynchronize(st));
+      *out = *hslot(0);
+      *how = res_outcome(out->status == ST_RUN, *fail);
     }
     return 0;
   }
@@ -1719,14 +1713,19 @@ struct CgRun {
     bool resident = W.resident;
     for (;;) {
       if (resident) {
-        bool held = true;
-        FX_TRY(run_resident(&held, &s));
-        if (!held) {  // the launch does not fit this device: kernel by kernel
+        ResOutcome how;
+        FX_TRY(run_resident(launches, &how, &s));
+        ++launches;
+        if (how == RES_REFUSED) {  // on from here kernel by kernel
           W.resident = resident = false;
           continue;
         }
+        if (how == RES_LOST) {  // b and the caller's x are untouched
+          W.resident = false;
+          return run(b, x_user, res, PP, pc_dtype);
+        }
         if (s.status == ST_RUN) {  // a full launch: its iterations are done
-          FX_CHECK(++launches <= (uint64_t)PP.maxIter / kResLaunchIters + 4 + host_steps,
+          FX_CHECK(launches <= (uint64_t)PP.maxIter / kResLaunchIters + 4 + 2 * host_steps,
                    FX_ERROR_DEVICE, "resident CG loop did not stop");
           continue;
         }
@@ -1758,6 +1757,7 @@ struct CgRun {
       if (fin) break;
       FX_TRY(write_state(s));
     }
+    S->last_resident = resident;
     res->numIter = s.numIter;
     W.last_iters = host_steps == 1 ? s.numIter : 0;  // a prediction only for plain runs
     if (!(s.numIter == PP.minIter && s.numIter == PP.maxIter)) {
@@ -1903,9 +1903,9 @@ struct IrInner {
 
   // The resident loop, a launch of kResLaunchIters iterations at a time; the
   // work behind is queued behind the first launch, to act if that one ends
-  // the loop.  *held = false when the device cannot hold it.
+  // the loop.
   int run_resident(uint32_t maxIter, IrState& out, const std::function<int()>& behind,
-                   bool* behind_ran, bool* held) {
+                   bool* behind_ran, ResOutcome* how) {
     const ResShape rs = res_shape(W.n, W.ctx->sms);
     const void* k = res_pick(rs.rows, res_mode<float>(As, rs.rows), [](auto r, auto m) {
       return (const void*)&k_ir_resident<decltype(r)::value, decltype(m)::value>;
@@ -1920,18 +1920,20 @@ struct IrInner {
     const uint64_t max_launches = (uint64_t)maxIter / kResLaunchIters + 4;
     for (uint64_t l = 0;; ++l) {
       FX_CHECK(l <= max_launches, FX_ERROR_DEVICE, "resident IR inner loop did not stop");
-      const int rc = k ? res_launch(W.ctx, k, rs.wgs, W.comm, args) : 1;
+      const int rc = k ? res_launch(W.ctx, k, rs.wgs, W.comm, args, l) : 1;
       if (rc < 0) return rc;
-      FX_CHECK(rc == 0 || l == 0, FX_ERROR_DEVICE, "resident IR inner loop: no launch");
-      *held = rc == 0;
-      if (!*held) return 0;
+      if (rc) {  // the loop in kernels keeps p and y otherwise: not from the middle of this one
+        *how = l == 0 ? RES_REFUSED : RES_LOST;
+        return 0;
+      }
       unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
       FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
       FX_HIP(hipEventRecord(W.ev[0], st));
       if (l == 0 && behind) FX_TRY(behind());
       FX_HIP(hipEventSynchronize(W.ev[0]));
-      FX_CHECK(*fail == 0, FX_ERROR_DEVICE, "a wait of the resident IR inner loop gave up");
       out = *hs;
+      *how = res_outcome(out.status == ST_RUN, *fail);
+      if (*how == RES_LOST) return 0;
       if (out.status != ST_RUN) {
         if (behind_ran) *behind_ran = l == 0 && (bool)behind;
         return 0;
@@ -1946,14 +1948,17 @@ struct IrInner {
   // Iteration hint launches the step that finds the loop stopped, so the
   // loop is predicted to launch hint + 1; the replay predicted to end it is
   // cut to that count (rounded up to even).
-  // behind / behind_ran: see replay_loop.
-  int run(uint32_t maxIter, IrState& out, uint32_t hint,
-          const std::function<int()>& behind = nullptr, bool* behind_ran = nullptr) {
+  // behind / behind_ran: see replay_loop.  again: forms r and the starting
+  // state once more, for a resident loop that was lost on the way (the work
+  // behind it found the loop running and did nothing).
+  int run(uint32_t maxIter, IrState& out, uint32_t hint, const std::function<int()>& behind,
+          bool* behind_ran, const std::function<int()>& again) {
     if (W.resident) {
-      bool held = true;
-      FX_TRY(run_resident(maxIter, out, behind, behind_ran, &held));
-      if (held) return 0;
-      W.resident = false;  // the launch does not fit this device: kernel by kernel
+      ResOutcome how;
+      FX_TRY(run_resident(maxIter, out, behind, behind_ran, &how));
+      if (how == RES_RAN) return 0;
+      W.resident = false;  // kernel by kernel
+      if (how == RES_LOST) FX_TRY(again());
     }
     ReplayPace pace;
     pace.hint = hint;
@@ -2077,6 +2082,7 @@ struct fx_ir_s {
   float* vs32o = nullptr;  // vs32 in a sorted matrix's row order
   std::vector<uint32_t> inner_counts;  // each outer step's inner iterations, last solve
   uint32_t outer_last = 0;             // outer steps of the last solve (0: none)
+  bool last_resident = false;          // its inner loops ran resident
   IrOuterRec* hrec = nullptr;          // pinned
   double* sco = nullptr;  // sorted matrices: S and b in the stored row order
   double* bo = nullptr;
@@ -2365,7 +2371,7 @@ int fx_ir_solve(fx_ir ir, fx_vec b, fx_vec x, fx_result* result, uint32_t* inner
         bool behind_ran = false;
         rc = in.run(ir->inner.maxIter, fs, hint,
                     [&]() { return outer_step(true, (const IrState*)ir->W->state); },
-                    &behind_ran);
+                    &behind_ran, [&]() { return outer_step(false, nullptr); });
         if (rc) break;
         if (fs.reason == IR_OUTER) {  // queued ahead, but the outer loop was done
           --outer_it;
@@ -2419,6 +2425,7 @@ int fx_ir_solve(fx_ir ir, fx_vec b, fx_vec x, fx_result* result, uint32_t* inner
   }
   (void)hipEventRecord(e1, st);
   (void)hipEventSynchronize(e1);
+  ir->last_resident = ir->scaled && ir->W->resident;
   if (ir->scaled) {
     // the last residual's record (the host did not wait for every one)
     if (ir->hrec) resAbs = ir->hrec->resAbs;
@@ -2435,6 +2442,13 @@ int fx_ir_solve(fx_ir ir, fx_vec b, fx_vec x, fx_result* result, uint32_t* inner
   result->retcode = rc ? rc : err;
   if (inner_iters) *inner_iters = inner_total;
   return result->retcode;
+}
+
+int fx_ir_last_resident(fx_ir ir, int* resident) {
+  clear_error();
+  FX_CHECK(ir && resident, FX_ERROR_INPUT_PAR, "null argument");
+  *resident = ir->last_resident;
+  return 0;
 }
 
 int fx_ir_destroy(fx_ir ir) {

@@ -16,8 +16,14 @@
 // them; a reader looks at the data only after it has seen that.
 //
 // The launch is cooperative: every workgroup is on the chip, so each wait
-// ends.  Waits are bounded all the same; one that runs out raises *fail,
-// every workgroup leaves, and the host runs the solve kernel by kernel.
+// ends.  Waits are bounded all the same; one that runs out raises *fail and
+// every workgroup leaves.  The host then starts over kernel by kernel, from
+// the caller's x (the refinement: from its last outer iterate).  A launch that
+// is refused goes on kernel by kernel from where the last one ended.
+//
+// Environment, for tests: FASPXX_FX_NORESIDENT=1 none of this;
+// FASPXX_FX_RESIDENT_SPINS=N polls before a wait gives up;
+// FASPXX_FX_RESIDENT_LAUNCHES=N launches of one loop before they are refused.
 #pragma once
 
 #include <cstdlib>
@@ -34,21 +40,23 @@ constexpr int kResBufs = 8;           // slot buffers in rotation
 constexpr int kResSlot = 8;           // doubles per slot: one 64-byte line
 constexpr uint32_t kResRowMax = 32;   // longest row the gathers take
 constexpr unsigned long long kResEmpty = ~0ull;  // a NaN that is never published
-constexpr int kResSpinMax = 1 << 21;  // polls before a wait gives up (seconds)
+constexpr int kResSpins = 1 << 21;    // polls before a wait gives up (seconds)
 
 struct ResComm {
   unsigned long long* slots;  // [kResBufs][kResMaxWgs][kResSlot]
   unsigned long long* gsum;   // [kResBufs][8][kResSlot]
   unsigned long long* flags;  // [kResMaxWgs]: iterations whose export is visible
   unsigned long long* fail;
+  int spins;  // polls before a wait gives up
 };
 constexpr size_t kResSlotWords = (size_t)kResBufs * kResMaxWgs * kResSlot;
 constexpr size_t kResGsumWords = (size_t)kResBufs * 8 * kResSlot;
 constexpr size_t kResCommWords = kResSlotWords + kResGsumWords + kResMaxWgs + 8;
 inline ResComm res_comm(void* mem) {
   unsigned long long* w = (unsigned long long*)mem;
+  const char* e = std::getenv("FASPXX_FX_RESIDENT_SPINS");
   return {w, w + kResSlotWords, w + kResSlotWords + kResGsumWords,
-          w + kResSlotWords + kResGsumWords + kResMaxWgs};
+          w + kResSlotWords + kResGsumWords + kResMaxWgs, e ? std::atoi(e) : kResSpins};
 }
 
 // Empty slots and zero flags, before each launch.
@@ -201,7 +209,7 @@ __device__ __forceinline__ bool res_allreduce(double (&v)[K], const ResComm& cm,
         for (int spin = 0;; ++spin) {
           if (active) x = res_load(p);
           if (__all(!active || x != kResEmpty)) break;
-          if (spin > kResSpinMax || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
+          if (spin > cm.spins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
             ok = false;
             break;
           }
@@ -223,7 +231,7 @@ __device__ __forceinline__ bool res_allreduce(double (&v)[K], const ResComm& cm,
           });
           res_for<I>([&](auto i) { have = have && (!act[i] || x[i] != kResEmpty); });
           if (__all(have)) break;
-          if (spin > kResSpinMax || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
+          if (spin > cm.spins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
             ok = false;
             break;
           }
@@ -289,7 +297,7 @@ __device__ __forceinline__ bool res_exchange(const ResComm& cm, unsigned long lo
   const uint32_t w = lo + threadIdx.x;
   if (w <= hi && w != blockIdx.x) {
     for (int spin = 0; res_load(cm.flags + w) < epoch; ++spin) {
-      if (spin > kResSpinMax || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
+      if (spin > cm.spins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
         sh.bad = 1;
         res_store(cm.fail, 1ull);
         break;
@@ -617,8 +625,12 @@ inline const void* res_pick(uint32_t rows, int mode, const F& make) {
 // One cooperative launch of `kernel` on a comm block that is cleared first;
 // 1 when it cannot be had (the device cannot hold all its workgroups at
 // once, or another process on the card holds its cooperative queue: the
-// caller then goes kernel by kernel), else 0 or an error.
-inline int res_launch(fx_ctx ctx, const void* kernel, uint32_t wgs, void* comm, void** args) {
+// caller then goes kernel by kernel), else 0 or an error.  before: the
+// launches of this loop so far.
+inline int res_launch(fx_ctx ctx, const void* kernel, uint32_t wgs, void* comm, void** args,
+                      uint64_t before) {
+  const char* e = std::getenv("FASPXX_FX_RESIDENT_LAUNCHES");
+  if (e && before >= (uint64_t)std::atoll(e)) return 1;
   int per_cu = 0, coop = 0;
   FX_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
   FX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kResThreads, 0));
@@ -636,6 +648,18 @@ inline int res_launch(fx_ctx ctx, const void* kernel, uint32_t wgs, void* comm, 
 
 // Iterations of one launch (the host looks at the state in between).
 constexpr uint32_t kResLaunchIters = 2048;
+
+// What became of a launch.  A loop that stopped is whole even where a wait
+// gave up: workgroup 0 stops on a reduction that every workgroup entered, so
+// the one that gave up waiting for its result had done all the work before it.
+enum ResOutcome {
+  RES_RAN,      // the state tells whether the loop goes on
+  RES_REFUSED,  // no launch: vectors and state are as they were
+  RES_LOST      // a wait gave up on the way: start over
+};
+inline ResOutcome res_outcome(bool running, unsigned long long fail) {
+  return running && fail != 0 ? RES_LOST : RES_RAN;
+}
 
 inline bool resident_disabled() {
   const char* e = std::getenv("FASPXX_FX_NORESIDENT");

@@ -908,6 +908,7 @@ int fx_solver_solve(fx_solver s, fx_vec b, fx_vec x, fx_result* res) {
   int rc = 0;
   try {
     s->last_path = fast_eligible(s) ? FX_PATH_FUSED : FX_PATH_OPS;
+    s->last_resident = false;
     if (s->last_path == FX_PATH_FUSED) {
       rc = fast_solve(s, b, x, res);
     } else {
@@ -951,6 +952,13 @@ int fx_solver_last_path(fx_solver s, int* path) {
   clear_error();
   FX_CHECK(s && path, FX_ERROR_INPUT_PAR, "null argument");
   *path = s->last_path;
+  return 0;
+}
+
+int fx_solver_last_resident(fx_solver s, int* resident) {
+  clear_error();
+  FX_CHECK(s && resident, FX_ERROR_INPUT_PAR, "null argument");
+  *resident = s->last_resident;
   return 0;
 }
 

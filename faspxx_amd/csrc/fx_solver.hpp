@@ -33,6 +33,7 @@ struct fx_solver_s {
   std::vector<double> hist_host;
   uint32_t hist_count = 0;
   int last_path = FX_PATH_OPS;  // the form the last Solve ran
+  bool last_resident = false;   // its loop ran resident to the end
   // GMRES / FGMRES: the restart length the last Solve ended with (0: as set
   // up).  The reference keeps it in the solver: Setup resets it
   // (src/GMRES.cxx:44,75-79), Solve adapts it per cycle (:255-265) and the

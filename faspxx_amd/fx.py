@@ -150,6 +150,7 @@ _SIGS = {
     "fx_solver_solve": (C.c_int, [_P, _P, _P, C.POINTER(Result)]),
     "fx_solver_history": (C.c_int, [_P, _P, C.c_uint32, C.POINTER(C.c_uint32)]),
     "fx_solver_last_path": (C.c_int, [_P, C.POINTER(C.c_int)]),
+    "fx_solver_last_resident": (C.c_int, [_P, C.POINTER(C.c_int)]),
     "fx_solver_update": (C.c_int, [_P, _P, _P, C.POINTER(Params)]),
     "fx_solver_clean": (C.c_int, [_P]),
     "fx_solver_update_op": (C.c_int, [_P, _P, _P, C.POINTER(Params)]),
@@ -162,6 +163,7 @@ _SIGS = {
     "fx_ir_create": (C.c_int, [_P, C.c_int, _P, C.c_double, C.POINTER(Params),
                                C.POINTER(Params), C.POINTER(_P)]),
     "fx_ir_solve": (C.c_int, [_P, _P, _P, C.POINTER(Result), C.POINTER(C.c_uint32)]),
+    "fx_ir_last_resident": (C.c_int, [_P, C.POINTER(C.c_int)]),
     "fx_ir_destroy": (C.c_int, [_P]),
 }
 
@@ -705,6 +707,13 @@ class Solver:
         _chk(load().fx_solver_last_path(self.h, C.byref(p)))
         return "fused" if p.value == 1 else "ops"
 
+    @property
+    def last_resident(self) -> bool:
+        """Whether the last Solve's loop ran to its end within resident launches."""
+        p = C.c_int()
+        _chk(load().fx_solver_last_resident(self.h, C.byref(p)))
+        return bool(p.value)
+
     def history(self) -> np.ndarray:
         cnt = C.c_uint32()
         load().fx_solver_history(self.h, None, 0, C.byref(cnt))
@@ -763,6 +772,13 @@ class IR:
         if rc in (-90, -12, -16, -20):
             _chk(rc)
         return res, it.value
+
+    @property
+    def last_resident(self) -> bool:
+        """Whether the last solve's inner loops ran resident."""
+        p = C.c_int()
+        _chk(load().fx_ir_last_resident(self.h, C.byref(p)))
+        return bool(p.value)
 
     def close(self):
         if self.h:

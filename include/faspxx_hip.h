@@ -367,6 +367,9 @@ int fx_solver_history(fx_solver s, double* out, uint32_t cap, uint32_t* count);
 #define FX_PATH_OPS 0
 #define FX_PATH_FUSED 1
 int fx_solver_last_path(fx_solver s, int* path);
+/* Whether the last Solve's loop (CG, BiCGStab) ran to its end within resident
+ * launches, and not kernel by kernel: 1 or 0. */
+int fx_solver_last_resident(fx_solver s, int* resident);
 int fx_solver_destroy(fx_solver s);
 
 /* Free function Krylov(A, b, x, pcd, params), src/Krylov.cxx:16-53: name
@@ -401,6 +404,8 @@ int fx_solve_ir(fx_ctx ctx, int inner_type, fx_csr A, double weight, const fx_pa
 int fx_ir_create(fx_ctx ctx, int inner_type, fx_csr A, double weight, const fx_params* outer,
                  const fx_params* inner, fx_ir* out);
 int fx_ir_solve(fx_ir ir, fx_vec b, fx_vec x, fx_result* result, uint32_t* inner_iters);
+/* Whether the last solve's inner loops ran resident: 1 or 0. */
+int fx_ir_last_resident(fx_ir ir, int* resident);
 int fx_ir_destroy(fx_ir ir);
 
 #ifdef __cplusplus
