@@ -868,7 +868,9 @@ struct BiRun {
       const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args, before);
       if (rc) return rc < 0 ? rc : 0;
       unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
-      FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
+      *fail = 0;
+      if (rs.wgs > 1)
+        FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
       FX_HIP(hipStreamSynchronize(st));
       *out = *hslot(0);
       *how = res_outcome(out->status == ST_RUN, *fail);

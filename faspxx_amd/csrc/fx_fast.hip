@@ -1638,7 +1638,9 @@ struct CgRun {
       const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args, before);
       if (rc) return rc < 0 ? rc : 0;
       unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
-      FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
+      *fail = 0;
+      if (rs.wgs > 1)
+        FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
       FX_HIP(hipStreamSynchronize(st));
       *out = *hslot(0);
       *how = res_outcome(out->status == ST_RUN, *fail);
@@ -1927,7 +1929,9 @@ struct IrInner {
         return 0;
       }
       unsigned long long* fail = (unsigned long long*)hslot(1);  // pinned
-      FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
+      *fail = 0;
+      if (rs.wgs > 1)
+        FX_HIP(hipMemcpyAsync(fail, cm.fail, sizeof(*fail), hipMemcpyDeviceToHost, st));
       FX_HIP(hipEventRecord(W.ev[0], st));
       if (l == 0 && behind) FX_TRY(behind());
       FX_HIP(hipEventSynchronize(W.ev[0]));

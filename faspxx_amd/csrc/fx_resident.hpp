@@ -622,7 +622,10 @@ inline const void* res_pick(uint32_t rows, int mode, const F& make) {
   return k;
 }
 
-// One cooperative launch of `kernel` on a comm block that is cleared first;
+// One cooperative launch of `kernel` on a comm block that is cleared first
+// (one workgroup waits for nobody: an ordinary launch, which those of other
+// streams may overlap, and nothing to clear; the runtime takes cooperative
+// launches one after the other);
 // 1 when it cannot be had (the device cannot hold all its workgroups at
 // once, or another process on the card holds its cooperative queue: the
 // caller then goes kernel by kernel), else 0 or an error.  before: the
@@ -631,6 +634,10 @@ inline int res_launch(fx_ctx ctx, const void* kernel, uint32_t wgs, void* comm, 
                       uint64_t before) {
   const char* e = std::getenv("FASPXX_FX_RESIDENT_LAUNCHES");
   if (e && before >= (uint64_t)std::atoll(e)) return 1;
+  if (wgs == 1) {
+    FX_HIP(hipLaunchKernel(kernel, dim3(1), dim3(kResThreads), args, 0, ctx->stream));
+    return 0;
+  }
   int per_cu = 0, coop = 0;
   FX_HIP(hipDeviceGetAttribute(&coop, hipDeviceAttributeCooperativeLaunch, ctx->device));
   FX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kResThreads, 0));

@@ -84,3 +84,38 @@ def test_later_launch_refused_ir(ctx, monkeypatch):
     r, x, resident = Case(ctx, "ir", A, **prm).solve()
     assert not resident and (r.retcode, r.numIter) == (r0.retcode, r0.numIter)
     assert np.array_equal(x, x0)
+
+
+def test_one_workgroup_solves_overlap():
+    """Solves of one workgroup on two contexts run side by side: both take less
+    than one after the other would."""
+    import threading
+    import time
+
+    A = P.poisson2d(44)
+    cs = [Case(fx.Context(0), fx.CG, A, maxIter=800, minIter=800) for _ in range(2)]
+    for c in cs:
+        c.b, c.x0 = 1e80 * c.b, np.zeros(A.nrow)  # (p, q) of 800 iterations stays above 1e-40
+        r, _, resident = c.solve()
+        assert resident and r.numIter == 800
+
+    def seconds(which):
+        gate = threading.Barrier(len(which) + 1)
+
+        def work(c):
+            gate.wait()
+            for _ in range(4):
+                c.solve()
+        ts = [threading.Thread(target=work, args=(c,)) for c in which]
+        for t in ts:
+            t.start()
+        gate.wait()
+        t0 = time.perf_counter()
+        for t in ts:
+            t.join()
+        return time.perf_counter() - t0
+
+    alone, both = min(seconds(cs[:1]) for _ in range(3)), min(seconds(cs) for _ in range(3))
+    assert both < 1.6 * alone
+    for c in cs:
+        c.ctx.close()
