@@ -2031,9 +2031,8 @@ int fast_solve(fx_solver S, fx_vec b, fx_vec x, fx_result* res) {
   FastWs& W = *S->fast;
   // resident loops: a banded matrix of short rows that fits the chip
   if (!W.comm && !S->op && (S->type == FX_SOLVER_CG || S->type == FX_SOLVER_BICGSTAB) &&
-      !resident_disabled() &&
-      !(S->pc->kind == 1 && S->pc->iters > 1) && res_matrix_ok(S->A) &&
-      res_shape(n, S->ctx->sms).rows) {
+      !resident_disabled() && !(S->pc->kind == 1 && S->pc->iters > 1) &&
+      res_suits<double>(S->A, S->type == FX_SOLVER_CG ? RES_CG : RES_BICGSTAB, S->ctx->sms)) {
     FX_HIP(hipMalloc(&W.comm, kResCommWords * sizeof(unsigned long long)));
     W.resident = true;
   }
@@ -2250,7 +2249,7 @@ int fx_ir_create(fx_ctx ctx, int inner_type, fx_csr A, double weight, const fx_p
     // from memory spill too many registers (1400^2 variable coefficients:
     // 41 against 28 us per iteration kernel by kernel)
     const ResShape rs = res_shape(n, ctx->sms);
-    if (ir->scaled && !resident_disabled() && res_matrix_ok(A) && rs.rows &&
+    if (ir->scaled && !resident_disabled() && res_suits<float>(&ir->As, RES_IR, ctx->sms) &&
         !(rs.rows == 8 && res_mode<float>(&ir->As, rs.rows) == RM_MEM)) {
       if (hipMalloc(&ir->W->comm, kResCommWords * sizeof(unsigned long long))) {
         set_error("IR workspace allocation failed");

@@ -133,6 +133,7 @@ struct fx_csr_s {
   uint8_t* pid = nullptr;
   int32_t* pdict = nullptr;
   uint32_t plen = 0, npat = 0;
+  uint32_t reach = 0;  // the largest |column - row|
   uint32_t pat_rows = 256;  // rows per row block of a row-pattern matrix (256 or 512)
   // Row values, for a row-pattern matrix whose rows of one pattern also hold
   // the same values bit for bit (constant-coefficient stencils): entry j of

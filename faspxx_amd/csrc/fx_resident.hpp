@@ -38,7 +38,6 @@ constexpr int kResWaves = kResThreads / 64;
 constexpr uint32_t kResMaxWgs = 256;  // 8 groups of 32 slots
 constexpr int kResBufs = 8;           // slot buffers in rotation
 constexpr int kResSlot = 8;           // doubles per slot: one 64-byte line
-constexpr uint32_t kResRowMax = 32;   // longest row the gathers take
 constexpr unsigned long long kResEmpty = ~0ull;  // a NaN that is never published
 constexpr int kResSpins = 1 << 21;    // polls before a wait gives up (seconds)
 
@@ -581,12 +580,6 @@ inline ResShape res_shape(uint32_t n, int cus) {
   return {};
 }
 
-// Whether a matrix suits the resident loops: banded forms (row patterns or
-// 16-bit column deltas; scattered columns would all be gathered past L2)
-// with short rows.
-inline bool res_matrix_ok(const fx_csr_s* A) {
-  return A && A->has_values && (A->pid || A->cd) && A->max_row <= kResRowMax && A->nrow == A->mcol;
-}
 template <class MT>
 inline ResMat res_mat(const fx_csr_s* A) {
   const void* va = sizeof(MT) == 8 ? (const void*)A->va : (const void*)A->va32;
@@ -600,6 +593,45 @@ inline int res_mode(const fx_csr_s* A, uint32_t rows) {
   if (rows > 1 && has_row_values<MT>(A) && A->vstride == 8) return RM_VAL;
   if (rows == 2 && A->max_row <= 8) return RM_REG;
   return RM_MEM;
+}
+
+// Whether a matrix suits a resident loop: banded forms (row patterns or
+// 16-bit column deltas; scattered columns would all be gathered past L2), and
+// rows that are faster there than kernel by kernel.  Rows held in registers
+// or as row values (at most 8 entries) always are.  Where values are re-read
+// from memory, a row's entries past the eighth are one dependent gather each,
+// and every entry outside the workgroup's rows is one past the L2; so the
+// lines lie by length and by how far the row reaches (near: no offset leaves
+// a workgroup's rows altogether).  us per iteration, resident against kernel
+// by kernel; k: entries of a row:
+//   one workgroup, 900 rows: CG k 17 13.1 / 17.2, k 25 20.9 / 17.4
+//   one row per thread: CG k 11 13.9 .. 26.8 / 18.2 .. 26.6,
+//     k 13 14.8 .. 36.8 / 18.2 .. 28.1, k 27 (64^3) 182 / 35
+//   two: CG k 11 near 24.5 / 26.6, far 33.3 / 28.5; k 9 no patterns 24.9 / 27.1
+//   four: CG k 5 22.8 / 35.6, k 7 far 30.0 / 31.2, k 9 near 39.0 / 41.0, far
+//     38.0 / 35.1; k 9 with row values for the kernels 34.4 / 31.8; k 7 no
+//     patterns 35.2 / 32.2 at 551368 rows and 38.9 / 41.3 at 1000000
+//     (BiCGStab 61.5 / 61.4, 70.8 / 81.9)
+//   four, refinement: k 5 10.9 / 17.9, k 9 near 18.8 / 20.6, k 7 far 18.1 / 15.5
+enum ResLoop { RES_CG, RES_BICGSTAB, RES_IR };
+template <class MT>
+inline bool res_suits(const fx_csr_s* A, ResLoop loop, int cus) {
+  if (!A || !A->has_values || !(A->pid || A->cd) || A->nrow != A->mcol) return false;
+  const ResShape rs = res_shape(A->nrow, cus);
+  if (rs.rows == 0) return false;
+  if (res_mode<MT>(A, rs.rows) != RM_MEM) return true;
+  const uint32_t k = A->max_row;
+  const bool near = rs.wgs == 1 || (A->pid && A->reach <= rs.rows * kResThreads);
+  const uint32_t near9 = near && !A->vconst ? 9 : 8;
+  if (rs.rows == 1) return k <= (rs.wgs == 1 ? 17u : 11u);
+  if (rs.rows == 2) return k <= (near ? 11u : 9u);
+  if (rs.rows == 4) {
+    if (k <= 5) return true;
+    if (loop == RES_IR) return near && k <= near9;
+    if (A->pid) return k <= near9;
+    return k <= 8 && (loop == RES_BICGSTAB || A->nrow > 3u << 18);
+  }
+  return k <= 8;
 }
 
 // make(rows, mode) for the instantiations that res_shape and res_mode give.
