@@ -2245,12 +2245,7 @@ int fx_ir_create(fx_ctx ctx, int inner_type, fx_csr A, double weight, const fx_p
     const size_t sb = sizeof(CgState) > sizeof(IrState) ? sizeof(CgState) : sizeof(IrState);
     rc = ws_alloc(*ir->W, ctx, FX_F32, n, inner->maxIter, sb, spmv_grid_max<float>(A));
     if (rc) return fail(rc);
-    // resident inner loop; eight rows per thread whose values are re-read
-    // from memory spill too many registers (1400^2 variable coefficients:
-    // 41 against 28 us per iteration kernel by kernel)
-    const ResShape rs = res_shape(n, ctx->sms);
-    if (ir->scaled && !resident_disabled() && res_suits<float>(&ir->As, RES_IR, ctx->sms) &&
-        !(rs.rows == 8 && res_mode<float>(&ir->As, rs.rows) == RM_MEM)) {
+    if (ir->scaled && !resident_disabled() && res_suits<float>(&ir->As, RES_IR, ctx->sms)) {
       if (hipMalloc(&ir->W->comm, kResCommWords * sizeof(unsigned long long))) {
         set_error("IR workspace allocation failed");
         return fail(FX_ERROR_ALLOC_MEM);

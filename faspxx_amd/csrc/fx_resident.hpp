@@ -613,6 +613,10 @@ inline int res_mode(const fx_csr_s* A, uint32_t rows) {
 //     patterns 35.2 / 32.2 at 551368 rows and 38.9 / 41.3 at 1000000
 //     (BiCGStab 61.5 / 61.4, 70.8 / 81.9)
 //   four, refinement: k 5 10.9 / 17.9, k 9 near 18.8 / 20.6, k 7 far 18.1 / 15.5
+//   eight (this form spills 165 registers): CG k 5 near 41.1 / 40.5 at 1210000
+//     rows, 42.1 / 43.5 at 1345600, 46.8 / 59.1 at 2096704; no patterns 51.2 /
+//     39.1 .. 53.9 / 53.7 to 1690000; k 7 far 58.8 / 43.0 .. 67.6 / 64.7;
+//     k 9 66.7 / 39.1; refinement k 5 41 / 28
 enum ResLoop { RES_CG, RES_BICGSTAB, RES_IR };
 template <class MT>
 inline bool res_suits(const fx_csr_s* A, ResLoop loop, int cus) {
@@ -631,7 +635,7 @@ inline bool res_suits(const fx_csr_s* A, ResLoop loop, int cus) {
     if (A->pid) return k <= near9;
     return k <= 8 && (loop == RES_BICGSTAB || A->nrow > 3u << 18);
   }
-  return k <= 8;
+  return loop == RES_CG && near && k <= 5 && A->nrow > 5u << 18;
 }
 
 // make(rows, mode) for the instantiations that res_shape and res_mode give.

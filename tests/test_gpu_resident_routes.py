@@ -79,10 +79,25 @@ def resident(ctx, kind, A):
     ("9 entries near, 800^2", lambda: star(800, 9), True, True, True),
     ("7 entries far, 82^3", lambda: stencil(82, [(1, 0, 0), (0, 1, 0), (0, 0, 1)]),
      True, True, False),
+    # eight: CG where rows of five entries reach no further than their workgroup
+    ("5 entries, 1100^2", lambda: star(1100, 5), False, False, False),
+    ("5 entries, 1160^2", lambda: star(1160, 5), True, False, False),
+    ("9 entries, 1160^2", lambda: star(1160, 9), False, False, False),
+    ("7 entries far, 110^3", lambda: stencil(110, [(1, 0, 0), (0, 1, 0), (0, 0, 1)]),
+     False, False, False),
+    ("5 entries, 1449^2", lambda: star(1449, 5), False, False, False),  # does not fit
 ])
 def test_resident_routes(ctx, name, make, cg, bi, ir):
     A = make()
     assert [resident(ctx, k, A) for k in (fx.CG, fx.BICGSTAB, "ir")] == [cg, bi, ir]
+
+
+@pytest.mark.parametrize("pc", ["jacobi", "identity"])
+@pytest.mark.parametrize("m", [1160, 1448])
+def test_cg_eight_rows_per_thread(ctx, monkeypatch, m, pc):
+    """Values re-read from memory, a ragged and the largest last workgroup."""
+    check(ctx, monkeypatch, fx.CG, P.varcoef_fv(m)[0],
+          dict(maxIter=60, relTol=1e-30, absTol=0.0), pc=pc)
 
 
 @pytest.mark.parametrize("m,entries", [(30, 17), (45, 11), (70, 11), (520, 11), (800, 9)])
