@@ -1206,6 +1206,8 @@ __global__ __launch_bounds__(kWideThreads) void k_ir_update(
   }
 }
 
+constexpr uint32_t kIrResRows = 4;  // most rows per thread of the resident inner loop
+
 // The same inner iteration with r in LDS and w, s, p, y in registers, up to
 // max_it per launch (fx_resident.hpp): r is exported after each update for
 // the gathers of other workgroups, and (w, r), (r, r) are one exchange.  p
@@ -1909,9 +1911,14 @@ struct IrInner {
   int run_resident(uint32_t maxIter, IrState& out, const std::function<int()>& behind,
                    bool* behind_ran, ResOutcome* how) {
     const ResShape rs = res_shape(W.n, W.ctx->sms);
-    const void* k = res_pick(rs.rows, res_mode<float>(As, rs.rows), [](auto r, auto m) {
-      return (const void*)&k_ir_resident<decltype(r)::value, decltype(m)::value>;
-    });
+    const void* k = nullptr;
+    if (rs.rows <= kIrResRows)
+      k = res_pick(rs.rows, res_mode<float>(As, rs.rows), [](auto r, auto m) -> const void* {
+        if constexpr (decltype(r)::value <= (int)kIrResRows)
+          return (const void*)&k_ir_resident<decltype(r)::value, decltype(m)::value>;
+        else
+          return nullptr;
+      });
     ResMat M = res_mat<float>(As);
     ResComm cm = res_comm(W.comm);
     float *r = (float*)W.r, *p = (float*)W.p, *s = (float*)W.x2, *y = (float*)W.x;

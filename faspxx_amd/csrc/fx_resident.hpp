@@ -616,13 +616,16 @@ inline int res_mode(const fx_csr_s* A, uint32_t rows) {
 //   eight (this form spills 165 registers): CG k 5 near 41.1 / 40.5 at 1210000
 //     rows, 42.1 / 43.5 at 1345600, 46.8 / 59.1 at 2096704; no patterns 51.2 /
 //     39.1 .. 53.9 / 53.7 to 1690000; k 7 far 58.8 / 43.0 .. 67.6 / 64.7;
-//     k 9 66.7 / 39.1; refinement k 5 41 / 28
+//     k 9 66.7 / 39.1
+// The refinement's loop is left out with eight rows per thread: with row
+// values 19.1 / 17.7 at 102^3, 20.9 / 20.2 at 115^3, 24.1 / 24.1 at 128^3; with
+// values from memory 41 / 28.
 enum ResLoop { RES_CG, RES_BICGSTAB, RES_IR };
 template <class MT>
 inline bool res_suits(const fx_csr_s* A, ResLoop loop, int cus) {
   if (!A || !A->has_values || !(A->pid || A->cd) || A->nrow != A->mcol) return false;
   const ResShape rs = res_shape(A->nrow, cus);
-  if (rs.rows == 0) return false;
+  if (rs.rows == 0 || (rs.rows == 8 && loop == RES_IR)) return false;
   if (res_mode<MT>(A, rs.rows) != RM_MEM) return true;
   const uint32_t k = A->max_row;
   const bool near = rs.wgs == 1 || (A->pid && A->reach <= rs.rows * kResThreads);
@@ -635,7 +638,7 @@ inline bool res_suits(const fx_csr_s* A, ResLoop loop, int cus) {
     if (A->pid) return k <= near9;
     return k <= 8 && (loop == RES_BICGSTAB || A->nrow > 3u << 18);
   }
-  return loop == RES_CG && near && k <= 5 && A->nrow > 5u << 18;
+  return near && k <= 5 && A->nrow > 5u << 18;
 }
 
 // make(rows, mode) for the instantiations that res_shape and res_mode give.

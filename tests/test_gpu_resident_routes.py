@@ -85,6 +85,9 @@ def resident(ctx, kind, A):
     ("9 entries, 1160^2", lambda: star(1160, 9), False, False, False),
     ("7 entries far, 110^3", lambda: stencil(110, [(1, 0, 0), (0, 1, 0), (0, 0, 1)]),
      False, False, False),
+    ("row values, 101^3", lambda: P.poisson3d(101), True, True, True),
+    ("row values, 102^3", lambda: P.poisson3d(102), True, False, False),
+    ("row values, 128^3", lambda: P.poisson3d(128), True, False, False),
     ("5 entries, 1449^2", lambda: star(1449, 5), False, False, False),  # does not fit
 ])
 def test_resident_routes(ctx, name, make, cg, bi, ir):
