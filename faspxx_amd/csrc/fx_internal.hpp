@@ -285,19 +285,28 @@ inline uint32_t spmv_blocks_of(const fx_csr_s* A) {
 // nothing to read there, so a workgroup of 256 rows is only latency (flag,
 // dictionary, gathers, reduction, one after the other): on the 128^3 stencil
 // the f64 product takes 14.2 us with 1024 rows per workgroup and 16 us with
-// 256 (24.5 us streaming the values).  Up to kRowValMin rows the values
-// stay in L2, 1024 rows per workgroup would leave CUs without one, and the
-// dictionary is one more dependent load (256^2 points, FGMRES: 17.0 against
-// 16.9 ms), so the kernels stream the values there.
+// 256 (24.5 us streaming the values).  The kernels stream the values of
+// smaller matrices: the latency of such a workgroup, some 5 us, is then more
+// than the stream takes.  Apply and Residual, streamed / by row values: f64
+// 274625 rows 16.5 / 18.8 us, 405224 18.9 / 19.2, 512000 22.1 / 19.6; f32 405224
+// 16.0 / 18.3, 636056 18.0 / 18.8, 778688 19.8 / 19.0.  The dictionary itself is
+// made from kRowValMin rows on: the resident loops hold several rows per thread
+// by it.
 constexpr uint32_t kRowValRows = 1024;
 constexpr uint32_t kRowValMin = 256 * kRowValRows;
+constexpr uint32_t kRowValSpmv64 = 400 * kRowValRows;
+constexpr uint32_t kRowValSpmv32 = 704 * kRowValRows;
 template <class MT>
 inline bool has_row_values(const fx_csr_s* A) {
   return A->vconst && A->nrow > kRowValMin && (sizeof(MT) == 8 || A->vd32);
 }
 template <class MT>
+inline bool spmv_by_row_values(const fx_csr_s* A) {
+  return has_row_values<MT>(A) && A->nrow > (sizeof(MT) == 8 ? kRowValSpmv64 : kRowValSpmv32);
+}
+template <class MT>
 inline uint32_t spmv_units(const fx_csr_s* A) {
-  if (has_row_values<MT>(A)) return (A->nrow + kRowValRows - 1) / kRowValRows;
+  if (spmv_by_row_values<MT>(A)) return (A->nrow + kRowValRows - 1) / kRowValRows;
   return spmv_blocks_of<MT>(A);
 }
 template <class MT>

@@ -94,7 +94,7 @@ inline SpmvIn<double, double> spmv_in<double, double>(fx_csr A) {
           A->plen, A->npat * A->plen,
           A->swin, A->soff, A->slane, A->scol, A->has_values ? A->sval : nullptr,
           A->lwin, A->lrow, nullptr,
-          has_row_values<double>(A) ? A->vok : nullptr, A->vd64, A->pcnt,
+          spmv_by_row_values<double>(A) ? A->vok : nullptr, A->vd64, A->pcnt,
           A->vdict, A->npat, A->vstride, A->nrow};
 }
 template <>
@@ -110,7 +110,7 @@ inline SpmvIn<float, float> spmv_in<float, float>(fx_csr A) {
           A->plen, A->npat * A->plen,
           nullptr, nullptr, nullptr, nullptr, nullptr,
           nullptr, nullptr, nullptr,
-          has_row_values<float>(A) ? A->vok : nullptr, A->vd32, A->pcnt,
+          spmv_by_row_values<float>(A) ? A->vok : nullptr, A->vd32, A->pcnt,
           A->vdict, A->npat, A->vstride, A->nrow};
 }
 
@@ -962,7 +962,7 @@ template <class MT, class VT, int MODE, int NRED, unsigned MAXMASK, class XF, cl
 inline int launch_spmv(fx_csr A, hipStream_t st, XF xf, BF bf, Epi epi, double* partials,
                        hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr, bool finisher = true) {
   const unsigned g = spmv_grid_of<MT>(A, A->ctx->sms);
-  if (has_row_values<MT>(A))
+  if (spmv_by_row_values<MT>(A))
     launch_spmv_k<MT, VT, MODE, NRED, MAXMASK, XF, BF, Epi, CF_ROWVAL>(A, st, xf, bf, epi,
                                                                        partials, e0, e1, g);
   else if (A->pid && sizeof(MT) == 4 && A->pat_rows == kPat2Rows)  // f32 copies only
