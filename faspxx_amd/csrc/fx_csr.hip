@@ -583,14 +583,18 @@ int csr_row_values(fx_csr A, const float* va, float* vd, int* vok, bool* host_ok
 // Later launches are not given the row values (vconst), and solvers set up
 // on A make new replay graphs (gen) on the grid of single row blocks;
 // launches that a caller captured earlier find the flag cleared when they
-// run.
+// run.  It is cleared before this returns, on a stream of its own: the
+// context's stream may be one that is captured, and the caller may write the
+// values and replay those launches on another.  Products that run meanwhile
+// read the entries, which are still the same.
 int csr_drop_row_values(fx_csr A) {
   if (!A->vconst) return 0;
   A->vconst = false;
   A->gen = next_handle_gen();
-  hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1), 0, A->ctx->stream, A->vok);
-  FX_HIP(hipGetLastError());
-  return 0;
+  return on_own_stream([&](hipStream_t st) {
+    hipLaunchKernelGGL(k_clear_flag, dim3(1), dim3(1), 0, st, A->vok);
+    return hipGetLastError();
+  });
 }
 
 // The values of the slices from the CSR values: dst[p] = src[smap[p]]

@@ -242,6 +242,25 @@ constexpr uint32_t kSellRows = kThreads;
 constexpr uint32_t kSellMax = FX_SELL_MAX;
 constexpr uint32_t kSellNoRow = 0xFFFFFFFFu;
 
+// enqueue(stream) on a stream made for it, waited for; also while this thread
+// captures another stream.
+template <class F>
+inline int on_own_stream(const F& enqueue) {
+  hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+  FX_HIP(hipThreadExchangeStreamCaptureMode(&mode));
+  hipStream_t st = nullptr;
+  hipError_t e = hipStreamCreateWithFlags(&st, hipStreamNonBlocking);
+  if (e == hipSuccess) {
+    e = enqueue(st);
+    const hipError_t w = hipStreamSynchronize(st);
+    if (e == hipSuccess) e = w;
+    (void)hipStreamDestroy(st);
+  }
+  (void)hipThreadExchangeStreamCaptureMode(&mode);
+  FX_HIP(e);
+  return 0;
+}
+
 // The first n (at most 8) of the 32-bit words at dev, once the work queued
 // before is done (fx_core.hip).
 int read_words(fx_ctx ctx, const uint32_t* dev, int n, uint32_t* out);

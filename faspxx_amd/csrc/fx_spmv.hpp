@@ -451,7 +451,7 @@ __device__ __forceinline__ void row_value_block(const SpmvIn<MT, VT>& in,
   constexpr int H = kRowValRows / (P * kThreads);     // passes
   constexpr int kDv = kPatDict / kThreads;
   static_assert(kPatMax <= kThreads, "one length per thread");
-  if (*in.vok == 0) {
+  auto by_entry = [&]() {
     for (uint32_t i = r0 + tid; i < r0 + nr; i += kThreads) {
       double t = (MODE == ROW_AX) ? 0.0 : (double)bf(i);
       const uint32_t s = in.rp[i], e = in.rp[i + 1];
@@ -464,8 +464,7 @@ __device__ __forceinline__ void row_value_block(const SpmvIn<MT, VT>& in,
       }
       epi.row(i, t, acc);
     }
-    return;
-  }
+  };
   auto pid_at = [&](uint32_t i) { return (uint32_t)in.pid[r0 + min(i, nr - 1)]; };
   uint32_t pidv[P];
 #pragma unroll
@@ -485,7 +484,12 @@ __device__ __forceinline__ void row_value_block(const SpmvIn<MT, VT>& in,
     lds.va[tid + j * kThreads] = vv[j];
   }
   if (tid < (int)kPatMax) lds.rp[tid] = cnt;
+  if (tid == 0) lds.ci[0] = (uint32_t)*in.vok;
   __syncthreads();
+  if (lds.ci[0] == 0) {  // one answer for the workgroup: it may be cleared meanwhile
+    by_entry();
+    return;
+  }
   if (in.vstride == 8) {
 #pragma unroll 1
     for (int h = 0; h < H; ++h) {

@@ -62,3 +62,40 @@ def test_captured_product_follows_new_values(name):
             assert np.array_equal(y.cpu().numpy(), want)
         del g
         c.close()
+
+
+def test_pointer_asked_for_during_a_capture():
+    """The values' pointer handed out while the context's stream is captured:
+    a product captured before it reads what is then written through it, though
+    the second graph never runs."""
+    import torch
+    from faspxx_amd import fx
+    A = SYSTEMS["poisson3d_90"]()
+    n = A.nrow
+    st = torch.cuda.Stream()
+    with torch.cuda.stream(st):
+        c = fx.Context(0, stream=st.cuda_stream)
+        M = fx.Csr.from_problem(c, A)
+        x = torch.tensor(np.random.default_rng(1).uniform(-1, 1, n), device="cuda")
+        y, z = torch.zeros_like(x), torch.zeros_like(x)
+        v = np.random.default_rng(2).uniform(1, 2, A.nnz)
+        vx, vy = fx.Vec.wrap(c, x.data_ptr(), n), fx.Vec.wrap(c, y.data_ptr(), n)
+        fx.Csr.from_problem(c, P.CSR(n, n, A.row_ptr, A.col_ind, v, A.diag_ptr)).Apply(vx, vy)
+        st.synchronize()
+        want = y.cpu().numpy()
+        g0, g1 = torch.cuda.CUDAGraph(), torch.cuda.CUDAGraph()
+        g0.capture_begin(capture_error_mode="thread_local")
+        M.Apply(vx, vy)
+        g0.capture_end()
+        g1.capture_begin(capture_error_mode="thread_local")
+        z.fill_(1.0)
+        ptr = M.values_ptr
+        g1.capture_end()
+        fx.Vec.wrap(c, ptr, A.nnz).upload(v)
+        for _ in range(3):
+            y.zero_()
+            g0.replay()
+            st.synchronize()
+            assert np.array_equal(y.cpu().numpy(), want)
+        del g0, g1
+        c.close()
