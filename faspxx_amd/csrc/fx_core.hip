@@ -425,10 +425,8 @@ static int ctx_init(fx_ctx c) {
   FX_HIP(hipMalloc(&c->dscal, sizeof(double) * 64));
   FX_HIP(hipMalloc(&c->rcount, sizeof(unsigned) * kRedStride * kRedCounts));
   const size_t cb = sizeof(unsigned) * kRedStride * kRedCounts;
-  if (c->own_stream)  // a caller's stream may be one that is captured
-    FX_HIP(hipMemsetAsync(c->rcount, 0, cb, c->stream));
-  else
-    FX_HIP(hipMemset(c->rcount, 0, cb));
+  // waited for: a caller's stream is ordered after no other (and may be captured)
+  FX_TRY(on_own_stream([&](hipStream_t st) { return hipMemsetAsync(c->rcount, 0, cb, st); }));
   FX_HIP(hipHostMalloc(&c->hpin, sizeof(double) * 64, hipHostMallocDefault));
   hipDeviceProp_t prop;
   FX_HIP(hipGetDeviceProperties(&prop, c->device));

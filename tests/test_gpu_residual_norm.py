@@ -30,3 +30,25 @@ def test_residual_shortcut(ctx, n):
             got = r.numpy()
             assert np.all(np.abs(got - want) <= np.finfo(npdt).eps * np.abs(want))
             assert np.array_equal(got, b) == (at is None)
+
+
+def test_reductions_on_a_callers_stream_behind_a_busy_null_stream():
+    """A context made on a non-blocking stream while the null stream is busy:
+    its first reductions find their counts cleared."""
+    import torch
+    from faspxx_amd import fx
+    st = torch.cuda.Stream()
+    a = torch.randn(4096, 4096, device="cuda")
+    with torch.cuda.stream(st):
+        t = torch.arange(100000, dtype=torch.float64, device="cuda")
+        torch.cuda.synchronize()
+        for _ in range(5):
+            with torch.cuda.stream(torch.cuda.default_stream()):
+                for _ in range(4):
+                    a @ a
+            c = fx.Context(0, stream=st.cuda_stream)
+            x = fx.Vec.wrap(c, t.data_ptr(), t.numel())
+            assert [x.NormInf() for _ in range(3)] == [99999.0] * 3
+            x.close()
+            c.close()
+        torch.cuda.synchronize()
