@@ -128,7 +128,7 @@ __global__ __launch_bounds__(kWideThreads) void k_gm_start(VT* __restrict__ v0, 
 // the other, a reduction per j.  Three forms:
 //   up to kGmOneRows rows (one workgroup): all steps and the Givens update in
 //     one kernel, w in registers (k_gm_orth_one);
-//   cycles of up to kGmLowMax: the same h_j by linearity from one pass over the
+//   cycles of kGmLowMin to kGmLowMax: the same h_j by linearity from one pass over the
 //     basis, h_j = (V[j], w) - sum_{i<j} (V[j], V[i]) h_i, i.e. (I + L) h = V^T w
 //     with L the strictly lower part of V^T V, whose row k is formed in the
 //     pass of step k.  (Low-synchronization modified Gram-Schmidt:
@@ -139,10 +139,14 @@ __global__ __launch_bounds__(kWideThreads) void k_gm_start(VT* __restrict__ v0, 
 //     per column instead of w, V[j], V[j+1] read and w written for every j,
 //     and 3 kernels replace k + 1.  The second pass runs from V[k] down, so
 //     that it begins with what the first one read last;
-//   longer cycles: a kernel per j (k_gm_mgs).
+//   shorter and longer cycles: a kernel per j (k_gm_mgs).
 // Measured, this part of an iteration of GMRES(30): 1024^2 unknowns 41 us (18.6
 // + 4.6 + 17.9) against 79 us a kernel per j; 256^2 13.7 us in 3 kernels
 // against 56 us in 13 on average; 40^2 one kernel.
+// Three columns take two kernels each on average one by one: GMRES(3) at
+// 100^2 28.0 us per iteration a kernel per j, 29.0 in three kernels, FGMRES(3)
+// 32.6 and 33.9; GMRES(4) 27.6 and 26.3, FGMRES(4) 31.6 and 31.2.
+constexpr uint32_t kGmLowMin = 4;
 constexpr uint32_t kGmLowMax = 63;   // one lane per column in the triangular solve
 constexpr uint32_t kGmLowLd = 64;    // row length of L
 
@@ -981,7 +985,7 @@ struct GmRun {
       }
       const double* pin = pa;
       unsigned gin = gs;
-      if (m <= kGmLowMax) {
+      if (m >= kGmLowMin && m <= kGmLowMax) {
         double* hv = G.low + (size_t)kGmLowMax * kGmLowLd;
         static_assert(Pack16<VT>::W == 2, "the dot products' grid counts f64 packs");
         const unsigned gd = gm_dot_wgs(n, cus);
