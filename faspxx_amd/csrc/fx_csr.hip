@@ -442,15 +442,13 @@ int csr_alloc(fx_csr A) {
 }
 
 // Row patterns of a matrix given on the host: pid[i], a dictionary of
-// plen-strided offset lists (col - row), each pattern's first row and the
-// largest offset either way.  False when some row is longer than kPatMaxLen,
+// plen-strided offset lists (col - row) and each pattern's first row.  False when some row is longer than kPatMaxLen,
 // there are more than kPatMax distinct patterns, or the dictionary exceeds
 // kPatDict offsets.  Each pattern is found by a hash of (length, offsets) and then compared entry by
 // entry, so a hash collision cannot merge two patterns.
 bool build_patterns(uint32_t nrow, const uint32_t* rp, const uint32_t* ci, uint32_t max_row,
                     std::vector<uint8_t>& pid, std::vector<int32_t>& dict,
-                    std::vector<uint32_t>& first, uint32_t& plen, uint32_t& npat,
-                    uint32_t& reach) {
+                    std::vector<uint32_t>& first, uint32_t& plen, uint32_t& npat) {
   if (max_row > kPatMaxLen || nrow == 0) return false;
   plen = max_row ? max_row : 1;
   std::vector<std::vector<int32_t>> pats;
@@ -478,7 +476,6 @@ bool build_patterns(uint32_t nrow, const uint32_t* rp, const uint32_t* ci, uint3
       found = (int)pats.size();
       pats.emplace_back(off.begin(), off.begin() + len);
       first.push_back(i);
-      for (uint32_t j = 0; j < len; ++j) reach = std::max(reach, (uint32_t)std::abs(off[j]));
       ids.push_back((uint32_t)found);
     }
     pid[i] = (uint8_t)found;
@@ -825,13 +822,12 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
   std::vector<uint8_t> pid;
   std::vector<int32_t> dict;
   std::vector<uint32_t> first;
-  uint32_t plen = 0, npat = 0, reach = 0;
+  uint32_t plen = 0, npat = 0;
   bool pat = false;
   if (host_ci && A->nnz && !col32 && !patterns_disabled()) {
     uint32_t longest = 0;
     for (uint32_t r = 0; r < A->nrow; ++r) longest = std::max(longest, host_rp[r + 1] - host_rp[r]);
-    pat = build_patterns(A->nrow, host_rp, host_ci, longest, pid, dict, first, plen, npat,
-                         reach);
+    pat = build_patterns(A->nrow, host_rp, host_ci, longest, pid, dict, first, plen, npat);
   }
   hipStream_t st = A->ctx->stream;
   uint32_t mx = 0;
@@ -863,7 +859,8 @@ int csr_set_blocks(fx_csr A, const uint32_t* host_rp, const uint32_t* host_ci) {
                           hipMemcpyHostToDevice, st));
     A->plen = plen;
     A->npat = npat;
-    A->reach = reach;
+    A->reach = 0;
+    for (const int32_t o : dict) A->reach = std::max(A->reach, (uint32_t)std::abs(o));
     if (A->has_values && A->nrow > kRowValMin && row_values_enabled()) {
       std::vector<uint32_t> cnt(npat);
       for (uint32_t p = 0; p < npat; ++p) cnt[p] = host_rp[first[p] + 1] - host_rp[first[p]];
