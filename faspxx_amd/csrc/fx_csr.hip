@@ -263,8 +263,13 @@ __global__ void k_pattern_grad(const uint32_t* __restrict__ rp, const uint32_t* 
 // tile of rows from every row that a block coming out of the tile before can
 // end at (a block has at most kBlockRows rows), and the tiles' answers are
 // then strung together.  (The chain on the host, with the copies of the row
-// pointers there and of the tables back, took 0.6 ms at 262144 rows.)
+// pointers there and of the tables back, took 0.6 ms at 262144 rows.)  Three
+// launches, two up to kBlkChain tiles, whose answers every workgroup strings
+// together for itself, and one for a single tile: a launch is some 4 us, which
+// shows in small matrices (the sum of two of 1600 rows: 103 us with the host's
+// chain, 107 in three launches, 94 in one).
 constexpr uint32_t kBlkTile = 2048;
+constexpr uint32_t kBlkChain = 32;
 
 struct BlkStage {
   uint32_t rp[kBlkTile + kBlockRows + 1];
@@ -327,7 +332,7 @@ __global__ __launch_bounds__(kThreads) void k_blk_chain(const uint32_t* __restri
                                                         uint32_t ntile, uint32_t* __restrict__ entry,
                                                         uint32_t* __restrict__ before,
                                                         uint32_t* __restrict__ out) {
-  constexpr uint32_t kAt = 32;  // tiles staged at a time
+  constexpr uint32_t kAt = kBlkChain;  // tiles staged at a time
   __shared__ uint32_t w[kAt * kBlockRows];
   __shared__ uint32_t mx;
   if (threadIdx.x == 0) mx = 0;
@@ -354,29 +359,63 @@ __global__ __launch_bounds__(kThreads) void k_blk_chain(const uint32_t* __restri
   if (threadIdx.x == 0) out[0] = c, out[1] = mx, out[2] = 0;
 }
 
-__global__ __launch_bounds__(kThreads) void k_blk_fill(const uint32_t* __restrict__ rp,
-                                                       uint32_t nrow,
-                                                       const uint32_t* __restrict__ entry,
-                                                       const uint32_t* __restrict__ before,
-                                                       uint32_t* __restrict__ blk,
-                                                       const uint32_t* __restrict__ nblk,
-                                                       uint16_t* __restrict__ rpb) {
+// FORM: BLK_ENTRY reads entry and before; BLK_CHAIN forms them, and out, from
+// walk and longest of at most kBlkChain tiles; BLK_ONE is the only tile.
+enum { BLK_ENTRY = 0, BLK_CHAIN = 1, BLK_ONE = 2 };
+template <int FORM>
+__global__ __launch_bounds__(kThreads) void k_blk_fill(
+    const uint32_t* __restrict__ rp, uint32_t nrow, const uint32_t* __restrict__ entry,
+    const uint32_t* __restrict__ before, const uint32_t* __restrict__ walk,
+    const uint32_t* __restrict__ longest, uint32_t* __restrict__ blk, uint32_t* __restrict__ out,
+    uint16_t* __restrict__ rpb) {
   __shared__ BlkStage s;
   __shared__ uint16_t start[kBlkTile + 1];
-  __shared__ uint32_t count;
+  __shared__ uint32_t w[FORM == BLK_CHAIN ? kBlkChain * kBlockRows : 1];
+  __shared__ uint32_t count, first, mx;
+  const uint32_t ntile = gridDim.x;
+  if (threadIdx.x == 0) mx = 0;
+  if constexpr (FORM == BLK_CHAIN)
+    for (uint32_t i = threadIdx.x; i < ntile * kBlockRows; i += kThreads) w[i] = walk[i];
   blk_stage(rp, nrow, s);
   const uint32_t t0 = blockIdx.x * kBlkTile, left = min(kBlkTile, nrow - t0);
+  if constexpr (FORM == BLK_ONE) {
+    uint32_t m = 0;
+    for (uint32_t i = threadIdx.x; i < left; i += kThreads) m = max(m, s.rp[i + 1] - s.rp[i]);
+    atomicMax(&mx, m);
+  }
   if (threadIdx.x == 0) {
-    uint32_t at = entry[blockIdx.x], c = 0;
+    uint32_t at = 0, c = 0, all = 0;
+    first = 0;
+    if constexpr (FORM == BLK_ENTRY) {
+      at = entry[blockIdx.x];
+      first = before[blockIdx.x];
+    }
+    if constexpr (FORM == BLK_CHAIN) {
+      uint32_t e = 0, m = 0;
+      for (uint32_t t = 0; t < ntile; ++t) {
+        if (t == blockIdx.x) at = e, first = all;
+        const uint32_t v = w[t * kBlockRows + e];
+        all += v & 0xffffu;
+        e = v >> 16;
+        m = max(m, longest[t]);
+      }
+      if (blockIdx.x == 0) out[0] = all, out[1] = m, out[2] = 0;
+    }
     while (at < left) {
       start[c++] = (uint16_t)at;
       at = s.next[at];
     }
     start[c] = (uint16_t)at;
     count = c;
+    if (blockIdx.x == 0) {
+      const uint32_t total = FORM == BLK_ENTRY ? out[0] : FORM == BLK_CHAIN ? all : c;
+      blk[2 * total] = nrow;
+      blk[2 * total + 1] = rp[nrow];
+    }
   }
   __syncthreads();
-  const uint32_t lane = threadIdx.x & 63, b0 = before[blockIdx.x];
+  if (FORM == BLK_ONE && threadIdx.x == 0) out[0] = count, out[1] = mx, out[2] = 0;
+  const uint32_t lane = threadIdx.x & 63, b0 = first;
   for (uint32_t b = threadIdx.x >> 6; b < count; b += kWaves) {
     const uint32_t r0 = start[b], r1 = start[b + 1], k0 = s.rp[r0];
     if (lane == 0) {
@@ -384,10 +423,6 @@ __global__ __launch_bounds__(kThreads) void k_blk_fill(const uint32_t* __restric
       blk[2 * (b0 + b) + 1] = k0;
     }
     for (uint32_t r = r0 + lane; r < r1; r += 64) rpb[t0 + r] = (uint16_t)(s.rp[r] - k0);
-  }
-  if (blockIdx.x == 0 && threadIdx.x == 0) {
-    blk[2 * *nblk] = nrow;
-    blk[2 * *nblk + 1] = rp[nrow];
   }
 }
 
@@ -406,11 +441,17 @@ int device_blocks(fx_csr A, bool col32) {
   auto run = [&]() -> int {
     FX_HIP(hipMalloc(&A->rpb, sizeof(uint16_t) * A->nrow));
     FX_HIP(hipMalloc(&A->blk, sizeof(uint32_t) * 2 * (most + 1)));
-    hipLaunchKernelGGL(k_blk_walk, dim3(nt), dim3(kThreads), 0, st, A->rp, A->nrow, walk, longest);
-    hipLaunchKernelGGL(k_blk_chain, dim3(1), dim3(kThreads), 0, st, walk, longest, nt, entry,
-                       before, tmp);
-    hipLaunchKernelGGL(k_blk_fill, dim3(nt), dim3(kThreads), 0, st, A->rp, A->nrow, entry, before,
-                       A->blk, tmp, A->rpb);
+    if (nt > 1)
+      hipLaunchKernelGGL(k_blk_walk, dim3(nt), dim3(kThreads), 0, st, A->rp, A->nrow, walk,
+                         longest);
+    if (nt > kBlkChain)
+      hipLaunchKernelGGL(k_blk_chain, dim3(1), dim3(kThreads), 0, st, walk, longest, nt, entry,
+                         before, tmp);
+    const auto fill = nt > kBlkChain ? k_blk_fill<BLK_ENTRY>
+                      : nt > 1       ? k_blk_fill<BLK_CHAIN>
+                                     : k_blk_fill<BLK_ONE>;
+    hipLaunchKernelGGL(fill, dim3(nt), dim3(kThreads), 0, st, A->rp, A->nrow, entry, before, walk,
+                       longest, A->blk, tmp, A->rpb);
     if (!col32) {
       FX_HIP(hipMalloc(&A->cd, sizeof(int16_t) * A->nnz));
       hipLaunchKernelGGL(k_col_delta, dim3((unsigned)most), dim3(kThreads), 0, st, A->ci, A->blk,
