@@ -439,7 +439,7 @@ __global__ __launch_bounds__(kResThreads) void k_bi_resident(
   bool ok = true;
   for (uint32_t it = 0; it < max_it; ++it) {
     rows.fresh();
-    rows.template product<false>(A, ml, pl, (const double*)p, tv);
+    rows.product(A, ml, pl, (const double*)p, tv);
     double a1[1] = {0.0}, b1 = 0.0;  // even and odd rows: half the chain
 #pragma unroll
     for (int k = 0; k < R; ++k) {
@@ -474,7 +474,7 @@ __global__ __launch_bounds__(kResThreads) void k_bi_resident(
     ok = res_exchange(cm, 2 * (unsigned long long)it + 1, wlo, whi, sh);
     if (!ok) break;
     rows.fresh();
-    rows.template product<false>(A, ml, sl, (const double*)s, tv);
+    rows.product(A, ml, sl, (const double*)s, tv);
     double a2[2] = {0.0, 0.0}, b2[2] = {0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < R; ++k) {

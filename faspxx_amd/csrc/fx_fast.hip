@@ -518,7 +518,7 @@ __global__ __launch_bounds__(kResThreads) void k_cg_resident(
       else
         rows.product_within(pl, qv);
     } else {
-      rows.template product<false>(A, ml, pl, (const double*)p, qv);
+      rows.product(A, ml, pl, (const double*)p, qv);
     }
     double pq[1] = {0.0};
 #pragma unroll
@@ -1252,7 +1252,7 @@ __global__ __launch_bounds__(kResThreads) void k_ir_resident(ResMat A, float* r,
   bool ok = true;
   for (uint32_t it = 0; it < max_it; ++it) {
     double wv[R];
-    rows.template product<false>(A, ml, rl, (const float*)r, wv);
+    rows.product(A, ml, rl, (const float*)r, wv);
     double v[2] = {0.0, 0.0};
 #pragma unroll
     for (int k = 0; k < R; ++k) {

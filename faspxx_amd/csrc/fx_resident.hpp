@@ -317,7 +317,6 @@ struct ResMat {
   const void* __restrict__ va;       // values in CSR order
   const int32_t* __restrict__ vdict; // row values: offsets, vstride per pattern
   const void* __restrict__ vval;     // row values
-  const uint32_t* __restrict__ pcnt;
   uint32_t n, plen, npat, vstride;
 };
 
@@ -334,7 +333,6 @@ struct ResRows {
   struct Lds {
     alignas(16) int32_t dict[kPatDict];
     alignas(16) MT val[MM == RM_VAL ? kPatDict : 1];
-    uint16_t cnt[MM == RM_VAL ? kPatMax + 1 : 1];
     uint32_t lo, hi;
   };
   MT a[MM == RM_REG ? R : 1][8];
@@ -371,8 +369,6 @@ struct ResRows {
         l.dict[i] = d[i];
         if constexpr (MM == RM_VAL) l.val[i] = ((const MT*)A.vval)[i];
       }
-      if constexpr (MM == RM_VAL)
-        if (tid < A.npat) l.cnt[tid] = (uint16_t)A.pcnt[tid];
     }
     if (tid == 0) {
       l.lo = 0xffffffffu;
@@ -474,18 +470,16 @@ struct ResRows {
   }
 
   // (A v)_i of the thread's q-th row, left to right as in the SpMV kernels
-  // (w = v0 * x0, then fma); with NEG, out[q] - A v by fma(-a, x, t).  vl:
-  // the workgroup's own entries in LDS; vg: the exported vector.  Two rows
-  // at a time: their outside entries are all asked for before the first sum,
-  // and no more than two rows' are held in registers.
-  template <bool NEG, class VT>
+  // (w = v0 * x0, then fma).  vl: the workgroup's own entries in LDS; vg: the
+  // exported vector.  Two rows at a time: their outside entries are all asked
+  // for before the first sum, and no more than two rows' are held in registers.
+  template <class VT>
   __device__ __forceinline__ void product(const ResMat& A, const Lds& l, const VT* vl,
                                           const VT* vg, double (&out)[R]) const {
     constexpr int PQ = R < 2 ? 1 : 2;
     const uint32_t tid = threadIdx.x, base = blockIdx.x * kRows;
     auto term = [&](double& t, bool first, MT av, VT xv) {
-      if (NEG) t = fma(-(double)av, (double)xv, t);
-      else t = first ? (double)av * (double)xv : fma((double)av, (double)xv, t);
+      t = first ? (double)av * (double)xv : fma((double)av, (double)xv, t);
     };
     auto fetch = [&](uint32_t c) -> VT {
       const uint32_t d = c - base;
@@ -531,7 +525,7 @@ struct ResRows {
       for (int u = 0; u < PQ; ++u) {
         const int q = q0 + u;
         const uint32_t n = len(q);
-        double t = NEG ? out[q] : 0.0;
+        double t = 0.0;
         if constexpr (MM == RM_MEM) {
           const uint32_t i = base + q * kResThreads + tid;
           const MT* va = (const MT*)A.va + start[q];
@@ -584,8 +578,7 @@ template <class MT>
 inline ResMat res_mat(const fx_csr_s* A) {
   const void* va = sizeof(MT) == 8 ? (const void*)A->va : (const void*)A->va32;
   const void* vv = sizeof(MT) == 8 ? (const void*)A->vd64 : (const void*)A->vd32;
-  return {A->rp, A->ci, A->pid, A->pdict, va, A->vdict, vv, A->pcnt,
-          A->nrow, A->plen, A->npat, A->vstride};
+  return {A->rp, A->ci, A->pid, A->pdict, va, A->vdict, vv, A->nrow, A->plen, A->npat, A->vstride};
 }
 template <class MT>
 inline int res_mode(const fx_csr_s* A, uint32_t rows) {
