@@ -465,6 +465,9 @@ __device__ __forceinline__ void row_value_block(const SpmvIn<MT, VT>& in,
       epi.row(i, t, acc);
     }
   };
+  // It may be cleared while this runs, and the waves differ: each thread's rows
+  // are the same either way, and the dictionary is loaded by all.
+  const bool kept = *in.vok != 0;
   auto pid_at = [&](uint32_t i) { return (uint32_t)in.pid[r0 + min(i, nr - 1)]; };
   uint32_t pidv[P];
 #pragma unroll
@@ -484,9 +487,8 @@ __device__ __forceinline__ void row_value_block(const SpmvIn<MT, VT>& in,
     lds.va[tid + j * kThreads] = vv[j];
   }
   if (tid < (int)kPatMax) lds.rp[tid] = cnt;
-  if (tid == 0) lds.ci[0] = (uint32_t)*in.vok;
   __syncthreads();
-  if (lds.ci[0] == 0) {  // one answer for the workgroup: it may be cleared meanwhile
+  if (!kept) {
     by_entry();
     return;
   }
