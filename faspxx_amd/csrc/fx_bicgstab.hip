@@ -863,7 +863,7 @@ struct BiRun {
       double *x = vx(), *r = vr(), *p = vp(), *s = vs(), *pt = vpt();
       const double *r0s = vr0s(), *d = dinv;
       BiState *ds = dstate(0), *hs = hslot(0);
-      uint32_t most = kResLaunchIters;
+      uint32_t most = res_launch_iters(rs.wgs);
       void* args[] = {&M, &x, &r, &p, &s, &pt, &r0s, &d, &ds, &hs, &P, &W.hist, &cm, &most};
       const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args, before);
       if (rc) return rc < 0 ? rc : 0;

@@ -1635,7 +1635,7 @@ struct CgRun {
       double* z = (double*)W.x2;
       const double* d = dinv;
       CgState *ds = dstate(), *hs = hslot(0);
-      uint32_t most = kResLaunchIters;
+      uint32_t most = res_launch_iters(rs.wgs);
       void* args[] = {&M, &x, &r, &p, &q, &z, &d, &ds, &hs, &P, &W.hist, &cm, &most};
       const int rc = res_launch(W.ctx, k, rs.wgs, W.comm, args, before);
       if (rc) return rc < 0 ? rc : 0;
@@ -1923,7 +1923,7 @@ struct IrInner {
     ResComm cm = res_comm(W.comm);
     float *r = (float*)W.r, *p = (float*)W.p, *s = (float*)W.x2, *y = (float*)W.x;
     IrState *ds = dstate(0), *hs = hslot(0);
-    uint32_t most = kResLaunchIters;
+    uint32_t most = res_launch_iters(rs.wgs);
     void* args[] = {&M, &r, &p, &s, &y, &ds, &hs, &cm, &most};
     if (behind_ran) *behind_ran = false;
     const uint64_t max_launches = (uint64_t)maxIter / kResLaunchIters + 4;

@@ -22,8 +22,8 @@
 // is refused goes on kernel by kernel from where the last one ended.
 //
 // Environment, for tests: FASPXX_FX_NORESIDENT=1 none of this;
-// FASPXX_FX_RESIDENT_SPINS=N polls before a wait gives up;
-// FASPXX_FX_RESIDENT_LAUNCHES=N launches of one loop before they are refused.
+// FASPXX_FX_RESIDENT_FAIL=1 launches of one iteration that find *fail raised,
+// as by a wait that gave up; FASPXX_FX_RESIDENT_LAUNCHES=N launches of one loop before they are refused.
 #pragma once
 
 #include <cstdlib>
@@ -46,23 +46,24 @@ struct ResComm {
   unsigned long long* gsum;   // [kResBufs][8][kResSlot]
   unsigned long long* flags;  // [kResMaxWgs]: iterations whose export is visible
   unsigned long long* fail;
-  int spins;  // polls before a wait gives up
 };
 constexpr size_t kResSlotWords = (size_t)kResBufs * kResMaxWgs * kResSlot;
 constexpr size_t kResGsumWords = (size_t)kResBufs * 8 * kResSlot;
 constexpr size_t kResCommWords = kResSlotWords + kResGsumWords + kResMaxWgs + 8;
 inline ResComm res_comm(void* mem) {
   unsigned long long* w = (unsigned long long*)mem;
-  const char* e = std::getenv("FASPXX_FX_RESIDENT_SPINS");
   return {w, w + kResSlotWords, w + kResSlotWords + kResGsumWords,
-          w + kResSlotWords + kResGsumWords + kResMaxWgs, e ? std::atoi(e) : kResSpins};
+          w + kResSlotWords + kResGsumWords + kResMaxWgs};
 }
 
-// Empty slots and zero flags, before each launch.
-static __global__ __launch_bounds__(kThreads) void k_res_clear(unsigned long long* w) {
+// Empty slots and zero flags, before each launch; *fail as given.
+static __global__ __launch_bounds__(kThreads) void k_res_clear(unsigned long long* w,
+                                                               unsigned long long fail) {
   for (size_t i = blockIdx.x * kThreads + threadIdx.x; i < kResCommWords;
        i += (size_t)gridDim.x * kThreads)
-    w[i] = i < kResSlotWords + kResGsumWords ? kResEmpty : 0ull;
+    w[i] = i < kResSlotWords + kResGsumWords                ? kResEmpty
+           : i == kResSlotWords + kResGsumWords + kResMaxWgs ? fail
+                                                             : 0ull;
 }
 
 __device__ __forceinline__ void res_store(unsigned long long* p, unsigned long long v) {
@@ -208,7 +209,7 @@ __device__ __forceinline__ bool res_allreduce(double (&v)[K], const ResComm& cm,
         for (int spin = 0;; ++spin) {
           if (active) x = res_load(p);
           if (__all(!active || x != kResEmpty)) break;
-          if (spin > cm.spins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
+          if (spin > kResSpins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
             ok = false;
             break;
           }
@@ -230,7 +231,7 @@ __device__ __forceinline__ bool res_allreduce(double (&v)[K], const ResComm& cm,
           });
           res_for<I>([&](auto i) { have = have && (!act[i] || x[i] != kResEmpty); });
           if (__all(have)) break;
-          if (spin > cm.spins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
+          if (spin > kResSpins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
             ok = false;
             break;
           }
@@ -296,7 +297,7 @@ __device__ __forceinline__ bool res_exchange(const ResComm& cm, unsigned long lo
   const uint32_t w = lo + threadIdx.x;
   if (w <= hi && w != blockIdx.x) {
     for (int spin = 0; res_load(cm.flags + w) < epoch; ++spin) {
-      if (spin > cm.spins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
+      if (spin > kResSpins || ((spin & 1023) == 1023 && res_load(cm.fail) != 0)) {
         sh.bad = 1;
         res_store(cm.fail, 1ull);
         break;
@@ -654,6 +655,17 @@ inline const void* res_pick(uint32_t rows, int mode, const F& make) {
   return k;
 }
 
+inline bool res_fail_forced() {
+  const char* e = std::getenv("FASPXX_FX_RESIDENT_FAIL");
+  return e && e[0] == '1';
+}
+
+// Iterations of one launch (the host looks at the state in between).
+constexpr uint32_t kResLaunchIters = 2048;
+inline uint32_t res_launch_iters(uint32_t wgs) {
+  return wgs > 1 && res_fail_forced() ? 1 : kResLaunchIters;
+}
+
 // One cooperative launch of `kernel` on a comm block that is cleared first
 // (one workgroup waits for nobody: an ordinary launch, which those of other
 // streams may overlap, and nothing to clear; the runtime takes cooperative
@@ -675,7 +687,7 @@ inline int res_launch(fx_ctx ctx, const void* kernel, uint32_t wgs, void* comm, 
   FX_HIP(hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, kernel, kResThreads, 0));
   if (!coop || (uint64_t)per_cu * (uint64_t)ctx->sms < wgs) return 1;
   hipLaunchKernelGGL(k_res_clear, dim3(16), dim3(kThreads), 0, ctx->stream,
-                     (unsigned long long*)comm);
+                     (unsigned long long*)comm, res_fail_forced() ? 1ull : 0ull);
   FX_HIP(hipGetLastError());
   if (hipLaunchCooperativeKernel(kernel, dim3(wgs), dim3(kResThreads), args, 0, ctx->stream) !=
       hipSuccess) {
@@ -684,9 +696,6 @@ inline int res_launch(fx_ctx ctx, const void* kernel, uint32_t wgs, void* comm, 
   }
   return 0;
 }
-
-// Iterations of one launch (the host looks at the state in between).
-constexpr uint32_t kResLaunchIters = 2048;
 
 // What became of a launch.  A loop that stopped is whole even where a wait
 // gave up: workgroup 0 stops on a reduction that every workgroup entered, so

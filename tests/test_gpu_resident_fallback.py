@@ -46,16 +46,16 @@ def test_resident_is_reported(ctx, monkeypatch, kind, prm, m):
 
 
 @pytest.mark.parametrize("kind,prm", CASES)
-@pytest.mark.parametrize("m,env", [(32, "LAUNCHES"), (70, "LAUNCHES"), (70, "SPINS"),
-                                   (200, "SPINS")])
+@pytest.mark.parametrize("m,env", [(32, "LAUNCHES"), (70, "LAUNCHES"), (70, "FAIL"),
+                                   (200, "FAIL")])
 def test_starts_over(ctx, monkeypatch, kind, prm, m, env):
-    """A launch refused at once, and waits that give up after two polls, among
-    up to 32 workgroups and more: kernel by kernel from the caller's x, and
-    again so on the next solve."""
+    """A launch refused at once, and one whose workgroups leave as after a wait
+    that gave up: kernel by kernel from the caller's x, and again so on the
+    next solve."""
     monkeypatch.setenv("FASPXX_FX_NORESIDENT", "1")
     r0, x0, _ = Case(ctx, kind, P.poisson2d(m), **prm).solve()
     monkeypatch.delenv("FASPXX_FX_NORESIDENT")
-    monkeypatch.setenv("FASPXX_FX_RESIDENT_" + env, "0")
+    monkeypatch.setenv("FASPXX_FX_RESIDENT_" + env, "1" if env == "FAIL" else "0")
     c = Case(ctx, kind, P.poisson2d(m), **prm)
     for _ in range(2):
         r, x, resident = c.solve()
