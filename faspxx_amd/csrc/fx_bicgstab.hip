@@ -355,9 +355,12 @@ __device__ __forceinline__ void bi_after_update(BiState* S, const CgPrm& P, doub
 // in parentheses: 1024 unknowns 7.4 (22.3), 256^2 16.1 (24.5), 1024^2 27.6
 // (54.0), 95^3 37.5 (52.8).  Up to four rows per thread: eight rows' vectors
 // do not fit the registers.  The two dot products sum a thread's even and odd
-// rows apart, half the chain.  (At 1024^2 the upwind system's count is set by
-// rounding: 1240 to 1522 over right-hand sides an ulp apart, mean 1379, and
-// 1268 to 1462, mean 1361, with the five kernels.)
+// rows apart and the third reduction does not; one chain everywhere and pairs
+// everywhere take the same time (95^3 36.0, 36.1, 36.1 us per iteration in turn
+// with this order in the middle; 1024^2 26.1, 26.1, 26.2).  What the order does
+// set, as any rounding does, is the count on the upwind system at 1024^2: over
+// 24 right-hand sides an ulp apart 1389 to 1635, mean 1490, and 1396 to 1630,
+// mean 1504, with the five kernels.
 
 // The quotients above formed by the lanes of one wave at once.
 struct BiQuotientsWave {
@@ -440,7 +443,7 @@ __global__ __launch_bounds__(kResThreads) void k_bi_resident(
   for (uint32_t it = 0; it < max_it; ++it) {
     rows.fresh();
     rows.product(A, ml, pl, (const double*)p, tv);
-    double a1[1] = {0.0}, b1 = 0.0;  // even and odd rows: half the chain
+    double a1[1] = {0.0}, b1 = 0.0;  // even and odd rows
 #pragma unroll
     for (int k = 0; k < R; ++k) {
       tv[k] = tv[k] * dv[k];
