@@ -365,6 +365,7 @@ int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, double* dev_ou
 // A copy of a few words to pageable memory and a wait took some 30 us.
 int read_words(fx_ctx ctx, const uint32_t* dev, int n, uint32_t* out) {
   constexpr unsigned long long pending = ~0ull;  // no 32-bit word
+  std::lock_guard<std::mutex> hold(ctx->words);
   unsigned long long* slots = reinterpret_cast<unsigned long long*>(ctx->hpin) + 8;
   for (int i = 0; i < n; ++i) __atomic_store_n(slots + i, pending, __ATOMIC_RELEASE);
   hipLaunchKernelGGL(k_words_to_host, dim3(1), dim3(64), 0, ctx->stream, dev, n, slots);

@@ -10,6 +10,7 @@
 
 #include <cstdint>
 #include <cstdio>
+#include <mutex>
 #include <type_traits>
 #include <utility>
 #include <vector>
@@ -82,7 +83,11 @@ struct fx_ctx_s {
   bool own_stream = false;
   fx_red_ws ws;
   double* dscal = nullptr;  // device scalar slots for standalone reductions
-  double* hpin = nullptr;   // pinned: the scalar a reduction hands to the host
+  // pinned: the scalar a reduction hands to the host, and from the ninth on the
+  // words of read_words, one reader at a time (matrices of one context may be
+  // made by several threads)
+  double* hpin = nullptr;
+  std::mutex words;
   unsigned* rcount = nullptr;  // workgroups done, of the reduction that runs (fx_core.hip)
   hipEvent_t tev[2] = {nullptr, nullptr};  // dispatch-attached timing events (fx_spmv_timed)
   int sms = 256;
