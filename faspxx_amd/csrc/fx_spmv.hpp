@@ -59,9 +59,13 @@ struct SpmvIn {
   // rows sorted by length (u32 columns): the matrix row of each block row,
   // or null when block rows are matrix rows
   const uint32_t* __restrict__ rmap;
-  // row patterns whose rows also share their values (see fx_csr_s): the
-  // values and lengths of the patterns, used while *vok is 1; vok is null
-  // where the matrix has none
+};
+// Row patterns whose rows also share their values (see fx_csr_s): the values
+// and lengths of the patterns, used while *vok is 1.  Arguments of these
+// kernels alone (in every kernel's, Apply and Residual of a power-law matrix of
+// 104035 rows took 30.9 us, without 30.7).
+template <class MT, class VT>
+struct SpmvRvIn : SpmvIn<MT, VT> {
   const int* __restrict__ vok;
   const MT* __restrict__ pval;
   const uint32_t* __restrict__ pcnt;
@@ -88,14 +92,12 @@ inline SpmvIn<double, double> spmv_in<double, double>(fx_csr A) {
             A->oblk,  A->onblk, A->nnz, nullptr, nullptr,
             0,        0,
             nullptr, nullptr, nullptr, nullptr, nullptr,
-            nullptr, nullptr, A->omap, nullptr, nullptr, nullptr, nullptr, 0, 0, 0};
+            nullptr, nullptr, A->omap};
   return {A->rp,   A->rpb,  A->ci,  A->cd,    A->has_values ? A->va : nullptr,
           A->sell ? A->sblk : A->blk,  A->sell ? A->nwin : A->nblk, A->nnz, A->pid,   A->pdict,
           A->plen, A->npat * A->plen,
           A->swin, A->soff, A->slane, A->scol, A->has_values ? A->sval : nullptr,
-          A->lwin, A->lrow, nullptr,
-          spmv_by_row_values<double>(A) ? A->vok : nullptr, A->vd64, A->pcnt,
-          A->vdict, A->npat, A->vstride, A->nrow};
+          A->lwin, A->lrow, nullptr};
 }
 template <>
 inline SpmvIn<float, float> spmv_in<float, float>(fx_csr A) {
@@ -104,14 +106,34 @@ inline SpmvIn<float, float> spmv_in<float, float>(fx_csr A) {
             A->oblk,  A->onblk, A->nnz, nullptr, nullptr,
             0,        0,
             nullptr, nullptr, nullptr, nullptr, nullptr,
-            nullptr, nullptr, A->omap, nullptr, nullptr, nullptr, nullptr, 0, 0, 0};
+            nullptr, nullptr, A->omap};
   return {A->rp,   A->rpb,  A->ci,  A->cd,    A->has_values ? A->va32 : nullptr,
           A->blk,  A->nblk, A->nnz, A->pid,   A->pdict,
           A->plen, A->npat * A->plen,
           nullptr, nullptr, nullptr, nullptr, nullptr,
-          nullptr, nullptr, nullptr,
-          spmv_by_row_values<float>(A) ? A->vok : nullptr, A->vd32, A->pcnt,
-          A->vdict, A->npat, A->vstride, A->nrow};
+          nullptr, nullptr, nullptr};
+}
+
+// (a trait rather than a condition: an unnamed enum in a kernel's signature is
+// mangled differently for the host and for the device)
+template <class MT, class VT, int CF>
+struct SpmvArg {
+  using type = SpmvIn<MT, VT>;
+};
+template <class MT, class VT>
+struct SpmvArg<MT, VT, CF_ROWVAL> {
+  using type = SpmvRvIn<MT, VT>;
+};
+template <class MT, class VT, int CF>
+inline typename SpmvArg<MT, VT, CF>::type spmv_arg(fx_csr A) {
+  if constexpr (CF == CF_ROWVAL) {
+    const MT* values = nullptr;
+    if constexpr (sizeof(MT) == 8) values = A->vd64;
+    else values = A->vd32;
+    return {spmv_in<MT, VT>(A), A->vok, values, A->pcnt, A->vdict, A->npat, A->vstride, A->nrow};
+  } else {
+    return spmv_in<MT, VT>(A);
+  }
 }
 
 // Threads per row for a block of nr rows holding nz entries: one thread per
@@ -179,8 +201,9 @@ struct SpmvLds {
   static constexpr uint32_t kDict = (is_pat(CF) || CF == CF_ROWVAL) ? kPatDict : 1;
   RpT rp[kRows + 1];
   CiT ci[kCi];
-  alignas(16) int32_t dict[kDict];
-  alignas(16) MT va[kNnz];
+  static constexpr size_t kPacks = CF == CF_ROWVAL ? 16 : 4;  // read as 16-byte packs there
+  alignas(kPacks) int32_t dict[kDict];
+  alignas(kPacks > alignof(MT) ? kPacks : alignof(MT)) MT va[kNnz];
   __device__ __forceinline__ uint32_t col(uint32_t k, uint32_t r0) const {
     if constexpr (CF == CF_D16) return (uint32_t)((int32_t)r0 + (int32_t)ci[k]);
     else return ci[k];
@@ -442,7 +465,7 @@ __device__ __forceinline__ void pat_block(const SpmvIn<MT, VT>& in, SpmvLds<MT, 
 // been cleared (a launch captured before the values changed) the rows are
 // read entry by entry from the CSR arrays, summed in the same order.
 template <int MODE, int NRED, class MT, class VT, class XF, class BF, class Epi>
-__device__ __forceinline__ void row_value_block(const SpmvIn<MT, VT>& in,
+__device__ __forceinline__ void row_value_block(const SpmvRvIn<MT, VT>& in,
                                                 SpmvLds<MT, CF_ROWVAL>& lds, uint32_t r0,
                                                 uint32_t nr, int tid, const XF& xf, const BF& bf,
                                                 const Epi& epi,
@@ -727,8 +750,8 @@ __device__ __forceinline__ void emit_row(const Epi& epi, uint32_t pos, uint32_t 
 //   void fin(double (&sum)[NRED])          run by k_finish after the kernel
 template <class MT, class VT, int MODE, int NRED, unsigned MAXMASK, class XF, class BF, class Epi,
           int CF>
-__global__ __launch_bounds__(kThreads, CF == CF_ROWVAL ? 8 : 1) void k_spmv(SpmvIn<MT, VT> in, XF xf0, BF bf, Epi epi0,
-                                                   double* partials) {
+__global__ __launch_bounds__(kThreads, CF == CF_ROWVAL ? 8 : 1) void k_spmv(
+    typename SpmvArg<MT, VT, CF>::type in, XF xf0, BF bf, Epi epi0, double* partials) {
   if (epi0.skip()) return;
   XF xf = xf0;
   Epi epi = epi0;
@@ -957,11 +980,11 @@ inline void launch_spmv_k(fx_csr A, hipStream_t st, XF xf, BF bf, Epi epi, doubl
                           hipEvent_t e0, hipEvent_t e1, unsigned g) {
   if (e0)
     hipExtLaunchKernelGGL((k_spmv<MT, VT, MODE, NRED, MAXMASK, XF, BF, Epi, CF>), dim3(g),
-                          dim3(kThreads), 0, st, e0, e1, 0, spmv_in<MT, VT>(A), xf, bf, epi,
+                          dim3(kThreads), 0, st, e0, e1, 0, spmv_arg<MT, VT, CF>(A), xf, bf, epi,
                           partials);
   else
     hipLaunchKernelGGL((k_spmv<MT, VT, MODE, NRED, MAXMASK, XF, BF, Epi, CF>), dim3(g),
-                       dim3(kThreads), 0, st, spmv_in<MT, VT>(A), xf, bf, epi, partials);
+                       dim3(kThreads), 0, st, spmv_arg<MT, VT, CF>(A), xf, bf, epi, partials);
 }
 
 template <class MT, class VT, int MODE, int NRED, unsigned MAXMASK, class XF, class BF, class Epi>
