@@ -341,15 +341,18 @@ __global__ __launch_bounds__(kThreads) void k_norminf(const T* __restrict__ x, u
   block_partials<1, 1u>(acc, partials);
 }
 
-// Residual's first step.  Above kNormCounted elements the partials are left to
-// k_finish: the count, one workgroup after another's store, costs more there
-// than the second launch does.  Residual by count / with k_finish: 343000 rows
-// f32 10.1 / 9.7 us, 490000 rows f64 12.9 / 12.5; with the product before it, 230^2
-// rows f32, 11.5 / 13.9: there the host that queues the launches is slower.
-constexpr uint32_t kNormCounted = 192 * 1024;
+// Residual's first step.  Several workgroups count themselves done one store
+// after another, which takes longer than a second launch does: it is for calls
+// whose launches the host queues more slowly than the device runs them, short
+// rows (light) and no more than these.  Residual with the product before it, by
+// count / with k_finish: f32 230^2 rows 11.5 / 13.9 us, 57^3 12.3 / 13.8, 343000
+// 14.7 / 14.1; f64 51^3 13.4 / 13.6, 54^3 14.2 / 14.0, 57^3 14.6 / 14.2; a
+// power-law matrix of 104035 rows 30.7 / 30.4.
 template <class T>
-int norminf_of(fx_ctx ctx, const void* x, uint32_t n, double* dev_out) {
-  if (n <= kNormCounted)
+constexpr uint32_t kNormCounted = (sizeof(T) == 8 ? 128 : 192) * 1024;
+template <class T>
+int norminf_of(fx_ctx ctx, const void* x, uint32_t n, bool light, double* dev_out) {
+  if (stream_blocks(n) == 1 || (light && n <= kNormCounted<T>))
     return launch_reduce<T>(ctx, 2, 0, 0.0, x, nullptr, nullptr, n, dev_out, nullptr);
   const unsigned g = stream_blocks(n);
   hipLaunchKernelGGL(k_norminf<T>, dim3(g), dim3(kThreads), 0, ctx->stream, (const T*)x, n,
@@ -357,9 +360,9 @@ int norminf_of(fx_ctx ctx, const void* x, uint32_t n, double* dev_out) {
   FX_HIP(hipGetLastError());
   return launch_finish<1, 1u>(ctx->stream, ctx->ws.partials, g, FinStore<1>{dev_out, 0});
 }
-int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, double* dev_out) {
-  return dtype == FX_F64 ? norminf_of<double>(ctx, x, n, dev_out)
-                         : norminf_of<float>(ctx, x, n, dev_out);
+int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, bool light, double* dev_out) {
+  return dtype == FX_F64 ? norminf_of<double>(ctx, x, n, light, dev_out)
+                         : norminf_of<float>(ctx, x, n, light, dev_out);
 }
 
 // A copy of a few words to pageable memory and a wait took some 30 us.

@@ -269,8 +269,9 @@ inline int on_own_stream(const F& enqueue) {
 // The first n (at most 8) of the 32-bit words at dev, once the work queued
 // before is done (fx_core.hip).
 int read_words(fx_ctx ctx, const uint32_t* dev, int n, uint32_t* out);
-// ||x||_inf of n elements into *dev_out (no synchronisation; fx_core.hip).
-int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, double* dev_out);
+// ||x||_inf of n elements into *dev_out (no synchronisation; fx_core.hip); light:
+// before a product that takes little longer than its launch.
+int norminf_dev(fx_ctx ctx, const void* x, int dtype, uint32_t n, bool light, double* dev_out);
 int csr_spmv_dispatch(fx_ctx ctx, fx_csr A, const void* x, void* y, int dtype,
                       hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr);
 int ensure_dinv32(fx_pc pc);

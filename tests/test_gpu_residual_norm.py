@@ -1,6 +1,6 @@
 """Residual's max-norm on both sides of the size from which its partials are
-combined by a second launch (196608 rows): b - A x where some |x_i| >= 1e-20,
-wherever it is, and b itself where there is none."""
+combined by a second launch (f64 131072 rows, f32 196608): b - A x where some
+|x_i| >= 1e-20, wherever it is, and b itself where there is none."""
 import numpy as np
 import pytest
 
@@ -9,7 +9,8 @@ from test_gpu_rowvalues import diag
 pytestmark = pytest.mark.gpu
 
 
-@pytest.mark.parametrize("n", [1, 1025, 32 * 1024 + 1, 192 * 1024, 192 * 1024 + 1, 500003])
+@pytest.mark.parametrize("n", [1, 1025, 32 * 1024 + 1, 128 * 1024, 128 * 1024 + 1, 192 * 1024,
+                               192 * 1024 + 1, 500003])
 def test_residual_shortcut(ctx, n):
     from faspxx_amd import fx
     M = fx.Csr.from_problem(ctx, diag(n))
