@@ -129,7 +129,8 @@ def leg_convdiff(fx, P, ctx):
         out[name] = {"ms": round(min(ms), 3), "iters": r.numIter, "retcode": r.retcode,
                      "relres_fp64": relres(pr, x.numpy()),
                      "us_per_iter": round(min(ms) * 1e3 / max(r.numIter, 1), 1),
-                     "path": ("fused graph replay" if s.last_path == "fused"
+                     "path": ("resident loop" if s.last_resident
+                              else "fused graph replay" if s.last_path == "fused"
                               else "per-operation")}
         log(f"convdiff {name}: {min(ms):.1f} ms, {r.numIter} iters, relres "
             f"{out[name]['relres_fp64']:.2e}")
@@ -305,8 +306,9 @@ def main() -> int:
         jac_ms.append(r.solve_ms)
     sweep_bytes = 12 * nnz + 4 * (n + 1) + 4 * 8 * n
     jac = {"ms_50_sweeps": min(jac_ms), "iters": r.numIter, "final_norm2": r.norm2,
-           "GBs_per_sweep": sweep_bytes * 50 / min(jac_ms) / 1e6}
-    log(f"Jacobi 50 sweeps: {min(jac_ms):.2f} ms ({jac['GBs_per_sweep']:.0f} GB/s)")
+           # bytes of the reference's format (u32 columns); row values move fewer
+           "algorithmic_GBs_per_sweep": sweep_bytes * 50 / min(jac_ms) / 1e6}
+    log(f"Jacobi 50 sweeps: {min(jac_ms):.2f} ms")
 
     # ---- FP64 Jacobi-PCG to rtol 1e-8 ------------------------------------
     pc = fx.Precond(ctx, "jacobi", A, 1.0, 1)
@@ -322,7 +324,10 @@ def main() -> int:
     cg_relres = float(np.linalg.norm(pr.b - A64.matvec(xr)) / np.linalg.norm(pr.b))
     cg_iter_bytes = 12 * nnz + 4 * (n + 1) + 13 * 8 * n
     cg = {"ms": min(cg_ms), "iters": rcg.numIter, "relres_fp64": cg_relres,
-          "GBs_per_iter": cg_iter_bytes * rcg.numIter / min(cg_ms) / 1e6}
+          "path": "resident loop" if scg.last_resident else "fused graph replay",
+          # bytes of the kernel-by-kernel form on u32 columns; a resident loop moves
+          # the vector that its workgroups exchange
+          "algorithmic_GBs_per_iter": cg_iter_bytes * rcg.numIter / min(cg_ms) / 1e6}
     log(f"FP64 PCG: {min(cg_ms):.2f} ms, {rcg.numIter} iters, relres {cg_relres:.2e}")
 
     # ---- timed steps: FP32-inner / FP64-refined CG ------------------------
@@ -392,6 +397,10 @@ def main() -> int:
     traffic = profiled_traffic("k_spmv_f64_poisson3d_128_traffic.json", A.index_bytes, nnz)
 
     f64 = res_spmv["f64"]
+    # HBM bytes that the stored format moves, per second; without a counter
+    # profile of it, those of the reference's format (u32 columns)
+    moved = traffic or f64["bytes"]
+    achieved = moved / f64["ms_mean_flushed"] / 1e6
     line = {
         "metric": "CG time-to-rtol 1e-8 + SpMV GB/s, 3D Poisson 128³; FP32-refined vs FP64",
         "value": round(ir_ms, 4),
@@ -417,15 +426,11 @@ def main() -> int:
         "jacobi": jac,
         "setup_s": round(setup_s, 3),
         "roofline": {"bound": "hbm", "kernel": "k_spmv f64 (MAT::Apply)",
-                     "achieved": round(f64["GBs_flushed"], 1), "peak": HBM_PEAK_GBS,
-                     "unit": "GB/s", "frac": round(f64["GBs_flushed"] / HBM_PEAK_GBS, 4),
-                     "traffic": traffic, "algorithmic_bytes": f64["bytes"],
-                     "index_bytes": A.index_bytes,
-                     # the HBM bytes the stored format actually moves, per second
-                     "traffic_GBs": (round(traffic / f64["ms_mean_flushed"] / 1e6, 1)
-                                     if traffic else None),
-                     "traffic_frac": (round(traffic / f64["ms_mean_flushed"] / 1e6
-                                            / HBM_PEAK_GBS, 4) if traffic else None)},
+                     "achieved": round(achieved, 1), "peak": HBM_PEAK_GBS,
+                     "unit": "GB/s", "frac": round(achieved / HBM_PEAK_GBS, 4),
+                     "traffic": traffic, "index_bytes": A.index_bytes,
+                     "algorithmic_bytes": f64["bytes"],
+                     "algorithmic_GBs": round(f64["GBs_flushed"], 1)},
         "cpu_baseline": cpu,
         "other_configs": extra,
     }

@@ -152,8 +152,9 @@ int fx_sub(fx_ctx ctx, fx_vec v, fx_vec y);
 /* max / min entry   VEC::Max / Min, src/VEC.cxx:382-421 (start values -1e60 / 1e60) */
 int fx_max(fx_ctx ctx, fx_vec x, double* out);
 int fx_min(fx_ctx ctx, fx_vec x, double* out);
-/* Reductions returning a host double (synchronising), VEC::Dot / Norm2 /
- * NormInf, src/VEC.cxx:424-485.  Summation order is a fixed two-stage tree
+/* Reductions returning a host double, VEC::Dot / Norm2 / NormInf,
+ * src/VEC.cxx:424-485.  They wait for their result, and so for the work queued
+ * before it; the stream's own completion may be seen a little later.  Summation order is a fixed two-stage tree
  * (deterministic run to run); it differs from the reference's 4-way order. */
 int fx_dot(fx_ctx ctx, fx_vec x, fx_vec y, double* out);
 int fx_norm2(fx_ctx ctx, fx_vec x, double* out);
@@ -222,7 +223,9 @@ int fx_csr_download(fx_csr A, uint32_t* rowPtr, uint32_t* colInd, double* values
 int fx_csr_set_values_dev(fx_csr A, const double* dev_values);
 /* Device pointer to the f64 values (nnz doubles).  Values written through it
  * are seen by the f64 SpMV of a matrix without sorted or sliced rows; call
- * fx_csr_set_values_dev with it to refresh every copy. */
+ * fx_csr_set_values_dev with it to refresh every copy.  A matrix read from a
+ * dictionary of row values is read entry by entry from then on, as after
+ * fx_csr_set_values_dev. */
 double* fx_csr_values_dev(fx_csr A);
 /* Build (or rebuild) the f32 value copy used by f32 SpMV / mixed precision. */
 int fx_csr_make_f32(fx_csr A);
@@ -360,8 +363,8 @@ int fx_solver_solve(fx_solver s, fx_vec b, fx_vec x, fx_result* result);
 /* Residual norms the reference prints per iteration (SOL::PrintInfo,
  * src/SOL.cxx:46-64), index = iteration number. */
 int fx_solver_history(fx_solver s, double* out, uint32_t cap, uint32_t* count);
-/* Which form ran the last Solve: FX_PATH_FUSED (graph-replayed fused
- * kernels, scalars on the device) or FX_PATH_OPS (one device call per
+/* Which form ran the last Solve: FX_PATH_FUSED (fused kernels, replayed from
+ * graphs or resident on the chip, scalars on the device) or FX_PATH_OPS (one device call per
  * reference operation, scalars read back).  No reference counterpart (the
  * reference has one CPU path). */
 #define FX_PATH_OPS 0
