@@ -1,7 +1,7 @@
 // fx_bicgstab.hip -- fused, graph-replayed BiCGStab (src/BiCGStab.cxx:68-270)
 // with the identity or a one-sweep Jacobi preconditioner on the system
-// matrix.  Banded systems of up to 1048576 rows run their loop in one
-// cooperative launch (see "the resident iteration" below), others kernel by
+// matrix.  Banded systems of short rows, up to 1048576 of them, run their
+// loop in one launch (see "the resident iteration" below), others kernel by
 // kernel.
 //
 // The reference's recurrence is the preconditioned P.A form: the residual is
@@ -352,8 +352,8 @@ __device__ __forceinline__ void bi_after_update(BiState* S, const CgPrm& P, doub
 // itself from the same sums.  On leaving, x, r, p, pt and the state are where
 // the five kernels would have left them.  Bound by the exchanges' latency:
 // three reductions and two halos; us per iteration, with the five kernels'
-// in parentheses: 1024 unknowns 7.4 (22.3), 256^2 16.1 (24.5), 1024^2 27.6
-// (54.0), 95^3 37.5 (52.8).  Up to four rows per thread: eight rows' vectors
+// in parentheses: 1024 unknowns 7.4 (22.3), 256^2 16.1 (24.5), 1024^2 26.1
+// (53.4), 95^3 36.5 (51.9).  Up to four rows per thread: eight rows' vectors
 // do not fit the registers.  The two dot products sum a thread's even and odd
 // rows apart and the third reduction does not; one chain everywhere and pairs
 // everywhere take the same time (95^3 36.0, 36.1, 36.1 us per iteration in turn

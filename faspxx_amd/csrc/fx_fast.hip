@@ -14,8 +14,8 @@
 // a single-reduction form: 2 kernels and 11 vector passes per iteration
 // (see "the scaled inner solver of the refinement" below).
 //
-// Banded systems that fit the chip run the CG loop and the refinement's inner
-// loop in one cooperative launch (see "the resident iteration" below).  Else a
+// Banded systems of short rows that fit the chip run the CG loop and the
+// refinement's inner loop in one launch (see "the resident iteration" below).  Else a
 // CG iteration = 3 kernels (see "the three-kernel iteration" below), replayed
 // as a hipGraph of kChunk iterations; the last iteration of a replay copies
 // the state to a pinned host slot.  Per iteration HBM traffic: the SpMV's

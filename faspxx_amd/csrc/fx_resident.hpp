@@ -1,5 +1,5 @@
-// fx_resident.hpp -- solver loops that stay on the chip: one cooperative
-// launch runs many iterations, each workgroup owning a contiguous range of
+// fx_resident.hpp -- solver loops that stay on the chip: one launch (of more
+// than one workgroup: a cooperative one) runs many iterations, each workgroup owning a contiguous range of
 // rows whose vectors live in registers and LDS between the iterations.
 //
 // Kernel by kernel an iteration pays, for every kernel, a launch gap, the
@@ -15,8 +15,8 @@
 // for its stores (vmcnt) before it stores the flag or slot that announces
 // them; a reader looks at the data only after it has seen that.
 //
-// The launch is cooperative: every workgroup is on the chip, so each wait
-// ends.  Waits are bounded all the same; one that runs out raises *fail and
+// A launch that waits is cooperative: every workgroup is on the chip, so each
+// wait ends.  Waits are bounded all the same; one that runs out raises *fail and
 // every workgroup leaves.  The host then starts over kernel by kernel, from
 // the caller's x (the refinement: from its last outer iterate).  A launch that
 // is refused goes on kernel by kernel from where the last one ended.
