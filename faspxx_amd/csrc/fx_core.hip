@@ -429,8 +429,10 @@ static int ctx_init(fx_ctx c) {
   FX_HIP(hipMalloc(&c->dscal, sizeof(double) * 64));
   FX_HIP(hipMalloc(&c->rcount, sizeof(unsigned) * kRedStride * kRedCounts));
   const size_t cb = sizeof(unsigned) * kRedStride * kRedCounts;
-  // waited for: a caller's stream is ordered after no other (and may be captured)
-  FX_TRY(on_own_stream([&](hipStream_t st) { return hipMemsetAsync(c->rcount, 0, cb, st); }));
+  // the reductions run on c->stream; a caller's may be captured, so there the
+  // clear goes elsewhere and is waited for
+  if (c->own_stream) FX_HIP(hipMemsetAsync(c->rcount, 0, cb, c->stream));
+  else FX_TRY(on_own_stream([&](hipStream_t st) { return hipMemsetAsync(c->rcount, 0, cb, st); }));
   FX_HIP(hipHostMalloc(&c->hpin, sizeof(double) * 64, hipHostMallocDefault));
   hipDeviceProp_t prop;
   FX_HIP(hipGetDeviceProperties(&prop, c->device));
